@@ -129,6 +129,23 @@ def test_all_launch_shapes_agree(V, O, dims, bcs):
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("dims,most", [((31, 9, 2), 1), ((45, 33, 23), 1), ((112, 97, 31), 4)])
+def test_default_march_of_grids_that_do_not_fill_the_chip(V, O, dims, most, dtype):
+    """The default launch shortens the z march (at most `most` planes per workgroup
+    here); every face of a short last chunk and of one-plane chunks is covered."""
+    bcs = [(2, 1), (0, 0), (1, 2)]
+    U = smooth_state(dims, seed=3, dtype=dtype)
+    sim = make_sim(V, dims, bcs, 5.0 / 3.0, dtype, U)
+    assert 1 <= sim.launch()["zchunk"] <= most
+    g = oracle_grid(O, dims, bcs, 5.0 / 3.0)
+    Uo = U.copy()
+    O.step(g, Uo, 1e-3, floor64=dtype == np.float32)
+    V.step(sim, 1e-3)
+    assert np.array_equal(sim.state(), Uo), sim.launch()
+    sim.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_device_dt_loop_bitwise(V, O, dtype):
     dims = (40, 24, 20)
     bcs = [(0, 0), (2, 2), (1, 1)]

@@ -21,6 +21,44 @@ int fail(int code, const char* fmt, const char* a = "", long long b = 0);
 
 namespace vh {
 
+// Estimated time (in units of a few µs) of a z-marching stage launch: `wgs` workgroups
+// of `planes` planes each. A plane of a workgroup costs 2 + r when r workgroups
+// share a compute unit (measured at 32³-200³: 5.5, 7.4 and 9.3 µs for r = 1, 2, 3 in
+// the exact Float64 form; the fixed part is the latency of its loads and barriers),
+// and the prologue 0.7 planes. per_cu: resident workgroups of the kernel per unit.
+inline double march_cost(long long wgs, int planes, int per_cu, int cus) {
+  const long long slots = (long long)per_cu * cus;
+  const long long rem = wgs % slots;
+  const long long r = (rem + cus - 1) / cus;
+  return (planes + 0.7) * ((double)(wgs / slots) * (2 + per_cu) + (rem ? 2 + r : 0));
+}
+
+// Planes per workgroup for `columns` tiles of an nz-plane grid: `most` (the fastest on
+// grids that fill the chip) unless a shorter march is estimated 5% faster, because
+// the grid would leave compute units idle. Stage 1 / stage 2 measured at the pick
+// against `most` = 16 (µs): 60×52×44 f64 exact 21/23 (1 plane) for 97/102; 96³ f64 exact 60/64
+// (5) for 96/102; 171×130×97 f32 exact 97/107 (10) for 117/129; 128³ and 256³ keep 16 ± 5%.
+inline int march_planes(long long columns, int nz, int most, int per_cu, int cus, double* cost = nullptr) {
+  int best = most < nz ? most : nz;
+  double c = march_cost(columns * ((nz + best - 1) / best), best, per_cu, cus);
+  const double limit = 0.95 * c;
+  for (int z = best - 1; z >= 1; --z) {
+    const double cz = march_cost(columns * ((nz + z - 1) / z), z, per_cu, cus);
+    if (cz < limit && cz < c) {
+      c = cz;
+      best = z;
+    }
+  }
+  if (cost) *cost = c;
+  return best;
+}
+
+// Compute units of `device` (256 on MI355X; also if the query fails).
+inline int cu_count(int device) {
+  int n = 0;
+  return hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && n > 0 ? n : 256;
+}
+
 // Clock kernels of the uniform-grid context, shared with the block context.
 // clock: [0] t, [1] dt, [2] max CFL term, [3] steps.
 void enqueue_dt_finalize(hipStream_t s, const double* partials, int np, double cfl, double tfinal, int clip,

@@ -228,7 +228,6 @@ int vh_muscl_create(vh_muscl** out, const int32_t* dims, int32_t ng, double gamm
   vh_muscl* m = new vh_muscl();
   for (int d = 0; d < 3; ++d) m->G.n[d] = dims[d];
   m->G.ng = ng;
-  m->G.zchunk = 8;
   m->G.xcd_remap = 1;
   m->G.ncell = n;
   m->G.gamma = gamma;
@@ -240,11 +239,17 @@ int vh_muscl_create(vh_muscl** out, const int32_t* dims, int32_t ng, double gamm
   m->dtype = dtype;
   m->esize = dtype == VH_F64 ? 8 : 4;
   m->variant = 0;
-  set_tiles(m);
   if (hipGetDevice(&m->device) != hipSuccess) {
     delete m;
     return fail(-2, "no HIP device%s", "");
   }
+  // 16×16 tiles; planes per workgroup from the grid's size (at most 8; Float64 runs two
+  // workgroups per compute unit, Float32 four). Step times at the pick against 8
+  // planes (µs): 48×42×36 f64 dual, recording 42 (1) for 185; 72³ f64 fast 71 (4) for 98;
+  // 108×100×90 f32 113 (6) for 139; 136³ f64 and 264³ keep 8 ± 5%.
+  const long long columns = (long long)((dims[0] + 15) / 16) * ((dims[1] + 15) / 16);
+  m->G.zchunk = march_planes(columns, dims[2], 8, dtype == VH_F64 ? 2 : 4, cu_count(m->device));
+  set_tiles(m);
   const size_t bytes = (size_t)5 * n * m->esize;
   if (hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess || hipMalloc(&m->U, bytes) != hipSuccess ||
       hipMalloc(&m->U1, bytes) != hipSuccess || hipMalloc(&m->partials, sizeof(double) * kWsWgs) != hipSuccess) {
