@@ -174,6 +174,27 @@ def test_single_rate_evolve_bitwise(O, name):
     s.close()
 
 
+@pytest.mark.parametrize("graph", [True, False])
+def test_evolve_in_legs_bitwise(O, graph):
+    """Steps queued past a leg's end time do nothing, and a captured step serves legs
+    of other end times: three legs (one cut by max_steps) against the step-by-step loop."""
+    m = random_mesh(6, seed=4, rank=2, edges=(8, 16))
+    bo = O.BlockOracle(m)
+    U = _state(m, np.float64, seed=8)
+    s = _sim(m, np.float64, use_graph=graph)
+    s.upload(U)
+    t = 0.0
+    for tf, most in ((0.011, 0), (0.05, 5), (0.043, 0)):
+        k = 0
+        while t < tf * (1 - 1e-12) and (most <= 0 or k < most):
+            dt = min(bo.compute_dt(U, 0.3), tf - t)
+            bo.step(U, dt)
+            t, k = t + dt, k + 1
+        assert s.evolve(tf, max_steps=most) == (t, k)
+        np.testing.assert_array_equal(s.state(), U)
+    s.close()
+
+
 def test_launch_shapes_and_methods_agree(O):
     """zchunk, the workgroup cap, graphs and the per-block launch loop all give
     the same bits as the oracle."""

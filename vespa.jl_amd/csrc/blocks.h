@@ -120,7 +120,7 @@ __device__ __forceinline__ Prim<T> link_face_state(const T* __restrict__ U, long
 template <typename T, bool FLOOR64>
 __global__ void __launch_bounds__(256) link_flux_kernel(const T* __restrict__ U, BlocksDev B, T* __restrict__ F) {
   const int f = blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= B.nfaces) return;
+  if (f >= B.nfaces || (B.stop && *B.stop != 0.0)) return;
   const LinkFaceDev* L = B.faces + f;
   const int iL = L->iL, iR = L->iR, axis = L->axis;
   const int l0 = L->nL[0], l1 = L->nL[1], r0 = L->nR[0], r1 = L->nR[1];
@@ -181,6 +181,7 @@ template <typename T, int RANK, bool STAGE2, bool FLOOR64, bool GRAV = false, in
 __global__ void __launch_bounds__(CTX ? CTX * CTY : BNT, sizeof(T) == 4 ? VH_BLOCK_MIN_WAVES_F32 : VH_BLOCK_MIN_WAVES) block_stage_kernel(const T* __restrict__ Us, const T* U0, T* Uout,
                                                                        const double* __restrict__ dtp,
                                                                        double* __restrict__ partials, BlocksDev B) {
+  if (B.stop && *B.stop != 0.0) return;
   constexpr int NT = CTX ? CTX * CTY : BNT;   // lanes per workgroup
   constexpr int NW = NT / 64;                 // waves per workgroup
   static_assert(NT % 64 == 0 && NT <= BNT, "tile shape");

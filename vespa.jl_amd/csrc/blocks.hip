@@ -1131,6 +1131,8 @@ struct vh_blocks {
   double* partials = nullptr;
   int npartials = 0;
   double* clock = nullptr;
+  double* clock_host = nullptr;   // pinned copy of the clock, written by its kernels
+  bool in_loop = false;           // kernels of a step loop look at its end flag
   hipStream_t stream = nullptr;
   hipGraphExec_t graph = nullptr;
   int graph_np = -1;
@@ -1177,6 +1179,7 @@ static BlocksDev blocks_dev(const vh_blocks* m) {
   B.igm1 = 1.0 / (m->gamma - 1.0);
   B.ntiles = 0;
   B.nfaces = (int)m->H.faces.size();
+  B.stop = m->in_loop ? m->clock + 7 : nullptr;
   if (m->grav) {
     B.gravg = m->grav->g;
     B.gravG = m->grav->P.G;
@@ -1335,35 +1338,33 @@ static void enqueue_step(vh_blocks* m, int level, double dt_for_regs, const Acti
   }
 }
 
-static int get_clock(vh_blocks* m, double clk[4]) {
-  VH_HIP(hipMemcpyAsync(clk, m->clock, 4 * sizeof(double), hipMemcpyDeviceToHost, m->stream));
-  VH_HIP(hipStreamSynchronize(m->stream));
-  return 0;
-}
-
 static int compute_dt_sync(vh_blocks* m, double cfl, int level, double* dt) {
   enqueue_cfl(m, level);
-  enqueue_dt_finalize(m->stream, m->partials, kCflWgs, cfl, 0.0, 0, m->clock);
+  enqueue_dt_finalize(m->stream, m->partials, kCflWgs, cfl, m->clock, m->clock_host);
   VH_HIP(hipGetLastError());
-  double clk[4];
-  int rc = get_clock(m, clk);
-  if (rc) return rc;
-  *dt = clk[1];
+  VH_HIP(hipStreamSynchronize(m->stream));
+  *dt = m->clock_host[1];
   return 0;
 }
 
-// Single-rate step body (dt finalize from the partials of the previous stage
-// 2, step, clock advance), optionally replayed from a captured graph.
-static int single_rate_step(vh_blocks* m, double cfl, double tfinal, int clip, int np) {
+// One step of a single-rate loop (enqueue_loop_begin before the first), optionally
+// replayed from a captured graph: the loop's parameters are read from the device
+// clock, so one capture serves every loop.
+static int single_rate_step(vh_blocks* m) {
   const ActiveRegs none{};
+  const int np = list_wgs(m, 0);
+  auto enqueue = [&]() {
+    m->in_loop = true;
+    enqueue_step(m, -1, 0.0, none);
+    m->in_loop = false;
+    enqueue_step_tail(m->stream, m->partials, np, m->clock, m->clock_host);
+  };
   if (m->use_graph) {
     if (!m->graph || m->graph_np != np) {
       drop_graph(m);
       hipGraph_t gr = nullptr;
       VH_HIP(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
-      enqueue_dt_finalize(m->stream, m->partials, np, cfl, tfinal, clip, m->clock);
-      enqueue_step(m, -1, 0.0, none);
-      enqueue_advance_clock(m->stream, m->clock);
+      enqueue();
       VH_HIP(hipStreamEndCapture(m->stream, &gr));
       hipError_t e = hipGraphInstantiate(&m->graph, gr, nullptr, nullptr, 0);
       (void)hipGraphDestroy(gr);
@@ -1372,9 +1373,7 @@ static int single_rate_step(vh_blocks* m, double cfl, double tfinal, int clip, i
     }
     VH_HIP(hipGraphLaunch(m->graph, m->stream));
   } else {
-    enqueue_dt_finalize(m->stream, m->partials, np, cfl, tfinal, clip, m->clock);
-    enqueue_step(m, -1, 0.0, none);
-    enqueue_advance_clock(m->stream, m->clock);
+    enqueue();
   }
   VH_HIP(hipGetLastError());
   return 0;
@@ -1803,7 +1802,8 @@ int vh_blocks_create(vh_blocks** out, int32_t rank, int32_t nblocks, int32_t max
   const long long n = m->T.off[m->T.nb];
   const size_t bytes = (size_t)5 * n * m->esize;
   if (hipMalloc(&m->U, bytes) != hipSuccess || hipMalloc(&m->U1, bytes) != hipSuccess ||
-      hipMalloc(&m->clock, 4 * sizeof(double)) != hipSuccess) {
+      hipMalloc(&m->clock, kClockDoubles * sizeof(double)) != hipSuccess ||
+      hipHostMalloc(&m->clock_host, kClockDoubles * sizeof(double)) != hipSuccess) {
     vh_blocks_destroy(m);
     return fail(-2, "device allocation of %s%lld bytes failed", "", (long long)(2 * bytes));
   }
@@ -1811,7 +1811,7 @@ int vh_blocks_create(vh_blocks** out, int32_t rank, int32_t nblocks, int32_t max
   rc = upload_tables(m, m->H, m->T.nb, 0);
   if (!rc) rc = alloc_partials(m);
   if (rc) { vh_blocks_destroy(m); return rc; }
-  VH_HIP(hipMemsetAsync(m->clock, 0, 4 * sizeof(double), m->stream));
+  VH_HIP(hipMemsetAsync(m->clock, 0, kClockDoubles * sizeof(double), m->stream));
   VH_HIP(hipMemsetAsync(m->U, 0, bytes, m->stream));
   VH_HIP(hipStreamSynchronize(m->stream));
   *out = m;
@@ -1830,6 +1830,7 @@ int vh_blocks_destroy(vh_blocks* m) {
   (void)hipFree(m->U1);
   (void)hipFree(m->partials);
   (void)hipFree(m->clock);
+  if (m->clock_host) (void)hipHostFree(m->clock_host);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;
   return 0;
@@ -1887,8 +1888,6 @@ int vh_blocks_run(vh_blocks* m, double cfl, double tfinal, int64_t max_steps, in
   if (!clip && max_steps <= 0) return fail(-1, "need tfinal > 0 or max_steps > 0%s", "");
   if (subcycle && !clip) return fail(-1, "subcycling needs tfinal > 0%s", "");
   VH_HIP(hipSetDevice(m->device));
-  double clk[4] = {*t_io, 0.0, 0.0, 0.0};
-  VH_HIP(hipMemcpyAsync(m->clock, clk, sizeof clk, hipMemcpyHostToDevice, m->stream));
   int64_t k = 0;
   double t = *t_io;
   int rc = 0;
@@ -1911,16 +1910,19 @@ int vh_blocks_run(vh_blocks* m, double cfl, double tfinal, int64_t max_steps, in
       t += dt;
       ++k;
     }
-    clk[0] = t;
-    clk[3] = (double)k;
-    VH_HIP(hipMemcpyAsync(m->clock, clk, sizeof clk, hipMemcpyHostToDevice, m->stream));
     VH_HIP(hipStreamSynchronize(m->stream));
   } else {
     enqueue_cfl(m, -1);
-    int np = kCflWgs;
-    while (true) {
-      if (max_steps > 0 && k >= max_steps) break;
-      if (clip && !(t < tfinal * (1 - 1e-12))) break;
+    enqueue_loop_begin(m->stream, m->partials, kCflWgs, t, cfl, tfinal, clip, m->clock);
+    const int64_t limit = max_steps > 0 ? max_steps : INT64_MAX;
+    int64_t queued = 0;
+    double* clk = m->clock_host;
+    clk[0] = t;
+    clk[3] = 0.0;
+    clk[7] = clip && !(t < tfinal * (1 - 1e-12)) ? 1.0 : 0.0;
+    while (queued < limit && clk[7] == 0.0) {
+      int64_t n = loop_chunk(clip, limit - queued, queued ? clk : nullptr);
+      const int saved = m->use_graph;
       if (m->grav) {
         // solve_poisson! before each step (src/driver.jl:498), g held over the step;
         // the CG loop synchronises, so these steps are enqueued eagerly
@@ -1929,23 +1931,17 @@ int vh_blocks_run(vh_blocks* m, double cfl, double tfinal, int64_t max_steps, in
         m->grav->B.rho = m->U;
         if ((rc = grav_csr_solve(m->stream, m->dtype, m->grav->A, m->grav->P, m->grav->B, &it, &rr))) return rc;
         enqueue_grav_accel(m);
-        const int saved = m->use_graph;
         m->use_graph = 0;
-        rc = single_rate_step(m, cfl, tfinal, clip ? 1 : 0, np);
-        m->use_graph = saved;
-        if (rc) return rc;
-      } else if ((rc = single_rate_step(m, cfl, tfinal, clip ? 1 : 0, np))) {
-        return rc;
+        n = 1;
       }
-      np = list_wgs(m, 0);
-      ++k;
-      if (clip) {
-        if ((rc = get_clock(m, clk))) return rc;
-        t = clk[0];
-      }
+      for (int64_t i = 0; i < n && !rc; ++i) rc = single_rate_step(m);
+      m->use_graph = saved;
+      if (rc) return rc;
+      queued += n;
+      if (clip || queued >= limit) VH_HIP(hipStreamSynchronize(m->stream));
     }
-    if ((rc = get_clock(m, clk))) return rc;
     t = clk[0];
+    k = (int64_t)clk[3];
   }
   *t_io = t;
   if (steps) *steps = k;
@@ -2321,27 +2317,25 @@ int vh_blocks_time_steps(vh_blocks* m, double cfl, int64_t nsteps, int32_t metho
   const int saved_graph = m->use_graph;
   m->use_graph = method == 2;
   const ActiveRegs none{};
-  const int np_steady = method == 1 ? m->H.block_tile_start[m->T.nb] : list_wgs(m, 0);
-  auto one_step = [&](int np) -> int {
+  auto one_step = [&]() -> int {
     if (method == 1) {
-      enqueue_dt_finalize(m->stream, m->partials, np, cfl, 0.0, 0, m->clock);
       enqueue_step(m, -1, 0.0, none, true);
-      enqueue_advance_clock(m->stream, m->clock);
+      enqueue_step_tail(m->stream, m->partials, m->H.block_tile_start[m->T.nb], m->clock, nullptr);
       VH_HIP(hipGetLastError());
       return 0;
     }
-    return single_rate_step(m, cfl, 0.0, 0, np);
+    return single_rate_step(m);
   };
-  // two untimed steps: the first reduces the CFL partials of the initial state,
-  // the second builds the steady-state graph when graphs are used
+  // two untimed steps (the first builds the graph when graphs are used)
   enqueue_cfl(m, -1);
-  int rc = one_step(kCflWgs);
-  if (!rc) rc = one_step(np_steady);
+  enqueue_loop_begin(m->stream, m->partials, kCflWgs, 0.0, cfl, 0.0, false, m->clock);
+  int rc = one_step();
+  if (!rc) rc = one_step();
   hipEvent_t e0 = nullptr, e1 = nullptr;
   float tot = 0;
   if (!rc && hipEventCreate(&e0) == hipSuccess && hipEventCreate(&e1) == hipSuccess) {
     (void)hipEventRecord(e0, m->stream);
-    for (int64_t k = 0; k < nsteps && !rc; ++k) rc = one_step(np_steady);
+    for (int64_t k = 0; k < nsteps && !rc; ++k) rc = one_step();
     (void)hipEventRecord(e1, m->stream);
     hipError_t e = hipStreamSynchronize(m->stream);
     if (!rc && e != hipSuccess) rc = fail(-2, "HIP error %s while timing%s", hipGetErrorString(e));
@@ -2357,9 +2351,8 @@ int vh_blocks_time_steps(vh_blocks* m, double cfl, int64_t nsteps, int32_t metho
     for (auto& e : ev)
       if (hipEventCreate(&e) != hipSuccess) rc = fail(-2, "hipEventCreate failed%s", "");
     for (int k = 0; k < k2 && !rc; ++k) {
-      enqueue_dt_finalize(m->stream, m->partials, list_wgs(m, 0), cfl, 0.0, 0, m->clock);
       enqueue_step(m, -1, 0.0, none, false, ev[2 * k], ev[2 * k + 1]);
-      enqueue_advance_clock(m->stream, m->clock);
+      enqueue_step_tail(m->stream, m->partials, list_wgs(m, 0), m->clock, nullptr);
     }
     hipError_t e = hipStreamSynchronize(m->stream);
     if (!rc && e != hipSuccess) rc = fail(-2, "HIP error %s while timing%s", hipGetErrorString(e));

@@ -53,6 +53,7 @@ struct GridDev {
   int gper;        // bit d: φ periodic along axis d
   int pad_;
   const void* pg;  // ParentGhost states (5 Tf primitives per boundary face slot) or null
+  const double* stop;  // step loops: non-zero once the loop has ended (the stage does nothing), or null
 };
 
 // ---- batched blocks (block-structured AMR) ----
@@ -136,6 +137,7 @@ struct BlocksDev {
   long long ncell;
   double gamma, igm1;
   double gravG;            // gravitational constant (self-gravity)
+  const double* stop;      // as GridDev::stop
   int ntiles;
   int nfaces;
 };

@@ -60,11 +60,23 @@ inline int cu_count(int device) {
 }
 
 // Clock kernels of the uniform-grid context, shared with the block context.
-// clock: [0] t, [1] dt, [2] max CFL term, [3] steps.
-void enqueue_dt_finalize(hipStream_t s, const double* partials, int np, double cfl, double tfinal, int clip,
-                         double* clock);
+// clock (kClockDoubles): [0] t, [1] dt, [2] max CFL term, [3] steps; of a step loop also
+// [4] cfl, [5] tfinal (infinite: no clip), [6] the time at which the loop ends, [7] non-zero
+// once it has ended. `host` is pinned memory that receives a copy (null: none).
+constexpr int kClockDoubles = 8;
+void enqueue_dt_finalize(hipStream_t s, const double* partials, int np, double cfl, double* clock, double* host);
 void enqueue_set_dt(hipStream_t s, double* clock, double dt);
-void enqueue_advance_clock(hipStream_t s, double* clock);
+// A step loop: begin sets the clock from the CFL partials of the current state; a
+// tail after each step's stage 2 advances the clock and sets the next dt from the
+// partials of the new state (and stores it to *dt_log unless null).
+void enqueue_loop_begin(hipStream_t s, const double* partials, int np, double t, double cfl, double tfinal, bool clip,
+                        double* clock, double* dt_log = nullptr);
+void enqueue_step_tail(hipStream_t s, const double* partials, int np, double* clock, double* host,
+                       double* dt_log = nullptr);
+// Steps to queue before the host looks at the clock again: all that are left without
+// a final time; with one, 8 before the first look (clk null) and then as many as the
+// remaining time holds at the current dt, at most 64. Steps queued beyond the end do nothing.
+long long loop_chunk(bool clip, long long left, const double* clk);
 
 }  // namespace vh
 

@@ -287,6 +287,7 @@ template <typename T, int RANK, int TX, int TY, bool STAGE2, bool FLOOR64, bool 
 __global__ void __launch_bounds__(TX* TY, sizeof(T) == 4 ? VH_MIN_WAVES_F32 : VH_MIN_WAVES) rk_stage_kernel(const T* __restrict__ Us, const T* U0,
                                                           T* Uout, const double* __restrict__ dtp,
                                                           double* __restrict__ partials, GridDev G) {
+  if (G.stop && *G.stop != 0.0) return;
   constexpr int NT = TX * TY;
   __shared__ PlaneLDS<T, TX, TY, RANK> S;
   using L_ = PlaneLDS<T, TX, TY, RANK>;

@@ -37,28 +37,77 @@ int fail(int code, const char* fmt, const char* a, long long b) {
 // ----------------------------------------------------------------------------
 // reductions
 
-// clock: [0] t, [1] dt, [2] invdt, [3] steps (as double)
-__global__ void __launch_bounds__(256) dt_finalize_kernel(const double* __restrict__ partials, int np,
-                                                          double cfl, double tfinal, int clip,
-                                                          double* clock) {
-  __shared__ double red[16];
+// Reductions of the CFL partials and the clock (layout in host.h). One workgroup of
+// 1024 lanes: a 256³ grid leaves 4096 partials, four loads per lane.
+constexpr int kClockLanes = 1024;
+
+__device__ __forceinline__ double partials_max(const double* __restrict__ partials, int np, double* red) {
   double m = 0.0;
-  for (int i = threadIdx.x; i < np; i += 256) m = vmax(m, partials[i]);
-  m = block_max<256>(m, red);
+  for (int i = threadIdx.x; i < np; i += kClockLanes) m = vmax(m, partials[i]);
+  return block_max<kClockLanes>(m, red);
+}
+
+__device__ __forceinline__ void clock_to_host(const double* clock, double* host) {
+  if (host)
+    for (int i = 0; i < kClockDoubles; ++i) host[i] = clock[i];
+}
+
+// Next dt of a step loop from the largest CFL term m; ends the loop at its end time.
+__device__ __forceinline__ void clock_next(double* clock, double m, double* dt_log) {
+  const double tfinal = clock[5];
+  double dt = m == 0.0 ? HUGE_VAL : clock[4] / m;
+  if (tfinal < HUGE_VAL) {
+    dt = vmin(dt, tfinal - clock[0]);
+    if (!(clock[0] < clock[6])) clock[7] = 1.0;
+  }
+  clock[1] = dt;
+  clock[2] = m;
+  if (dt_log) *dt_log = dt;
+}
+
+__global__ void __launch_bounds__(kClockLanes) dt_finalize_kernel(const double* __restrict__ partials, int np,
+                                                                  double cfl, double* clock, double* host) {
+  __shared__ double red[kClockLanes / 64];
+  const double m = partials_max(partials, np, red);
   if (threadIdx.x == 0) {
-    double dt = m == 0.0 ? HUGE_VAL : cfl / m;
-    if (clip) dt = vmin(dt, tfinal - clock[0]);
-    clock[1] = dt;
+    clock[1] = m == 0.0 ? HUGE_VAL : cfl / m;
     clock[2] = m;
+    clock_to_host(clock, host);
+  }
+}
+
+__global__ void __launch_bounds__(kClockLanes) loop_begin_kernel(const double* __restrict__ partials, int np, double t,
+                                                                 double cfl, double tfinal, double tstop, double* clock,
+                                                                 double* dt_log) {
+  __shared__ double red[kClockLanes / 64];
+  const double m = partials_max(partials, np, red);
+  if (threadIdx.x == 0) {
+    clock[0] = t;
+    clock[3] = 0.0;
+    clock[4] = cfl;
+    clock[5] = tfinal;
+    clock[6] = tstop;
+    clock[7] = 0.0;
+    clock_next(clock, m, dt_log);
+  }
+}
+
+// One launch after stage 2 in place of a clock-advance, a dt-reduction and a copy of
+// the clock to the host (2.7 + 3.1 + 3.0 µs and their gaps per step).
+__global__ void __launch_bounds__(kClockLanes) step_tail_kernel(const double* __restrict__ partials, int np,
+                                                                double* clock, double* host, double* dt_log) {
+  __shared__ double red[kClockLanes / 64];
+  if (clock[7] != 0.0) return;
+  const double m = partials_max(partials, np, red);
+  if (threadIdx.x == 0) {
+    clock[0] = clock[0] + clock[1];
+    clock[3] = clock[3] + 1.0;
+    clock_next(clock, m, dt_log);
+    clock_to_host(clock, host);
   }
 }
 
 __global__ void set_dt_kernel(double* clock, double dt) { clock[1] = dt; }
-
-__global__ void advance_clock_kernel(double* clock) {
-  clock[0] = clock[0] + clock[1];
-  clock[3] = clock[3] + 1.0;
-}
 
 template <typename T>
 __global__ void __launch_bounds__(256) totals_kernel(const T* __restrict__ U, long long n, double V,
@@ -88,15 +137,28 @@ __global__ void sub_kernel(const T* __restrict__ a, const T* __restrict__ b, T* 
   if (i < n) out[i] = a[i] - b[i];
 }
 
-void enqueue_dt_finalize(hipStream_t s, const double* partials, int np, double cfl, double tfinal, int clip,
-                         double* clock) {
-  hipLaunchKernelGGL(dt_finalize_kernel, dim3(1), dim3(256), 0, s, partials, np, cfl, tfinal, clip, clock);
+void enqueue_dt_finalize(hipStream_t s, const double* partials, int np, double cfl, double* clock, double* host) {
+  hipLaunchKernelGGL(dt_finalize_kernel, dim3(1), dim3(kClockLanes), 0, s, partials, np, cfl, clock, host);
 }
 void enqueue_set_dt(hipStream_t s, double* clock, double dt) {
   hipLaunchKernelGGL(set_dt_kernel, dim3(1), dim3(1), 0, s, clock, dt);
 }
-void enqueue_advance_clock(hipStream_t s, double* clock) {
-  hipLaunchKernelGGL(advance_clock_kernel, dim3(1), dim3(1), 0, s, clock);
+void enqueue_loop_begin(hipStream_t s, const double* partials, int np, double t, double cfl, double tfinal, bool clip,
+                        double* clock, double* dt_log) {
+  hipLaunchKernelGGL(loop_begin_kernel, dim3(1), dim3(kClockLanes), 0, s, partials, np, t, cfl,
+                     clip ? tfinal : HUGE_VAL, tfinal * (1 - 1e-12), clock, dt_log);
+}
+void enqueue_step_tail(hipStream_t s, const double* partials, int np, double* clock, double* host, double* dt_log) {
+  hipLaunchKernelGGL(step_tail_kernel, dim3(1), dim3(kClockLanes), 0, s, partials, np, clock, host, dt_log);
+}
+long long loop_chunk(bool clip, long long left, const double* clk) {
+  if (!clip) return left;
+  double n = 8.0;
+  if (clk) {
+    n = std::ceil((clk[5] - clk[0]) / clk[1]);
+    n = n >= 1.0 ? std::min(n, 64.0) : 1.0;   // also for a NaN
+  }
+  return std::min<long long>(left, (long long)n);
 }
 
 }  // namespace vh
@@ -124,6 +186,7 @@ struct vh_grid {
   double* partials;
   int npartials;
   double* clock;
+  double* clock_host;    // pinned copy of the clock, written by its kernels
   double* totals_partials;
   hipStream_t stream;
   struct AdjWork* adj;   // reverse-mode work buffers (allocated on first use)
@@ -259,14 +322,13 @@ static void enqueue_cfl(vh_grid* g) {
 
 // One RK2 step reading dt from clock[1]; stage 2 leaves the partial CFL maxima
 // of the new state in g->partials (g->stage_blocks entries). Optional events
-// bracket the two stage kernels.
+// bracket the two stage kernels. In a step loop a tail follows.
 static void enqueue_step(vh_grid* g, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr, hipEvent_t e2 = nullptr) {
   if (e0) (void)hipEventRecord(e0, g->stream);
   enqueue_stage(g, false, g->U, g->U, g->U1);
   if (e1) (void)hipEventRecord(e1, g->stream);
   enqueue_stage(g, true, g->U1, g->U, g->U);
   if (e2) (void)hipEventRecord(e2, g->stream);
-  hipLaunchKernelGGL(advance_clock_kernel, dim3(1), dim3(1), 0, g->stream, g->clock);
 }
 
 extern "C" {
@@ -537,7 +599,8 @@ int vh_grid_create(vh_grid** out, int32_t rank, const int64_t* dims, const doubl
   if (rc) { vh_grid_destroy(g); return rc; }
   const size_t bytes = (size_t)5 * n * g->esize;
   if (hipMalloc(&g->U, bytes) != hipSuccess || hipMalloc(&g->U1, bytes) != hipSuccess ||
-      hipMalloc(&g->clock, 4 * sizeof(double)) != hipSuccess ||
+      hipMalloc(&g->clock, kClockDoubles * sizeof(double)) != hipSuccess ||
+      hipHostMalloc(&g->clock_host, kClockDoubles * sizeof(double)) != hipSuccess ||
       hipMalloc(&g->totals_partials, 5 * kMaxCflBlocks * sizeof(double)) != hipSuccess) {
     vh_grid_destroy(g);
     return fail(-2, "device allocation of %s%lld bytes failed", "", (long long)(2 * bytes));
@@ -546,7 +609,7 @@ int vh_grid_create(vh_grid** out, int32_t rank, const int64_t* dims, const doubl
     vh_grid_destroy(g);
     return fail(-2, "stream creation failed%s", "");
   }
-  VH_HIP(hipMemsetAsync(g->clock, 0, 4 * sizeof(double), g->stream));
+  VH_HIP(hipMemsetAsync(g->clock, 0, kClockDoubles * sizeof(double), g->stream));
   VH_HIP(hipMemsetAsync(g->U, 0, bytes, g->stream));
   VH_HIP(hipStreamSynchronize(g->stream));
   const long long cb = (n + 255) / 256;
@@ -566,6 +629,7 @@ int vh_grid_destroy(vh_grid* g) {
   if (g->U1) (void)hipFree(g->U1);
   if (g->partials) (void)hipFree(g->partials);
   if (g->clock) (void)hipFree(g->clock);
+  if (g->clock_host) (void)hipHostFree(g->clock_host);
   if (g->totals_partials) (void)hipFree(g->totals_partials);
   if (g->pg) (void)hipFree(g->pg);
   if (g->stream) (void)hipStreamDestroy(g->stream);
@@ -625,13 +689,10 @@ int vh_grid_compute_dt(vh_grid* g, double cfl, double* dt) {
   if (!g || !dt) return fail(-1, "null argument%s", "");
   VH_HIP(hipSetDevice(g->device));
   enqueue_cfl(g);
-  hipLaunchKernelGGL(dt_finalize_kernel, dim3(1), dim3(256), 0, g->stream, g->partials, g->cfl_blocks, cfl, 0.0,
-                     0, g->clock);
+  enqueue_dt_finalize(g->stream, g->partials, g->cfl_blocks, cfl, g->clock, g->clock_host);
   VH_HIP(hipGetLastError());
-  double clk[4];
-  VH_HIP(hipMemcpyAsync(clk, g->clock, sizeof clk, hipMemcpyDeviceToHost, g->stream));
   VH_HIP(hipStreamSynchronize(g->stream));
-  *dt = clk[1];
+  *dt = g->clock_host[1];
   return 0;
 }
 
@@ -672,38 +733,36 @@ int vh_grid_run(vh_grid* g, double cfl, double tfinal, int64_t max_steps, double
   if (!clip && max_steps <= 0) return fail(-1, "need tfinal > 0 or max_steps > 0%s", "");
   if (int rc = need_parent_states(g)) return rc;
   VH_HIP(hipSetDevice(g->device));
-  double clk[4] = {*t_io, 0.0, 0.0, 0.0};
-  VH_HIP(hipMemcpyAsync(g->clock, clk, sizeof clk, hipMemcpyHostToDevice, g->stream));
-  int64_t k = 0;
   enqueue_cfl(g);   // CFL partials of the current state
-  int np = g->cfl_blocks;
-  double t = *t_io;
-  while (true) {
-    if (max_steps > 0 && k >= max_steps) break;
-    if (clip && !(t < tfinal * (1 - 1e-12))) break;
+  enqueue_loop_begin(g->stream, g->partials, g->cfl_blocks, *t_io, cfl, tfinal, clip, g->clock);
+  const int64_t limit = max_steps > 0 ? max_steps : INT64_MAX;
+  int64_t queued = 0;
+  double* clk = g->clock_host;
+  clk[0] = *t_io;
+  clk[3] = 0.0;
+  clk[7] = clip && !(*t_io < tfinal * (1 - 1e-12)) ? 1.0 : 0.0;
+  while (queued < limit && clk[7] == 0.0) {
+    int64_t n = loop_chunk(clip, limit - queued, queued ? clk : nullptr);
     if (g->grav) {   // φ(ρⁿ), held over the step (src/driver.jl:498)
       long long it;
       double rr;
       g->grav->B.rho = g->U;
       int rc = grav_solve(g->stream, g->dtype == VH_F64 ? 0 : 1, g->G, g->grav->P, g->grav->B, &it, &rr);
       if (rc) return rc;
+      n = 1;
     }
-    hipLaunchKernelGGL(dt_finalize_kernel, dim3(1), dim3(256), 0, g->stream, g->partials, np, cfl, tfinal,
-                       clip ? 1 : 0, g->clock);
-    enqueue_step(g);
+    g->G.stop = g->clock + 7;
+    for (int64_t i = 0; i < n; ++i) {
+      enqueue_step(g);
+      enqueue_step_tail(g->stream, g->partials, g->stage_blocks, g->clock, g->clock_host);
+    }
+    g->G.stop = nullptr;
+    queued += n;
     VH_HIP(hipGetLastError());
-    np = g->stage_blocks;
-    ++k;
-    if (clip) {
-      VH_HIP(hipMemcpyAsync(clk, g->clock, sizeof clk, hipMemcpyDeviceToHost, g->stream));
-      VH_HIP(hipStreamSynchronize(g->stream));
-      t = clk[0];
-    }
+    if (clip || queued >= limit) VH_HIP(hipStreamSynchronize(g->stream));
   }
-  VH_HIP(hipMemcpyAsync(clk, g->clock, sizeof clk, hipMemcpyDeviceToHost, g->stream));
-  VH_HIP(hipStreamSynchronize(g->stream));
   *t_io = clk[0];
-  if (steps) *steps = k;
+  if (steps) *steps = (int64_t)clk[3];
   return 0;
 }
 
@@ -888,12 +947,10 @@ int vh_grid_time_steps(vh_grid* g, double cfl, int64_t nsteps, double* ms_stage1
     if (hipEventCreate(&ev[i]) != hipSuccess) rc = fail(-2, "hipEventCreate failed%s", "");
   if (!rc) {
     enqueue_cfl(g);
-    int np = g->cfl_blocks;
+    enqueue_loop_begin(g->stream, g->partials, g->cfl_blocks, 0.0, cfl, 0.0, false, g->clock);
     for (int64_t k = 0; k < nsteps; ++k) {
-      hipLaunchKernelGGL(dt_finalize_kernel, dim3(1), dim3(256), 0, g->stream, g->partials, np, cfl, 0.0, 0,
-                         g->clock);
       enqueue_step(g, ev[3 * k], ev[3 * k + 1], ev[3 * k + 2]);
-      np = g->stage_blocks;
+      enqueue_step_tail(g->stream, g->partials, g->stage_blocks, g->clock, nullptr);
     }
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(g->stream);
@@ -930,7 +987,6 @@ int vh_grid_time_steps(vh_grid* g, double cfl, int64_t nsteps, double* ms_stage1
 
 namespace vh {
 __global__ void set_value_kernel(double* p, double v) { *p = v; }
-__global__ void copy_value_kernel(const double* src, double* dst) { *dst = *src; }
 }  // namespace vh
 
 struct AdjWork {
@@ -1142,14 +1198,12 @@ int vh_adjoint_forward(vh_adjoint* a, double cfl) {
   VH_HIP(hipEventRecord(e0, g->stream));
   VH_HIP(hipMemcpyAsync(a->ckpt, g->U, nb, hipMemcpyDeviceToDevice, g->stream));
   enqueue_cfl(g);
-  int np = g->cfl_blocks;
+  enqueue_loop_begin(g->stream, g->partials, g->cfl_blocks, 0.0, cfl, 0.0, false, g->clock, a->dts);
   // The last segment's states are kept as the forward run produces them (the
   // backward pass starts there and needs no recompute for it).
   const size_t n5 = 5 * (size_t)g->G.ncell;
   const int64_t klast = (int64_t)(a->nseg - 1) * a->every;
   for (int64_t k = 0; k < a->nsteps; ++k) {
-    hipLaunchKernelGGL(dt_finalize_kernel, dim3(1), dim3(256), 0, g->stream, g->partials, np, cfl, 0.0, 0, g->clock);
-    hipLaunchKernelGGL(copy_value_kernel, dim3(1), dim3(1), 0, g->stream, g->clock + 1, a->dts + k);
     if (k < klast) {
       enqueue_step(g);
     } else {
@@ -1160,9 +1214,9 @@ int vh_adjoint_forward(vh_adjoint* a, double cfl) {
       double* Un = k + 1 < a->nsteps ? a->segL + n5 * (j + 1) : (double*)g->U;
       enqueue_stage(g, false, Uk, Uk, U1k);
       enqueue_stage(g, true, U1k, Uk, Un);
-      hipLaunchKernelGGL(advance_clock_kernel, dim3(1), dim3(1), 0, g->stream, g->clock);
     }
-    np = g->stage_blocks;
+    enqueue_step_tail(g->stream, g->partials, g->stage_blocks, g->clock, nullptr,
+                      k + 1 < a->nsteps ? a->dts + k + 1 : nullptr);
     if ((k + 1) % a->every == 0 && k + 1 < a->nsteps)
       VH_HIP(hipMemcpyAsync((char*)a->ckpt + nb * ((k + 1) / a->every), g->U, nb, hipMemcpyDeviceToDevice, g->stream));
   }
