@@ -1976,7 +1976,7 @@ int vh_blocks_enable_gravity(vh_blocks* m, double G, int64_t maxiter, double tol
   if (e == hipSuccess) e = hipMalloc(&Gv->g, 3 * m->esize * n);
   if (e == hipSuccess) e = hipMalloc(&Gv->B.state, kGravStateBytes);
   if (e == hipSuccess) e = hipMalloc(&Gv->B.scal, 8 * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&Gv->B.partials, 4096 * sizeof(double));
+  if (e == hipSuccess) e = hipMalloc(&Gv->B.partials, kGravPartials * sizeof(double));
   if (e == hipSuccess) e = hipHostMalloc(&Gv->B.host_state, kGravStateBytes, 0);
   if (e == hipSuccess) e = hipMemsetAsync(Gv->B.phi, 0, m->esize * n, m->stream);
   if (e == hipSuccess) e = hipMemsetAsync(Gv->g, 0, 3 * m->esize * n, m->stream);

@@ -109,18 +109,18 @@ struct GravParams {
   int project_mean = 1;
   long long maxiter = 500;
   double tol = 1e-8;
-  int chunk = 16;          // iterations enqueued between host checks
 };
 struct GravBuffers {
   void* phi = nullptr;     // ncell values
-  void* work = nullptr;    // 4·ncell values: r, p, Ap, b
+  void* work = nullptr;    // 4·ncell values: r, two p, Ap (block meshes)
   const void* rho = nullptr;
   void* state = nullptr;   // CG state block (device)
-  double* scal = nullptr;  // 8 scalars (device)
-  double* partials = nullptr;  // 4096 per-workgroup partial sums (device)
-  void* host_state = nullptr;  // pinned copy of the state block
+  double* scal = nullptr;  // [1]: Σ V (device)
+  double* partials = nullptr;  // kGravPartials per-workgroup partial sums (device)
+  void* host_state = nullptr;  // pinned; the kernels write done, iters, relres here
 };
 constexpr int kGravStateBytes = 64;
+constexpr int kGravPartials = 4096;
 void grav_apply(hipStream_t s, int dtype, const GridDev& G, int gper, const void* x, void* out);
 void grav_accel(hipStream_t s, int dtype, const GridDev& G, int gper, const void* phi, void* g);
 int grav_solve(hipStream_t s, int dtype, const GridDev& G, const GravParams& P, GravBuffers& B, long long* iters,

@@ -789,7 +789,7 @@ int vh_grid_enable_gravity(vh_grid* g, double G, int32_t phi_periodic, int64_t m
   if (e == hipSuccess) e = hipMalloc(&w->B.work, 4 * g->esize * n);
   if (e == hipSuccess) e = hipMalloc(&w->B.state, kGravStateBytes);
   if (e == hipSuccess) e = hipMalloc(&w->B.scal, 8 * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&w->B.partials, 4096 * sizeof(double));
+  if (e == hipSuccess) e = hipMalloc(&w->B.partials, kGravPartials * sizeof(double));
   if (e == hipSuccess) e = hipHostMalloc(&w->B.host_state, kGravStateBytes);
   if (e == hipSuccess) e = hipMemsetAsync(w->B.phi, 0, g->esize * n, g->stream);
   if (e == hipSuccess) e = hipMemsetAsync(w->B.scal, 0, 8 * sizeof(double), g->stream);
