@@ -146,6 +146,33 @@ def test_default_march_of_grids_that_do_not_fill_the_chip(V, O, dims, most, dtyp
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n", [1, 2, 3, 63, 64, 1023, 1024, 2039, 2040, 2041])
+@pytest.mark.parametrize("bc", [(0, 0), (1, 2), (2, 1)])
+def test_line_step_loop_bitwise(V, O, n, bc, dtype):
+    """1D runs of one workgroup (one and two items per lane, faces past a full wave, the
+    largest grid it holds and the first it does not): a run cut by max_steps and one
+    that ends at its final time equal the oracle's step-by-step loop."""
+    if n < 2 and bc == (0, 0):
+        pytest.skip("a periodic axis needs two cells")
+    U = random_state((n,), seed=n, dtype=dtype)
+    sim = make_sim(V, (n,), [bc], 1.4, dtype, U)
+    g = oracle_grid(O, (n,), [bc], 1.4)
+    Uo, t, k = U.copy(), 0.0, 0
+    f64 = dtype == np.float32
+    for most, tf in ((3, 1.0), (50, 4.5 * O.compute_dt(g, U, 0.4, floor64=f64))):
+        sim.problem.tfinal = tf
+        done = 0
+        while done < most and t < tf * (1 - 1e-12):
+            dt = min(O.compute_dt(g, Uo, 0.4, floor64=f64), tf - t)
+            O.step(g, Uo, dt, floor64=f64)
+            t, k, done = t + dt, k + 1, done + 1
+        V.evolve(sim, max_steps=most)
+        assert (sim.t, sim.step_count) == (t, k)
+        assert np.array_equal(sim.state(), Uo)
+    sim.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_device_dt_loop_bitwise(V, O, dtype):
     dims = (40, 24, 20)
     bcs = [(0, 0), (2, 2), (1, 1)]

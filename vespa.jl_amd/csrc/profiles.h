@@ -25,6 +25,11 @@ inline TileShape tile_for(int rank, int variant) {
   return kTiles1[variant];
 }
 
+// 1D step loop in one workgroup (line.h): lanes, and the largest grid its LDS holds
+// (10 Float64 values per cell and its face).
+constexpr int kLineLanes = 1024;
+constexpr int kLineMax = 2040;
+
 // Tile shapes the rank-3 block stage kernel is compiled for (class 1..4; one
 // lane per cell). Tiles of any other shape, of rank 1 and 2 meshes and of meshes
 // with self-gravity run the runtime-shape kernel (class 0, 256 lanes).
@@ -44,6 +49,8 @@ inline int block_class_lanes(int cls) { return cls ? kBlockShapes[cls - 1].tx * 
   void launch_stage(int dtype, int rank, int variant, bool stage2, int blocks, hipStream_t s,       \
                     const void* Us, const void* U0, void* Uout, const double* dtp, double* partials, \
                     const GridDev& G);                                                              \
+  void launch_line(int dtype, hipStream_t s, void* U, const GridDev& G, double t, double cfl,       \
+                   double tfinal, double tstop, long long max_steps, double* host);                 \
   void launch_cfl(int dtype, int rank, int blocks, hipStream_t s, const void* U, const GridDev& G,  \
                   double* partials);                                                                \
   void launch_face_flux(int dtype, long long nf, hipStream_t s, const void* WL, const void* WR,     \

@@ -4,6 +4,7 @@
 #include "profiles.h"
 #include "stencil.h"
 #include "blocks.h"
+#include "line.h"
 
 namespace vh {
 namespace VH_PROFILE_NS {
@@ -89,6 +90,24 @@ void launch_stage(int dtype, int rank, int variant, bool stage2, int blocks, hip
     stage_dispatch<double, false>(rank, variant, stage2, blocks, s, Us, U0, Uout, dtp, partials, G);
   else
     stage_dispatch<float, true>(rank, variant, stage2, blocks, s, Us, U0, Uout, dtp, partials, G);
+}
+
+template <typename T, bool FLOOR64>
+static void line_t(hipStream_t s, void* U, const GridDev& G, double t, double cfl, double tfinal, double tstop,
+                   long long max_steps, double* host) {
+  const int items = G.n[0] + 1;
+  if (items <= kLineLanes)
+    hipLaunchKernelGGL((rk_line_kernel<T, FLOOR64, 1>), dim3(1), dim3((items + 63) / 64 * 64), 0, s, (T*)U, G, t, cfl,
+                       tfinal, tstop, max_steps, host);
+  else
+    hipLaunchKernelGGL((rk_line_kernel<T, FLOOR64, 2>), dim3(1), dim3((items + 127) / 128 * 64), 0, s, (T*)U, G, t, cfl,
+                       tfinal, tstop, max_steps, host);
+}
+
+void launch_line(int dtype, hipStream_t s, void* U, const GridDev& G, double t, double cfl, double tfinal,
+                 double tstop, long long max_steps, double* host) {
+  if (dtype == 0) line_t<double, false>(s, U, G, t, cfl, tfinal, tstop, max_steps, host);
+  else line_t<float, true>(s, U, G, t, cfl, tfinal, tstop, max_steps, host);
 }
 
 void launch_cfl(int dtype, int rank, int blocks, hipStream_t s, const void* U, const GridDev& G,

@@ -727,12 +727,41 @@ int vh_grid_step_bflux(vh_grid* g, double dt, void* dbflux) {
   return 0;
 }
 
+// 1D grids that one workgroup holds run their step loop in it (line.h).
+static bool line_fits(const vh_grid* g) {
+  return g->G.rank == 1 && g->G.n[0] <= kLineMax && !g->grav && !has_parent(g);
+}
+
+static int run_line(vh_grid* g, double cfl, double tfinal, int64_t max_steps, double* t_io, int64_t* steps) {
+  const bool clip = tfinal > 0.0;
+  const double tstop = tfinal * (1 - 1e-12);
+  // A launch takes at most this many steps (about 5 ms at 400 cells), so that no kernel
+  // runs unboundedly long.
+  constexpr int64_t kMost = 2048;
+  double* clk = g->clock_host;
+  int64_t k = 0;
+  while ((max_steps <= 0 || k < max_steps) && (!clip || *t_io < tstop)) {
+    const int64_t n = max_steps > 0 ? std::min(max_steps - k, kMost) : kMost;
+    if (g->mode == VH_FAST)
+      fast::launch_line(g->dtype, g->stream, g->U, g->G, *t_io, cfl, clip ? tfinal : HUGE_VAL, tstop, n, clk);
+    else
+      exact::launch_line(g->dtype, g->stream, g->U, g->G, *t_io, cfl, clip ? tfinal : HUGE_VAL, tstop, n, clk);
+    VH_HIP(hipGetLastError());
+    VH_HIP(hipStreamSynchronize(g->stream));
+    *t_io = clk[0];
+    k += (int64_t)clk[3];
+  }
+  if (steps) *steps = k;
+  return 0;
+}
+
 int vh_grid_run(vh_grid* g, double cfl, double tfinal, int64_t max_steps, double* t_io, int64_t* steps) {
   if (!g || !t_io) return fail(-1, "null argument%s", "");
   const bool clip = tfinal > 0.0;
   if (!clip && max_steps <= 0) return fail(-1, "need tfinal > 0 or max_steps > 0%s", "");
   if (int rc = need_parent_states(g)) return rc;
   VH_HIP(hipSetDevice(g->device));
+  if (line_fits(g)) return run_line(g, cfl, tfinal, max_steps, t_io, steps);
   enqueue_cfl(g);   // CFL partials of the current state
   enqueue_loop_begin(g->stream, g->partials, g->cfl_blocks, *t_io, cfl, tfinal, clip, g->clock);
   const int64_t limit = max_steps > 0 ? max_steps : INT64_MAX;
