@@ -57,6 +57,34 @@ def test_step_bitwise(O, dims, ng, dtype, variant):
         g.close()
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_extreme_operands_bitwise(O, dtype):
+    """Quotients by a shared denominator and the limiter where they could go wrong:
+    subnormal quotients and their ties (odd multiples of the least subnormal over even
+    densities), zeros, huge values, and cells holding infinities and NaN."""
+    dims, ng = (20, 18, 17), 3
+    rng = np.random.default_rng(5)
+    n = int(np.prod(dims))
+    least = np.finfo(dtype).smallest_subnormal
+    U = np.empty((5, n), dtype=dtype)
+    U[0] = rng.integers(1, 9, n)
+    for q in (1, 2, 3):
+        kind = rng.integers(0, 4, n)
+        U[q] = np.where(kind == 0, 0.0, np.where(kind == 1, rng.integers(-40, 40, n) * least, np.where(
+            kind == 2, rng.normal(size=n).astype(dtype) * np.finfo(dtype).tiny, rng.normal(size=n))))
+    U[4] = rng.uniform(2.0, 30.0, n)
+    for i, v in enumerate((np.inf, -np.inf, np.nan, np.finfo(dtype).max)):
+        U[i + 1, rng.integers(0, n, 2)] = v
+    g = M.MusclGrid(dims, ng, G14, 1.5, 0.05, 1e-10, eltype=dtype)
+    g.upload(U)
+    with np.errstate(all="ignore"):
+        O.muscl_step_3d(U, dims, ng, 0.004, G14, 1.5, 0.05, 1e-10)
+    g.step(0.004)
+    np.testing.assert_array_equal(g.state(), U)
+    assert np.isfinite(U).mean() > 0.5
+    g.close()
+
+
 def test_reference_driver_cases_bitwise(O):
     """The reference's conservation case (26³ blob, dt 0.02, dx 1, 3 steps) and a
     cold supersonic line (eint floor, zero-sign paths)."""

@@ -21,36 +21,37 @@ struct MuW {
   T r, e, vx, vy, vz;
 };
 
-// _plm_pt (lib/PPMKernels/src/muscl.jl:13-27): v + ½·minmod3((v−vm1)θ, (vp1−v)θ,
-// ½(vp1−vm1)) with Enzo's sign(0) = −1.
+// ½·minmod3(a, b, d), Enzo's 3-argument minmod (lib/PPMKernels/src/muscl.jl:13-19):
+// 0.25·(sa+sb)·|sa+sd|·min(|a|,|b|,|d|) with s = +1 for a positive argument and −1 otherwise. The
+// leading factor is exactly ±1 when the three signs agree and a zero otherwise, so the
+// product is ±½ or 0, selected from the three comparisons, times the minimum (a NaN or
+// an infinite minimum gives what the product gives; zeros may differ in sign).
+__device__ __forceinline__ float half_minmod3(float a, float b, float d) {
+  const bool pa = a > 0.0f, pb = b > 0.0f, pd = d > 0.0f;
+  const float f = pa == pb && pa == pd ? (pa ? 0.5f : -0.5f) : 0.0f;
+  return f * jmin(absT(a), jmin(absT(b), absT(d)));   // one v_minimum3_f32
+}
+// Float64 has no NaN-propagating minimum instruction: v_min_f64 and a NaN factor.
+__device__ __forceinline__ double half_minmod3(double a, double b, double d) {
+  const bool pa = a > 0.0, pb = b > 0.0, pd = d > 0.0;
+  double f = pa == pb && pa == pd ? (pa ? 0.5 : -0.5) : 0.0;
+  f = __builtin_isunordered(a, b) || d != d ? __builtin_nan("") : f;
+  return f * vmin(vmin(absT(a), absT(b)), absT(d));
+}
+// Hi-face value of the middle cell, _plm_pt (lib/PPMKernels/src/muscl.jl:22-27): v + ½·minmod3((v−vm1)θ,
+// (vp1−v)θ, ½(vp1−vm1)).
 template <typename T>
 __device__ __forceinline__ T plm_pt(T vm1, T v, T vp1, T th) {
-  const T a = (v - vm1) * th, b = (vp1 - v) * th, c = T(0.5) * (vp1 - vm1);
-  const T sa = a > T(0) ? T(1) : T(-1), sb = b > T(0) ? T(1) : T(-1), sc = c > T(0) ? T(1) : T(-1);
-  const T s = T(0.25) * (sa + sb) * absT(sa + sc) * jmin(absT(a), jmin(absT(b), absT(c)));
-  return v + T(0.5) * s;
+  return v + half_minmod3((v - vm1) * th, (vp1 - v) * th, T(0.5) * (vp1 - vm1));
 }
-// Both face values of the middle cell at once. The lo-face value is _plm_pt with
-// the neighbours exchanged (the reference's R state); its minmod arguments are the
-// exact negatives of the hi face's in swapped order, so it reuses their magnitudes
-// and minimum and only recomputes the signs: bit-identical to evaluating it anew,
-// zero signs included.
-// The leading factor of minmod3, 0.25·(sa+sb)·|sa+sd| with s = +1 for a positive
-// argument and −1 otherwise, is exactly ±1 when the three signs agree and a zero
-// otherwise: −0 when sa = sb = −1 ≠ sd, +0 in the other cases (the signs the
-// products give). Selected from the comparisons instead of multiplied out.
-template <typename T>
-__device__ __forceinline__ T minmod_factor(bool pa, bool pb, bool pd) {
-  const T full = pa ? T(1) : T(-1);
-  const T zero = pa ? T(0) : T(-0.0);
-  return pa == pb ? (pa == pd ? full : zero) : T(0);
-}
+// Both face values of the middle cell. The lo-face value is _plm_pt with the neighbours
+// exchanged (the reference's R state): its minmod arguments are the exact negatives of
+// the hi face's in swapped order, so its slope term is the negative of the hi face's.
 template <typename T>
 __device__ __forceinline__ void plm_pair(T m, T c, T p, T th, T& hi, T& lo) {
-  const T a = (c - m) * th, b = (p - c) * th, d = T(0.5) * (p - m);
-  const T mn = jmin(absT(a), jmin(absT(b), absT(d)));
-  hi = c + T(0.5) * (minmod_factor<T>(a > T(0), b > T(0), d > T(0)) * mn);
-  lo = c + T(0.5) * (minmod_factor<T>(b < T(0), a < T(0), d < T(0)) * mn);
+  const T s = half_minmod3((c - m) * th, (p - c) * th, T(0.5) * (p - m));
+  hi = c + s;
+  lo = c - s;
 }
 template <typename T>
 __device__ __forceinline__ void face_pair(const MuW<T>& m, const MuW<T>& c, const MuW<T>& p, T th, T sr, MuW<T>& hi,
@@ -76,15 +77,46 @@ __device__ __forceinline__ MuW<T> face_state(const MuW<T>& m, const MuW<T>& c, c
   return o;
 }
 
-// (a⁺F_L + a⁻F_R − a⁺a⁻(U_R − U_L)) / (a⁺ + a⁻); rinv = 1/(a⁺ + a⁻) in the fast profile.
-template <typename T>
-__device__ __forceinline__ T hll1(T ap, T am, T fl, T fr, T ul, T ur, T rinv) {
+// n[i] ← n[i]/d: several quotients by one denominator.
+template <int N, typename T>
+__device__ __forceinline__ void divide_all(T n[N], T d) {
 #if VH_FAST_PROFILE
-  return (ap * fl + am * fr - ap * am * (ur - ul)) * rinv;
+  const T r = fast_rcp(d);
+#pragma unroll
+  for (int i = 0; i < N; ++i) n[i] *= r;
 #else
-  (void)rinv;
-  return (ap * fl + am * fr - ap * am * (ur - ul)) / (ap + am);
+  if constexpr (sizeof(T) == 8) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) n[i] = n[i] / d;
+  } else {
+    // Correctly rounded through one Float64 reciprocal (4 operations per quotient for 11; the
+    // Float64 rate is that of Float32 here). n·r in Float64 is within 2^-51 of n/d, and a
+    // quotient of two 24-bit numbers that is no tie lies at least 2^-49 (relative) from
+    // one, so rounding the product rounds the quotient. A tie is possible only for a
+    // subnormal result: those are divided out. div_fixup gives zero, infinite and NaN
+    // operands their results.
+    const double r = fast_rcp((double)d);
+    T q[N];
+    bool sub = false;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      q[i] = __builtin_amdgcn_div_fixupf((float)((double)n[i] * r), d, n[i]);
+      sub |= __builtin_amdgcn_classf(q[i], 0x090);
+    }
+    if (__builtin_expect(sub, 0)) {
+#pragma unroll 1
+      for (int i = 0; i < N; ++i) q[i] = n[i] / d;
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) n[i] = q[i];
+  }
 #endif
+}
+
+// a⁺F_L + a⁻F_R − a⁺a⁻(U_R − U_L), the numerator of the HLL flux over a⁺ + a⁻
+template <typename T>
+__device__ __forceinline__ T hll1(T ap, T am, T fl, T fr, T ul, T ur) {
+  return ap * fl + am * fr - ap * am * (ur - ul);
 }
 // sqrt(γp/ρ)
 template <typename T>
@@ -114,20 +146,16 @@ __device__ __forceinline__ void hll_rot(const MuW<T>& L, const MuW<T>& R, T g, T
   const T lpr = ur + csr, lmr = ur - csr;
   const T ap = jmax(T(0), jmax(lpl, lpr));
   const T am = jmax(T(0), jmax(-lml, -lmr));
-#if VH_FAST_PROFILE
-  const T rinv = fast_rcp(ap + am);
-#else
-  const T rinv = T(0);
-#endif
-  F[0] = hll1(ap, am, FlD, FrD, rl, rr, rinv);
-  F[1] = hll1(ap, am, FlS1, FrS1, UlS1, UrS1, rinv);
-  F[2] = hll1(ap, am, FlS2, FrS2, UlS2, UrS2, rinv);
-  F[3] = hll1(ap, am, FlS3, FrS3, UlS3, UrS3, rinv);
-  F[4] = hll1(ap, am, FlE, FrE, UlE, UrE, rinv);
+  F[0] = hll1(ap, am, FlD, FrD, rl, rr);
+  F[1] = hll1(ap, am, FlS1, FrS1, UlS1, UrS1);
+  F[2] = hll1(ap, am, FlS2, FrS2, UlS2, UrS2);
+  F[3] = hll1(ap, am, FlS3, FrS3, UlS3, UrS3);
+  F[4] = hll1(ap, am, FlE, FrE, UlE, UrE);
   if constexpr (NF == 6) {   // _hll6's gas-energy flux: U = ρe, F = ρe·u
     const T UlG = rl * el, UrG = rr * er;
-    F[5] = hll1(ap, am, UlG * ul, UrG * ur, UlG, UrG, rinv);
+    F[5] = hll1(ap, am, UlG * ul, UrG * ur, UlG, UrG);
   }
+  divide_all<NF>(F, ap + am);
 }
 
 // Velocities of a state in the cyclic roles of axis a: (normal, t1, t2) =
@@ -178,22 +206,17 @@ __device__ __forceinline__ MuW<T> to_prim(const T* __restrict__ U, long long n, 
                                           T eta1) {
   MuW<T> w;
   const T d = U[c];
-#if VH_FAST_PROFILE
-  const T inv = fast_rcp(d);
-  const T u = U[n + c] * inv, v = U[2 * n + c] * inv, ww = U[3 * n + c] * inv, tod = U[4 * n + c] * inv;
-#else
-  const T u = U[n + c] / d, v = U[2 * n + c] / d, ww = U[3 * n + c] / d, tod = U[4 * n + c] / d;
-#endif
+  T s[NF - 1];
+#pragma unroll
+  for (int i = 0; i < NF - 1; ++i) s[i] = U[(i + 1) * n + c];
+  divide_all<NF - 1>(s, d);
+  const T u = s[0], v = s[1], ww = s[2], tod = s[3];
   w.r = d;
   w.vx = u;
   w.vy = v;
   w.vz = ww;
   if constexpr (NF == 6) {
-#if VH_FAST_PROFILE
-    const T god = U[5 * n + c] * inv;
-#else
-    const T god = U[5 * n + c] / d;
-#endif
+    const T god = s[4];
     w.e = dual_eint(tod, god, u * u + v * v + ww * ww, g, gm1, eta1, sr);
   } else {
     w.e = jmax(tod - T(0.5) * (u * u + v * v + ww * ww), sr);
@@ -415,13 +438,10 @@ __global__ void __launch_bounds__(TX* TY, sizeof(T) == 4 ? VH_MUSCL_WAVES_F32 : 
       }
       if constexpr (STAGE2 && NF == 6) {
         // dual_energy_sync! (lib/PPMKernels/src/muscl_grid.jl:97-107) on the new state
-#if VH_FAST_PROFILE
-        const T d = o[0], inv = fast_rcp(d), u = o[1] * inv, v = o[2] * inv, w = o[3] * inv;
-        const T tod = o[4] * inv, god = o[5] * inv;
-#else
-        const T d = o[0], u = o[1] / d, v = o[2] / d, w = o[3] / d;
-        const T tod = o[4] / d, god = o[5] / d;
-#endif
+        const T d = o[0];
+        T s[5] = {o[1], o[2], o[3], o[4], o[5]};
+        divide_all<5>(s, d);
+        const T u = s[0], v = s[1], w = s[2], tod = s[3], god = s[4];
         const T v2 = u * u + v * v + w * w;
         const T e = dual_eint(tod, god, v2, g, gm1, e1, sr);
         o[5] = d * e;

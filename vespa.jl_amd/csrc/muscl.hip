@@ -181,9 +181,10 @@ int apply_bc(vh_muscl* m, void* state, int stage) {
 }
 
 // One step: U1 = U + dU(U), then U = ½((U + U1) + dU(U1)) written over U.
-// With bc!, the input is copied to Ub and refilled there (U keeps the unfilled
-// input, the reference's D0), stage 1 writes U1 = U + dU(Ub), and U1 is
-// refilled in place before stage 2. A failing callback leaves U as it was.
+// With a periodic bc! the stages read ghost cells from their images. With a callback
+// the input is copied to Ub and refilled there (U keeps the unfilled input, the
+// reference's D0), stage 1 writes U1 = U + dU(Ub), and U1 is refilled in place
+// before stage 2. A failing callback leaves U as it was.
 int enqueue_step(vh_muscl* m, double dt, bool rec) {
   const double dtdx = m->dtype == VH_F64 ? dt / m->dx : (double)((float)dt / (float)m->dx);
   m->G.dtdx = dtdx;
@@ -243,12 +244,12 @@ int vh_muscl_create(vh_muscl** out, const int32_t* dims, int32_t ng, double gamm
     delete m;
     return fail(-2, "no HIP device%s", "");
   }
-  // 16×16 tiles; planes per workgroup from the grid's size (at most 8; Float64 runs two
+  // 16×16 tiles; planes per workgroup from the grid's size (at most 8; Float64 runs three
   // workgroups per compute unit, Float32 four). Step times at the pick against 8
   // planes (µs): 48×42×36 f64 dual, recording 42 (1) for 185; 72³ f64 fast 71 (4) for 98;
   // 108×100×90 f32 113 (6) for 139; 136³ f64 and 264³ keep 8 ± 5%.
   const long long columns = (long long)((dims[0] + 15) / 16) * ((dims[1] + 15) / 16);
-  m->G.zchunk = march_planes(columns, dims[2], 8, dtype == VH_F64 ? 2 : 4, cu_count(m->device));
+  m->G.zchunk = march_planes(columns, dims[2], 8, dtype == VH_F64 ? 3 : 4, cu_count(m->device));
   set_tiles(m);
   const size_t bytes = (size_t)5 * n * m->esize;
   if (hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess || hipMalloc(&m->U, bytes) != hipSuccess ||
