@@ -393,6 +393,30 @@ def test_bc_periodic_on_device_bitwise(O, dtype, dual):
         g.close()
 
 
+@pytest.mark.parametrize("mode", ["exact", "fast"])
+@pytest.mark.parametrize("dims,ng,dual,dtype", [((21, 12, 40), 4, False, np.float32), ((9, 12, 33), 2, True, np.float64),
+                                                ((10, 40, 9), 3, False, np.float64), ((37, 9, 18), 3, True, np.float32)])
+def test_bc_periodic_images_equal_the_filled_copy(O, V, dims, ng, dual, dtype, mode):
+    """Stages that read ghost cells from their periodic images against the general path,
+    which refills a copy (here by a host hook): states and recorded fluxes of three steps,
+    down to as many active cells as ghosts along an axis."""
+    U = smooth_state(dims, seed=3, dtype=dtype)
+    if dual:
+        U = with_ge(U)
+    gs = [M.MusclGrid(dims, ng, G14, 1.5, 0.05, 1e-10, eltype=dtype, dual=dual) for _ in range(2)]
+    gs[0].set_bc("periodic")
+    gs[1].set_bc(lambda W, stage: _periodic_fill(O, W.reshape(len(U), -1), dims, ng))
+    for g in gs:
+        g.set_mode(mode)
+        g.upload(U)
+        for k in range(3):
+            g.step(0.01, fluxrec=k == 2)
+    np.testing.assert_array_equal(gs[0].state(), gs[1].state())
+    np.testing.assert_array_equal(gs[0].fluxrec(), gs[1].fluxrec())
+    for g in gs:
+        g.close()
+
+
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_bc_host_callback_outflow_bitwise(O, dtype):
     """A host bc! (zero-gradient ghosts) through the C ABI's callback: the library

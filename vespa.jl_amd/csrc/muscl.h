@@ -255,6 +255,14 @@ __device__ __forceinline__ void put_f(T* base, int stride, int i, const T F[NF])
 
 __device__ __forceinline__ int clampi(int v, int n) { return v < 0 ? 0 : (v >= n ? n - 1 : v); }
 
+// Where the stage reads position v of an axis of n cells: clamped to the grid (what no
+// face uses), and a ghost cell from its periodic image `shift` cells away (0: ghosts are
+// read as they are).
+__device__ __forceinline__ int source_pos(int v, int n, int ng, int shift) {
+  v = clampi(v, n);
+  return v < ng ? v + shift : (v >= n - ng ? v - shift : v);
+}
+
 // Waves per SIMD the stage kernel is compiled for (Float64 / Float32 state).
 #ifndef VH_MUSCL_WAVES
 #define VH_MUSCL_WAVES 2
@@ -290,8 +298,9 @@ __global__ void __launch_bounds__(TX* TY, sizeof(T) == 4 ? VH_MUSCL_WAVES_F32 : 
   const long long plane = (long long)nx * ny;
   const int gx = x0 + tx, gy = y0 + ty;
   const bool inside = gx < nx && gy < ny;
-  const long long col = (long long)clampi(gy, ny) * nx + clampi(gx, nx);
-  auto zsrc = [&](int kk) { return col + (long long)clampi(kk, nz) * plane; };
+  const int sx = G.wrap ? nx - 2 * ng : 0, sy = G.wrap ? ny - 2 * ng : 0, sz = G.wrap ? nz - 2 * ng : 0;
+  const long long col = (long long)source_pos(gy, ny, ng, sy) * nx + source_pos(gx, nx, ng, sx);
+  auto zsrc = [&](int kk) { return col + (long long)source_pos(kk, nz, ng, sz) * plane; };
 
   // ---- z pipeline prologue: planes kz0-2 .. kz0+2, the face below kz0 ----
   MuW<T> w0, w1, w2, zhi;   // planes k, k+1, k+2 of the column; hi z state of plane k
@@ -326,6 +335,7 @@ __global__ void __launch_bounds__(TX* TY, sizeof(T) == 4 ? VH_MUSCL_WAVES_F32 : 
 
   for (int k = kz0; k < kz1; ++k) {
     const long long c = (long long)k * plane + (long long)gy * nx + gx;
+    const long long zplane = (long long)source_pos(k, nz, ng, sz) * plane;
     const int rot = (k + (int)blockIdx.x) % (NT / 64);
     const int lt = (tid + 64 * rot) % NT;   // rotating lane index for the side work
 
@@ -334,7 +344,8 @@ __global__ void __launch_bounds__(TX* TY, sizeof(T) == 4 ? VH_MUSCL_WAVES_F32 : 
     for (int h = lt; h < NHX + NHY; h += NT) {
       int lx, ly;
       halo_pos(h, lx, ly);
-      const long long src = (long long)k * plane + (long long)clampi(y0 + ly, ny) * nx + clampi(x0 + lx, nx);
+      const long long src =
+          zplane + (long long)source_pos(y0 + ly, ny, ng, sy) * nx + source_pos(x0 + lx, nx, ng, sx);
       put_w(wf, L_::WS, (ly + 2) * L_::WX + lx + 2, to_prim<T, NF>(Us, n, src, sr, g, gm1, e1));
     }
     __syncthreads();
@@ -432,7 +443,7 @@ __global__ void __launch_bounds__(TX* TY, sizeof(T) == 4 ? VH_MUSCL_WAVES_F32 : 
       }
       T o[NF];
       for (int q = 0; q < NF; ++q) {
-        const T us = Us[q * n + c];
+        const T us = Us[q * n + zplane + col];
         if constexpr (STAGE2) o[q] = T(0.5) * (U0[q * n + c] + us + acc[q]);
         else o[q] = U0[q * n + c] + acc[q];   // U0: the stage's base (Us itself unless bc! refilled a copy)
       }

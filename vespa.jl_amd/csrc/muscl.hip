@@ -193,6 +193,18 @@ int enqueue_step(vh_muscl* m, double dt, bool rec) {
     launch_stage(m, true, rec, m->U1, m->U, m->U);
     return 0;
   }
+  // fill_periodic! as the stages' reading rule: no copy of the input and no fill passes
+  // (264³ f32: 132 + 2·61 µs per step of 1.5 ms). Where an axis has fewer active cells than
+  // ghosts the image of a ghost cell is itself one, and the fill runs as such.
+  bool images = m->bc_kind == VH_MUSCL_BC_PERIODIC;
+  for (int d = 0; d < 3; ++d) images = images && m->G.n[d] - 2 * m->G.ng >= m->G.ng;
+  if (images) {
+    m->G.wrap = 1;
+    launch_stage(m, false, rec, m->U, m->U, m->U1);
+    launch_stage(m, true, rec, m->U1, m->U, m->U);
+    m->G.wrap = 0;
+    return 0;
+  }
   const size_t bytes = (size_t)m->G.nf * m->G.ncell * m->esize;
   if (m->ub_bytes < bytes) {
     VH_HIP(hipStreamSynchronize(m->stream));

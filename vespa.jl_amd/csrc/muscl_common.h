@@ -10,6 +10,7 @@ struct MusclDev {
   int ng;
   int tiles_x, tiles_y, chunks_z, zchunk;
   int xcd_remap, nf;                  // nf: 5 fields, or 6 with the gas energy ρe
+  int wrap;                           // 1: the stage reads its ghost cells from their periodic images
   long long ncell;
   double gamma, theta, small, dtdx;   // dtdx = T(dt)/T(dx), exact in T
   double eta1;                        // dual-energy selection threshold
