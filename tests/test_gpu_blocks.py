@@ -195,6 +195,27 @@ def test_evolve_in_legs_bitwise(O, graph):
     s.close()
 
 
+@pytest.mark.parametrize("nblocks,edges,most", [(3, (8, 16), 1), (12, (8, 16, 24, 32), 2), (40, (6, 16, 24), 6)])
+def test_default_chunks_and_side_streams_bitwise(O, nblocks, edges, most):
+    """The default z planes per tile follow the mesh (short on meshes that do not fill the
+    chip), and the shape classes of a stage (compiled and runtime shapes together) run side
+    by side: eager and captured steps equal the oracle."""
+    m = random_mesh(nblocks, seed=3, rank=3, edges=edges)
+    bo = O.BlockOracle(m)
+    U = _state(m, np.float64, seed=2)
+    s = BM.BlockSimulation(m, np.float64, cfl=0.3)
+    s.upload(U)
+    zc = s.info()["zchunk"]
+    assert 1 <= zc <= most
+    for _ in range(6):
+        bo.step(U, bo.compute_dt(U, 0.3))
+    s.evolve(max_steps=4)                       # captured
+    s.set_launch(zchunk=zc, use_graph=False)
+    s.evolve(max_steps=2)                       # eager
+    np.testing.assert_array_equal(s.state(), U)
+    s.close()
+
+
 def test_launch_shapes_and_methods_agree(O):
     """zchunk, the workgroup cap, graphs and the per-block launch loop all give
     the same bits as the oracle."""

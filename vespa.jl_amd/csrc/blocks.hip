@@ -364,6 +364,35 @@ struct BuildScratch {
 
 // Builds every table of a mesh. Returns 0 or a negative code (message set).
 // nthreads: 0 = the pool's size, 1 = serial; the tables do not depend on it.
+// Tile of a block of n cells, at most max_tx wide; false if no shape fits.
+static bool tile_shape(int rank, const int* n, int max_tx, int* tx, int* ty) {
+  if (rank == 1) {
+    *tx = balanced(n[0], 64);
+    *ty = 1;
+  } else {
+    *tx = balanced(n[0], std::min(kMaxE, std::max(4, max_tx)));
+    *ty = balanced(n[1], std::min(kLanes / *tx, kMaxE));
+  }
+  return !(*tx * *ty > kLanes || (*tx + 4) * (*ty + 4) > kMaxW ||
+           *ty * (*tx + 2) + (rank > 1 ? (*ty + 2) * *tx : 0) > kMaxFS || (rank > 1 && *tx > kMaxE) || *ty > kMaxE);
+}
+
+// z planes per tile that leave about 1500 tiles (two rounds of three workgroups per
+// compute unit), at most 6. Step times at the pick against 8 planes (µs, f64 fast): 20 blocks 109
+// (1 plane) for 204, 60 blocks 178 (2) for 253, 150 blocks 261 (5) for 327, 400 blocks 597 (6) for
+// 628, 1000 blocks 1574 (6) for 1592.
+static int default_zchunk(const Topo& T, int max_tx) {
+  if (T.rank < 3) return 8;   // not used
+  long long planes = 0;
+  for (int b = 0; b < T.nb; ++b) {
+    const int* n = &T.dims[3 * b];
+    int tx, ty;
+    if (!tile_shape(T.rank, n, max_tx, &tx, &ty)) return 6;   // refused by the table builder
+    planes += (long long)((n[0] + tx - 1) / tx) * ((n[1] + ty - 1) / ty) * n[2];
+  }
+  return (int)std::min(6LL, std::max(1LL, (planes + 750) / 1500));
+}
+
 static int build_tables(Topo& T, int zchunk, HostTables& H, int max_tx = 32, int nthreads = 0) {
   const int nb = T.nb, rank = T.rank;
   // ---- candidate neighbours by face plane ----
@@ -843,17 +872,7 @@ static int build_tables(Topo& T, int zchunk, HostTables& H, int max_tx = 32, int
     const BlockDev& bk = H.blocks[b];
     H.block_tile_start[b] = (int)base.size();
     int tx, ty;
-    if (rank == 1) {
-      tx = balanced(bk.n[0], 64);
-      ty = 1;
-    } else {
-      tx = balanced(bk.n[0], std::min(kMaxE, std::max(4, max_tx)));
-      int maxty = kLanes / tx;
-      if (maxty > kMaxE) maxty = kMaxE;
-      ty = balanced(bk.n[1], maxty);
-    }
-    if (tx * ty > kLanes || (tx + 4) * (ty + 4) > kMaxW || ty * (tx + 2) + (rank > 1 ? (ty + 2) * tx : 0) > kMaxFS ||
-        (rank > 1 && tx > kMaxE) || ty > kMaxE)
+    if (!tile_shape(rank, bk.n, max_tx, &tx, &ty))
       return fail(-1, "no tile shape fits block %s%lld", "", b);
     int zc = rank == 3 ? (zchunk > 0 ? zchunk : bk.n[2]) : 1;
     if (zc > bk.n[2]) zc = bk.n[2];
@@ -1094,6 +1113,7 @@ struct vh_blocks {
   int dtype = VH_F64, mode = VH_EXACT, device = 0;
   size_t esize = 8;
   int zchunk = 8;
+  bool zchunk_auto = true;   // zchunk follows the mesh until vh_blocks_set_launch sets it
   int max_tx = 32;        // widest tile along x
   int max_wgs = 0;        // persistent workgroups (0: 3 per CU)
   int ncu = 256;
@@ -1821,6 +1841,7 @@ int vh_blocks_create(vh_blocks** out, int32_t rank, int32_t nblocks, int32_t max
   if (!(gamma > 1.0)) return fail(-1, "gamma must exceed 1%s", "");
   vh_blocks* m = new vh_blocks();
   int rc = make_topo(m->T, rank, nblocks, maxlevel, h0, level, dims, origin, bc);
+  if (!rc) m->zchunk = default_zchunk(m->T, m->max_tx);
   if (!rc) rc = build_tables(m->T, m->zchunk, m->H, m->max_tx);
   if (rc) { delete m; return rc; }
   m->dtype = dtype;
@@ -2134,6 +2155,7 @@ int vh_blocks_set_launch(vh_blocks* m, int32_t zchunk, int32_t max_workgroups, i
   drop_graph(m);
   m->use_graph = use_graph ? 1 : 0;
   m->max_wgs = max_workgroups;
+  m->zchunk_auto = false;
   if (zchunk != m->zchunk) {
     HostTables& H = m->H2;
     int rc = build_tables(m->T, zchunk, H, m->max_tx);
@@ -2268,7 +2290,8 @@ int vh_blocks_regrid(vh_blocks* m, int32_t nblocks, const int32_t* level, const 
   HostTables& H = m->H2;
   const double h0[3] = {m->T.h0[0], m->T.h0[1], m->T.h0[2]};
   int rc = make_topo(N, m->T.rank, nblocks, m->T.maxlevel, h0, level, dims, origin, bc);
-  if (!rc) rc = build_tables(N, m->zchunk, H, m->max_tx);
+  const int zchunk = !rc && m->zchunk_auto ? default_zchunk(N, m->max_tx) : m->zchunk;
+  if (!rc) rc = build_tables(N, zchunk, H, m->max_tx);
   std::vector<RemapDev> map;
   if (!rc) rc = build_remap(N, m->T, src_block, map);
   if (rc) return rc;
@@ -2334,6 +2357,7 @@ int vh_blocks_regrid(vh_blocks* m, int32_t nblocks, const int32_t* level, const 
   }
   std::swap(m->T, N);
   std::swap(m->H, H);
+  m->zchunk = zchunk;
   rc = alloc_partials(m);
   if (rc) return rc;
   if (grav) {
