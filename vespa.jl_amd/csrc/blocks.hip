@@ -38,6 +38,7 @@
 
 #include "../../include/vespahip.h"
 #include "host.h"
+#include "hostpool.h"
 #include "profiles.h"
 
 namespace vh {
@@ -206,101 +207,6 @@ static int balanced(int n, int maxT) {
   const int nt = (n + maxT - 1) / maxT;
   return (n + nt - 1) / nt;
 }
-
-// ----------------------------------------------------------------------------
-// host thread pool for the table builder: run(n, f) calls f(i) for i in [0, n)
-// on the pool's workers and the caller, returning when all are done. Created on
-// first use with min(hardware threads, 16) threads (VESPAHIP_HOST_THREADS
-// overrides, 1 = serial); a child process after fork() builds its own (it
-// inherits no worker threads). The pool is never destroyed: its workers sleep
-// until the process ends.
-class HostPool {
- public:
-  static int threads() {
-    static const int n = [] {
-      const char* e = getenv("VESPAHIP_HOST_THREADS");
-      int v = e ? atoi(e) : (int)std::thread::hardware_concurrency();
-      return std::max(1, std::min(v, e ? 256 : 16));
-    }();
-    return n;
-  }
-  static void run(int n, const std::function<void(int)>& f) {
-    if (n <= 1 || threads() <= 1) {
-      for (int i = 0; i < n; ++i) f(i);
-      return;
-    }
-    static std::mutex create_mu;
-    static HostPool* pool = nullptr;
-    HostPool* p;
-    {
-      std::lock_guard<std::mutex> lk(create_mu);
-      if (!pool || pool->pid_ != getpid()) pool = new HostPool(threads() - 1);   // the old one stays (forked child)
-      p = pool;
-    }
-    p->go(n, f);
-  }
-
- private:
-  // A build issues a few jobs back to back: threads spin this many pauses
-  // (tens of microseconds) for the next job or the end of the current one
-  // before they sleep, which saves a wake-up per job.
-  static constexpr int kSpin = 1 << 14;
-  static void pause() { __builtin_ia32_pause(); }
-
-  explicit HostPool(int workers) : pid_(getpid()) {
-    for (int i = 0; i < workers; ++i) std::thread([this] { loop(); }).detach();
-    nworkers_ = workers;
-  }
-  void loop() {
-    long long seen = 0;
-    for (;;) {
-      long long g = gen_.load(std::memory_order_acquire);
-      for (int i = 0; g == seen && i < kSpin; ++i) {
-        pause();
-        g = gen_.load(std::memory_order_acquire);
-      }
-      if (g == seen) {
-        std::unique_lock<std::mutex> lk(mu_);
-        cv_.wait(lk, [&] { return gen_.load(std::memory_order_acquire) != seen; });
-        g = gen_.load(std::memory_order_acquire);
-      }
-      seen = g;
-      const std::function<void(int)>* f = job_;
-      const int n = njob_;
-      for (int i; (i = next_.fetch_add(1)) < n;) (*f)(i);
-      if (active_.fetch_sub(1, std::memory_order_acq_rel) == 1) {
-        std::lock_guard<std::mutex> lk(mu_);
-        done_.notify_one();
-      }
-    }
-  }
-  void go(int n, const std::function<void(int)>& f) {
-    std::lock_guard<std::mutex> run_lk(run_mu_);   // one job at a time
-    job_ = &f;
-    njob_ = n;
-    next_.store(0);
-    active_.store(nworkers_);
-    {
-      std::lock_guard<std::mutex> lk(mu_);
-      gen_.fetch_add(1, std::memory_order_release);   // publishes the job to spinning and sleeping workers
-    }
-    cv_.notify_all();
-    for (int i; (i = next_.fetch_add(1)) < n;) f(i);
-    for (int i = 0; active_.load(std::memory_order_acquire) != 0 && i < kSpin; ++i) pause();
-    if (active_.load(std::memory_order_acquire) != 0) {
-      std::unique_lock<std::mutex> lk(mu_);
-      done_.wait(lk, [&] { return active_.load(std::memory_order_acquire) == 0; });
-    }
-  }
-  pid_t pid_;
-  int nworkers_ = 0;
-  std::mutex run_mu_, mu_;
-  std::condition_variable cv_, done_;
-  const std::function<void(int)>* job_ = nullptr;
-  int njob_ = 0;
-  std::atomic<long long> gen_{0};
-  std::atomic<int> next_{0}, active_{0};
-};
 
 // Output of one chunk (a contiguous run of blocks) of the parallel table
 // phases; indices inside are chunk-local until the chunks are joined in order,
@@ -1911,16 +1817,14 @@ int vh_blocks_set_mode(vh_blocks* m, int32_t mode) {
 int vh_blocks_upload(vh_blocks* m, const void* U) {
   if (!m || !U) return fail(-1, "null argument%s", "");
   VH_HIP(hipSetDevice(m->device));
-  VH_HIP(hipMemcpyAsync(m->U, U, (size_t)5 * m->T.off[m->T.nb] * m->esize, hipMemcpyHostToDevice, m->stream));
-  VH_HIP(hipStreamSynchronize(m->stream));
+  VH_HIP(copy_up(m->U, U, (size_t)5 * m->T.off[m->T.nb] * m->esize, m->stream));
   return 0;
 }
 
 int vh_blocks_download(vh_blocks* m, void* U) {
   if (!m || !U) return fail(-1, "null argument%s", "");
   VH_HIP(hipSetDevice(m->device));
-  VH_HIP(hipMemcpyAsync(U, m->U, (size_t)5 * m->T.off[m->T.nb] * m->esize, hipMemcpyDeviceToHost, m->stream));
-  VH_HIP(hipStreamSynchronize(m->stream));
+  VH_HIP(copy_down(U, m->U, (size_t)5 * m->T.off[m->T.nb] * m->esize, m->stream));
   return 0;
 }
 
@@ -2095,16 +1999,14 @@ int vh_blocks_solve_poisson(vh_blocks* m, int64_t* iters, double* relres) {
 int vh_blocks_phi_upload(vh_blocks* m, const void* host) {
   if (int rc = need_grav(m)) return rc;
   if (!host) return fail(-1, "null argument%s", "");
-  VH_HIP(hipMemcpyAsync(m->grav->B.phi, host, m->esize * m->T.off[m->T.nb], hipMemcpyHostToDevice, m->stream));
-  VH_HIP(hipStreamSynchronize(m->stream));
+  VH_HIP(copy_up(m->grav->B.phi, host, m->esize * m->T.off[m->T.nb], m->stream));
   return 0;
 }
 
 int vh_blocks_phi_download(vh_blocks* m, void* host) {
   if (int rc = need_grav(m)) return rc;
   if (!host) return fail(-1, "null argument%s", "");
-  VH_HIP(hipMemcpyAsync(host, m->grav->B.phi, m->esize * m->T.off[m->T.nb], hipMemcpyDeviceToHost, m->stream));
-  VH_HIP(hipStreamSynchronize(m->stream));
+  VH_HIP(copy_down(host, m->grav->B.phi, m->esize * m->T.off[m->T.nb], m->stream));
   return 0;
 }
 
@@ -2139,8 +2041,7 @@ int vh_blocks_totals(vh_blocks* m, double* out5) {
                        m->d_cfl_blocks, m->d_cfl_prefix, nb, m->partials);
   VH_HIP(hipGetLastError());
   std::vector<double> h(5 * kCflWgs);
-  VH_HIP(hipMemcpyAsync(h.data(), m->partials, sizeof(double) * h.size(), hipMemcpyDeviceToHost, m->stream));
-  VH_HIP(hipStreamSynchronize(m->stream));
+  VH_HIP(copy_down(h.data(), m->partials, sizeof(double) * h.size(), m->stream));
   for (int f = 0; f < 5; ++f) out5[f] = 0.0;
   for (int b = 0; b < kCflWgs; ++b)
     for (int f = 0; f < 5; ++f) out5[f] += h[5 * b + f];

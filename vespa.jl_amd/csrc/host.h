@@ -59,6 +59,11 @@ inline int cu_count(int device) {
   return hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && n > 0 ? n : 256;
 }
 
+// Copy between the device (the current one) and a host array, ordered after the work on s and
+// complete on return (transfer.hip).
+hipError_t copy_up(void* dev, const void* host, size_t bytes, hipStream_t s);
+hipError_t copy_down(void* host, const void* dev, size_t bytes, hipStream_t s);
+
 // Clock kernels of the uniform-grid context, shared with the block context.
 // clock (kClockDoubles): [0] t, [1] dt, [2] max CFL term, [3] steps; of a step loop also
 // [4] cfl, [5] tfinal (infinite: no clip), [6] the time at which the loop ends, [7] non-zero

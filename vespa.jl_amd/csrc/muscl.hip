@@ -295,16 +295,14 @@ int64_t vh_muscl_ncell(const vh_muscl* m) { return m ? m->G.ncell : -1; }
 int vh_muscl_upload(vh_muscl* m, const void* U) {
   if (!m || !U) return fail(-1, "null argument%s", "");
   VH_HIP(hipSetDevice(m->device));
-  VH_HIP(hipMemcpyAsync(m->U, U, (size_t)m->G.nf * m->G.ncell * m->esize, hipMemcpyHostToDevice, m->stream));
-  VH_HIP(hipStreamSynchronize(m->stream));
+  VH_HIP(copy_up(m->U, U, (size_t)m->G.nf * m->G.ncell * m->esize, m->stream));
   return 0;
 }
 
 int vh_muscl_download(vh_muscl* m, void* U) {
   if (!m || !U) return fail(-1, "null argument%s", "");
   VH_HIP(hipSetDevice(m->device));
-  VH_HIP(hipMemcpyAsync(U, m->U, (size_t)m->G.nf * m->G.ncell * m->esize, hipMemcpyDeviceToHost, m->stream));
-  VH_HIP(hipStreamSynchronize(m->stream));
+  VH_HIP(copy_down(U, m->U, (size_t)m->G.nf * m->G.ncell * m->esize, m->stream));
   return 0;
 }
 
@@ -392,9 +390,7 @@ int vh_muscl_set_bc(vh_muscl* m, int32_t kind, vh_muscl_bc_fn fn, void* user) {
 int vh_muscl_fluxrec_download(vh_muscl* m, void* frec) {
   if (!m || !frec) return fail(-1, "null argument%s", "");
   if (!m->frec) return fail(-1, "no step has recorded fluxes yet%s", "");
-  VH_HIP(hipMemcpyAsync(frec, m->frec, (size_t)3 * m->G.nf * m->G.ncell * m->esize, hipMemcpyDeviceToHost,
-                        m->stream));
-  VH_HIP(hipStreamSynchronize(m->stream));
+  VH_HIP(copy_down(frec, m->frec, (size_t)3 * m->G.nf * m->G.ncell * m->esize, m->stream));
   return 0;
 }
 
@@ -414,8 +410,7 @@ int vh_muscl_max_wavespeed(vh_muscl* m, double* out) {
   else wavespeed_kernel<float><<<nb, 256, 0, m->stream>>>((const float*)m->U, m->G, m->partials);
   VH_HIP(hipGetLastError());
   std::vector<double> p(nb);
-  VH_HIP(hipMemcpyAsync(p.data(), m->partials, sizeof(double) * nb, hipMemcpyDeviceToHost, m->stream));
-  VH_HIP(hipStreamSynchronize(m->stream));
+  VH_HIP(copy_down(p.data(), m->partials, sizeof(double) * nb, m->stream));
   double r = p[0];
   for (int i = 1; i < nb; ++i) r = std::isnan(r) ? r : (std::isnan(p[i]) || p[i] > r ? p[i] : r);
   *out = r;
@@ -453,10 +448,8 @@ int vh_muscl_flux_register(vh_muscl* m, double dt, double* planes, double* inter
     op += 10 * t;
     oi += 5 * (act[a] - 1) * t;
   }
-  if (e == hipSuccess) e = hipMemcpyAsync(planes, d, sizeof(double) * np, hipMemcpyDeviceToHost, m->stream);
-  if (e == hipSuccess && interior)
-    e = hipMemcpyAsync(interior, d + np, sizeof(double) * ni, hipMemcpyDeviceToHost, m->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
+  if (e == hipSuccess) e = copy_down(planes, d, sizeof(double) * np, m->stream);
+  if (e == hipSuccess && interior) e = copy_down(interior, d + np, sizeof(double) * ni, m->stream);
   (void)hipFree(d);
   if (e != hipSuccess) return fail(-2, "HIP error %s in the flux register gather%s", hipGetErrorString(e));
   return 0;

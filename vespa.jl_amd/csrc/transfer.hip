@@ -1,0 +1,166 @@
+// Copies between pageable host arrays and the device.
+//
+// The runtime moves pageable memory through its own staging with one thread; a fresh host
+// array also takes its page faults in that thread. Here the copy is cut into chunks that
+// pass through pinned slots, the DMA of one chunk running while the pool's threads copy
+// others between the slots and the caller's array.
+//
+// Bound: the link (57 GB/s each way from pinned memory) and the threads' page faults. Measured,
+// runtime and here (GB/s): down 2 MiB 17.7 and 26.6, 16 MiB 16.9 and 34, 195 MiB 17.5 and 39.4; down
+// into a fresh array of 195 MiB 10.4 and 17.7; up 2 MiB 25.9 and 31.6, 64 MiB 29.5 and 38.5. At 512 KiB
+// both take 27-34 µs, so smaller copies go to the runtime.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <condition_variable>
+#include <cstring>
+#include <mutex>
+#include <vector>
+
+#include "host.h"
+#include "hostpool.h"
+
+namespace vh {
+namespace {
+
+constexpr size_t kChunk = (size_t)2 << 20;   // bytes per slot
+constexpr size_t kPiece = (size_t)128 << 10; // bytes per thread at a time
+constexpr int kSlots = 16;                   // pinned slots of the process (32 MiB)
+constexpr int kSlotsPerCopy = 4;
+// Copies of at most this many bytes go to the runtime.
+constexpr size_t kDirect = (size_t)512 << 10;
+
+// A slot's event belongs to the device it was made on.
+struct Slot {
+  char* mem = nullptr;
+  hipEvent_t ev = nullptr;
+  int device = -1;
+};
+
+// Slots are taken by a copy and given back at its end; a copy that finds none waits for one.
+class SlotPool {
+ public:
+  std::vector<Slot> take(int want, int device) {
+    std::vector<Slot> got;
+    std::unique_lock<std::mutex> lk(mu_);
+    for (;;) {
+      while ((int)got.size() < want && !free_.empty()) {
+        got.push_back(free_.back());
+        free_.pop_back();
+      }
+      while ((int)got.size() < want && made_ < kSlots) {
+        void* p = nullptr;
+        if (hipHostMalloc(&p, kChunk, hipHostMallocPortable) != hipSuccess) {
+          (void)hipGetLastError();
+          break;
+        }
+        ++made_;
+        got.push_back(Slot{(char*)p, nullptr, -1});
+      }
+      if (!got.empty() || made_ == 0) break;
+      cv_.wait(lk);
+    }
+    lk.unlock();
+    for (size_t i = 0; i < got.size(); ++i) {
+      Slot& s = got[i];
+      if (s.device == device) continue;
+      if (s.ev) (void)hipEventDestroy(s.ev);
+      s.ev = nullptr;
+      s.device = -1;
+      if (hipEventCreateWithFlags(&s.ev, hipEventDisableTiming) == hipSuccess) s.device = device;
+    }
+    return got;
+  }
+  void give_back(const std::vector<Slot>& slots) {
+    std::lock_guard<std::mutex> lk(mu_);
+    for (const Slot& s : slots) free_.push_back(s);
+    cv_.notify_all();
+  }
+
+ private:
+  std::mutex mu_;
+  std::condition_variable cv_;
+  std::vector<Slot> free_;
+  int made_ = 0;
+};
+SlotPool& slot_pool() {
+  static SlotPool* p = new SlotPool();   // never destroyed: copies may run while the process ends
+  return *p;
+}
+
+void copy_pieces(char* dst, const char* src, size_t n) {
+  HostPool::run((int)((n + kPiece - 1) / kPiece), [&](int i) {
+    const size_t o = (size_t)i * kPiece;
+    memcpy(dst + o, src + o, std::min(kPiece, n - o));
+  });
+}
+
+bool is_pinned(const void* p) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type == hipMemoryTypeHost;
+}
+
+hipError_t staged(char* dst, const char* src, size_t bytes, bool up, hipStream_t s, const std::vector<Slot>& slots) {
+  const size_t n = (bytes + kChunk - 1) / kChunk, ns = slots.size();
+  auto len = [&](size_t c) { return std::min(kChunk, bytes - c * kChunk); };
+  hipError_t e = hipSuccess;
+  if (up) {
+    for (size_t c = 0; c < n && e == hipSuccess; ++c) {
+      const Slot& sl = slots[c % ns];
+      if (c >= ns) e = hipEventSynchronize(sl.ev);
+      if (e != hipSuccess) break;
+      copy_pieces(sl.mem, src + c * kChunk, len(c));
+      e = hipMemcpyAsync(dst + c * kChunk, sl.mem, len(c), hipMemcpyHostToDevice, s);
+      if (e == hipSuccess) e = hipEventRecord(sl.ev, s);
+    }
+  } else {
+    auto issue = [&](size_t c) {
+      const Slot& sl = slots[c % ns];
+      hipError_t r = hipMemcpyAsync(sl.mem, src + c * kChunk, len(c), hipMemcpyDeviceToHost, s);
+      return r == hipSuccess ? hipEventRecord(sl.ev, s) : r;
+    };
+    for (size_t c = 0; c < std::min(n, ns) && e == hipSuccess; ++c) e = issue(c);
+    for (size_t c = 0; c < n && e == hipSuccess; ++c) {
+      e = hipEventSynchronize(slots[c % ns].ev);
+      if (e != hipSuccess) break;
+      copy_pieces(dst + c * kChunk, slots[c % ns].mem, len(c));
+      if (c + ns < n) e = issue(c + ns);
+    }
+  }
+  const hipError_t es = hipStreamSynchronize(s);   // the slots are free again, whatever happened
+  return e == hipSuccess ? es : e;
+}
+
+hipError_t host_copy(void* dst, const void* src, size_t bytes, bool up, hipStream_t s) {
+  if (bytes == 0) return hipStreamSynchronize(s);
+  int device = 0, stream_device = 0;
+  hipError_t e = hipGetDevice(&device);
+  if (e != hipSuccess) return e;
+  // the slots' events are the current device's: a stream of another takes the plain copy
+  if (!s || hipStreamGetDevice(s, &stream_device) != hipSuccess) stream_device = device;
+  if (bytes > kDirect && HostPool::threads() > 1 && stream_device == device && !is_pinned(up ? src : dst)) {
+    const size_t chunks = (bytes + kChunk - 1) / kChunk;
+    std::vector<Slot> slots = slot_pool().take((int)std::min<size_t>(kSlotsPerCopy, chunks), device);
+    bool usable = !slots.empty();
+    for (const Slot& sl : slots) usable = usable && sl.device == device;
+    if (usable) e = staged((char*)dst, (const char*)src, bytes, up, s, slots);
+    slot_pool().give_back(slots);
+    if (usable) return e;
+  }
+  e = hipMemcpyAsync(dst, src, bytes, up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, s);
+  const hipError_t es = hipStreamSynchronize(s);
+  return e == hipSuccess ? es : e;
+}
+
+}  // namespace
+
+hipError_t copy_up(void* dev, const void* host, size_t bytes, hipStream_t s) { return host_copy(dev, host, bytes, true, s); }
+hipError_t copy_down(void* host, const void* dev, size_t bytes, hipStream_t s) {
+  return host_copy(host, dev, bytes, false, s);
+}
+
+}  // namespace vh

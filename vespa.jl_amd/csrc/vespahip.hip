@@ -413,13 +413,12 @@ static int face_flux_host(const T* WL, const T* WR, const int32_t* ax, int64_t n
   T* dF = (T*)(base + 2 * nv_al);
   int32_t* dax = (int32_t*)(base + 3 * nv_al);
   hipStream_t s = g_stage.stream;
-  VH_HIP(hipMemcpyAsync(dWL, WL, nv, hipMemcpyHostToDevice, s));
-  VH_HIP(hipMemcpyAsync(dWR, WR, nv, hipMemcpyHostToDevice, s));
-  VH_HIP(hipMemcpyAsync(dax, ax, (size_t)nf * sizeof(int32_t), hipMemcpyHostToDevice, s));
+  VH_HIP(copy_up(dWL, WL, nv, s));
+  VH_HIP(copy_up(dWR, WR, nv, s));
+  VH_HIP(copy_up(dax, ax, (size_t)nf * sizeof(int32_t), s));
   exact::launch_face_flux(sizeof(T) == 8 ? 0 : 1, nf, s, dWL, dWR, dax, gamma, dF);
   VH_HIP(hipGetLastError());
-  VH_HIP(hipMemcpyAsync(F, dF, nv, hipMemcpyDeviceToHost, s));
-  VH_HIP(hipStreamSynchronize(s));
+  VH_HIP(copy_down(F, dF, nv, s));
   return 0;
 }
 
@@ -514,12 +513,12 @@ int vh_buffer_free(void* dptr) {
 }
 int vh_buffer_upload(void* dptr, const void* host, int64_t bytes) {
   if (bytes < 0 || (bytes > 0 && (!dptr || !host))) return fail(-1, "bad argument%s", "");
-  if (bytes) VH_HIP(hipMemcpy(dptr, host, (size_t)bytes, hipMemcpyHostToDevice));
+  if (bytes) VH_HIP(copy_up(dptr, host, (size_t)bytes, nullptr));
   return 0;
 }
 int vh_buffer_download(void* host, const void* dptr, int64_t bytes) {
   if (bytes < 0 || (bytes > 0 && (!dptr || !host))) return fail(-1, "bad argument%s", "");
-  if (bytes) VH_HIP(hipMemcpy(host, dptr, (size_t)bytes, hipMemcpyDeviceToHost));
+  if (bytes) VH_HIP(copy_down(host, dptr, (size_t)bytes, nullptr));
   return 0;
 }
 int vh_buffer_copy(void* ddst, const void* dsrc, int64_t bytes) {
@@ -666,16 +665,14 @@ int vh_grid_get_mode(const vh_grid* g) { return g ? g->mode : -1; }
 int vh_grid_upload(vh_grid* g, const void* U) {
   if (!g || !U) return fail(-1, "null argument%s", "");
   VH_HIP(hipSetDevice(g->device));
-  VH_HIP(hipMemcpyAsync(g->U, U, (size_t)5 * g->G.ncell * g->esize, hipMemcpyHostToDevice, g->stream));
-  VH_HIP(hipStreamSynchronize(g->stream));
+  VH_HIP(copy_up(g->U, U, (size_t)5 * g->G.ncell * g->esize, g->stream));
   return 0;
 }
 
 int vh_grid_download(vh_grid* g, void* U) {
   if (!g || !U) return fail(-1, "null argument%s", "");
   VH_HIP(hipSetDevice(g->device));
-  VH_HIP(hipMemcpyAsync(U, g->U, (size_t)5 * g->G.ncell * g->esize, hipMemcpyDeviceToHost, g->stream));
-  VH_HIP(hipStreamSynchronize(g->stream));
+  VH_HIP(copy_down(U, g->U, (size_t)5 * g->G.ncell * g->esize, g->stream));
   return 0;
 }
 
@@ -861,8 +858,7 @@ int vh_grid_phi_upload(vh_grid* g, const void* host) {
   if (!g || !host) return fail(-1, "null argument%s", "");
   if (!g->grav) return fail(-1, "self-gravity is not enabled%s", "");
   VH_HIP(hipSetDevice(g->device));
-  VH_HIP(hipMemcpyAsync(g->grav->B.phi, host, g->esize * g->G.ncell, hipMemcpyHostToDevice, g->stream));
-  VH_HIP(hipStreamSynchronize(g->stream));
+  VH_HIP(copy_up(g->grav->B.phi, host, g->esize * g->G.ncell, g->stream));
   return 0;
 }
 
@@ -870,8 +866,7 @@ int vh_grid_phi_download(vh_grid* g, void* host) {
   if (!g || !host) return fail(-1, "null argument%s", "");
   if (!g->grav) return fail(-1, "self-gravity is not enabled%s", "");
   VH_HIP(hipSetDevice(g->device));
-  VH_HIP(hipMemcpyAsync(host, g->grav->B.phi, g->esize * g->G.ncell, hipMemcpyDeviceToHost, g->stream));
-  VH_HIP(hipStreamSynchronize(g->stream));
+  VH_HIP(copy_down(host, g->grav->B.phi, g->esize * g->G.ncell, g->stream));
   return 0;
 }
 
@@ -934,8 +929,7 @@ int vh_grid_accumulate_flux(vh_grid* g, void* acc_host) {
     hipLaunchKernelGGL(sub_kernel<float>, dim3(blocks), dim3(256), 0, g->stream, (const float*)g->U1,
                        (const float*)g->U, (float*)g->U1, n5);
   VH_HIP(hipGetLastError());
-  VH_HIP(hipMemcpyAsync(acc_host, g->U1, (size_t)n5 * g->esize, hipMemcpyDeviceToHost, g->stream));
-  VH_HIP(hipStreamSynchronize(g->stream));
+  VH_HIP(copy_down(acc_host, g->U1, (size_t)n5 * g->esize, g->stream));
   return 0;
 }
 
