@@ -252,8 +252,8 @@ int vh_grid_time_steps(vh_grid* g, double cfl, int64_t nsteps, double* ms_stage1
 int vh_grid_step_vjp(vh_grid* g, const void* dU, double dt, const void* dWbar, void* dUbar);
 
 /* Kernel form of A'(U)ᵀλ inside the reverse mode: fused = 1 (default) uses one
- * tiled kernel per evaluation on 2D grids periodic on both axes with sizes that
- * are multiples of 32×8, fused = 0 always uses the three-pass form (any rank and
+ * tiled kernel per evaluation on 2D grids periodic on both axes with 10 to 16
+ * or more than 17 cells along each, fused = 0 always uses the three-pass form (any rank and
  * boundary). Both give the same values to round-off. */
 int vh_grid_set_adjoint_form(vh_grid* g, int32_t fused);
 

@@ -163,3 +163,20 @@ def test_fused_tile_form_matches_three_pass_form_and_oracle(O, dims):
     assert _rel(fused, ref) < 1e-12
     assert _rel(three, ref) < 1e-12
     sim.close()
+
+
+@pytest.mark.parametrize("dims", [(10, 10), (16, 48), (18, 33), (15, 64), (50, 37), (17, 40), (40, 9), (129, 19)])
+def test_fused_tiles_of_any_size(O, dims):
+    """Sizes that leave the last tiles partly filled, the smallest that wrap once, and
+    two (17 and 9 cells) that stay with the three-pass form; the bound is that of the
+    whole tiles (the forms differ in summation order only)."""
+    print(f"fused jat {dims}", flush=True)
+    shape = (5,) + tuple(reversed(dims))
+    U = random_state(shape[1:], seed=21, vmax=0.4)
+    g = O.make_grid(dims, [(0.0, 1.0)] * 2, "periodic", 1.4)
+    dt = 0.5 * O.compute_dt(g, U, 0.4)
+    w = np.random.default_rng(22).normal(size=shape)
+    ref = O.step_vjp(g, U, dt, w)
+    sim = _sim(dims, "periodic", U)
+    assert _rel(AD.step_vjp(sim, U, dt, w), ref) < 1e-12
+    sim.close()

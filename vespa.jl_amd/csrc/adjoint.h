@@ -516,78 +516,49 @@ __global__ void __launch_bounds__(256) adj_cell_kernel(const double* __restrict_
 }
 
 // ---------------------------------------------------------------------------
-// Fused A'(U)ᵀλ for 2D grids periodic on both axes: one workgroup per 32×8 tile
+// Fused A'(U)ᵀλ for 2D grids periodic on both axes: one workgroup per 16×16 tile
 // computes W for the tile and a cross-shaped halo of three cells, every face
 // adjoint its cells need (the tile's faces plus one more on each side), and the
 // gather, in LDS; one launch instead of four, no face buffers in HBM.
-constexpr int JTX = 32, JTY = 16, JNT = 512;
+// Bound: the phases wait for each other (loads, faces, gather, stores), so what
+// counts is that a second workgroup fills a compute unit meanwhile. 81,440 B of LDS
+// and 128 registers let two of 512 lanes share it; 608 faces over 512 lanes leave the
+// second pass to two waves. Per launch at 512²: one 32×16 tile per compute unit 29.0 µs
+// (at 512, 640, 768 and 1024 lanes alike, 26.5 with the cell's state kept in registers),
+// 16×16 with 320 lanes 33.0, with 512 25.8, with the XCD ranges below 23.1. At 256² 13.9 →
+// 9.9 µs, at 2048² 443 → 353 µs; sizes that the 32×16 tile did not divide went through
+// the passes: 500×400 60 → 23 µs, 10² 15 → 7.7 µs.
+constexpr int JTX = 16, JTY = 16, JNT = 512;
 constexpr int JNXF = JTY * (JTX + 3);   // x faces of a tile (one extra on the lo side, two on the hi)
 constexpr int JNYF = (JTY + 3) * JTX;   // y faces of a tile
 
-// One 32×16 tile per workgroup of 512 lanes (one workgroup per compute unit:
-// 256 VGPRs per lane, 150 KiB of LDS).
 struct JatLDS {
-  double Wx[5][JTY][JTX + 6];   // W, rows y0..y0+15, cols x0-3..x0+34
-  double Wy[5][6][JTX];         // W, rows y0-3..y0-1 and y0+16..y0+18, cols x0..x0+31
-  double Lx[5][JTY][JTX + 4];   // λ, rows y0..y0+15, cols x0-2..x0+33
-  double Ly[5][4][JTX];         // λ, rows y0-2, y0-1, y0+16, y0+17
-  double Gx[10][JNXF];          // x-face state adjoints (left 0..4, right 5..9)
-  double Gy[10][JNYF];          // y-face state adjoints
+  double W[5][JTY + 6][JTX + 6];   // rows y0-3..y0+JTY+2, cols x0-3..x0+JTX+2 (the corners stay unused)
+  double L[5][JTY + 4][JTX + 4];   // λ, rows y0-2..y0+JTY+1, cols x0-2..x0+JTX+1
+  double Gx[2][5][JTY][JTX + 2];   // x-face state adjoints: [0] left state of faces 1.., [1] right state of faces 0..
+  double Gy[2][5][JTY + 2][JTX];   // y-face state adjoints, the same
 };
 
-// Flat LDS offsets of the cross-shaped W and λ halos: (row, col) in tile
-// coordinates, row ∈ [−3, JTY+2] with col ∈ [0, JTX) or row ∈ [0, JTY) with
-// col ∈ [−3, JTX+2]; returns the address of field 0 and the field pitch.
-__device__ __forceinline__ const double* jat_w_at(const JatLDS& S, int row, int col, int& pitch) {
-  if (row >= 0 && row < JTY) {
-    pitch = JTY * (JTX + 6);
-    return &S.Wx[0][row][col + 3];
-  }
-  pitch = 6 * JTX;
-  return &S.Wy[0][row < 0 ? row + 3 : 3 + row - JTY][col];
-}
-__device__ __forceinline__ const double* jat_l_at(const JatLDS& S, int row, int col, int& pitch) {
-  if (row >= 0 && row < JTY) {
-    pitch = JTY * (JTX + 4);
-    return &S.Lx[0][row][col + 2];
-  }
-  pitch = 4 * JTX;
-  return &S.Ly[0][row < 0 ? row + 2 : 2 + row - JTY][col];
-}
+// W and λ of one cell, (row, col) in tile coordinates.
 __device__ __forceinline__ D5 jat_w(const JatLDS& S, int row, int col) {
-  int p;
-  const double* a = jat_w_at(S, row, col, p);
   D5 w;
-  w.r = a[0]; w.vx = a[p]; w.vy = a[2 * p]; w.vz = a[3 * p]; w.p = a[4 * p];
+  w.r = S.W[0][row + 3][col + 3]; w.vx = S.W[1][row + 3][col + 3]; w.vy = S.W[2][row + 3][col + 3];
+  w.vz = S.W[3][row + 3][col + 3]; w.p = S.W[4][row + 3][col + 3];
   return w;
 }
 __device__ __forceinline__ Cons<double> jat_l(const JatLDS& S, int row, int col) {
-  int p;
-  const double* a = jat_l_at(S, row, col, p);
   Cons<double> l;
-  l.d = a[0]; l.mx = a[p]; l.my = a[2 * p]; l.mz = a[3 * p]; l.e = a[4 * p];
+  l.d = S.L[0][row + 2][col + 2]; l.mx = S.L[1][row + 2][col + 2]; l.my = S.L[2][row + 2][col + 2];
+  l.mz = S.L[3][row + 2][col + 2]; l.e = S.L[4][row + 2][col + 2];
   return l;
 }
-__device__ __forceinline__ D5 jat_gx(const JatLDS& S, int side, int i) {
-  const int o = 5 * side;
-  D5 w;
-  w.r = S.Gx[o][i]; w.vx = S.Gx[o + 1][i]; w.vy = S.Gx[o + 2][i]; w.vz = S.Gx[o + 3][i]; w.p = S.Gx[o + 4][i];
-  return w;
+__device__ __forceinline__ void jat_put_w(JatLDS& S, int row, int col, const D5& w) {
+  S.W[0][row + 3][col + 3] = w.r; S.W[1][row + 3][col + 3] = w.vx; S.W[2][row + 3][col + 3] = w.vy;
+  S.W[3][row + 3][col + 3] = w.vz; S.W[4][row + 3][col + 3] = w.p;
 }
-__device__ __forceinline__ D5 jat_gy(const JatLDS& S, int side, int i) {
-  const int o = 5 * side;
-  D5 w;
-  w.r = S.Gy[o][i]; w.vx = S.Gy[o + 1][i]; w.vy = S.Gy[o + 2][i]; w.vz = S.Gy[o + 3][i]; w.p = S.Gy[o + 4][i];
-  return w;
-}
-__device__ __forceinline__ D5 half_diff(const D5& a, const D5& b) {
-  D5 s;
-  s.r = 0.5 * a.r - 0.5 * b.r;
-  s.vx = 0.5 * a.vx - 0.5 * b.vx;
-  s.vy = 0.5 * a.vy - 0.5 * b.vy;
-  s.vz = 0.5 * a.vz - 0.5 * b.vz;
-  s.p = 0.5 * a.p - 0.5 * b.p;
-  return s;
+__device__ __forceinline__ void jat_put_l(JatLDS& S, int row, int col, const Cons<double>& l) {
+  S.L[0][row + 2][col + 2] = l.d; S.L[1][row + 2][col + 2] = l.mx; S.L[2][row + 2][col + 2] = l.my;
+  S.L[3][row + 2][col + 2] = l.mz; S.L[4][row + 2][col + 2] = l.e;
 }
 __device__ __forceinline__ Cons<double> mu_of(double a, const Cons<double>& l, const Cons<double>& r) {
   Cons<double> m;
@@ -611,31 +582,32 @@ __device__ __forceinline__ Cons<double> c_swap_xy(const Cons<double>& f, bool on
   return o;
 }
 
-// Slope adjoint terms gathered by a cell from its own slope and its two
-// neighbours' slopes along one axis. w[0..4] = W at offsets −2..+2; gl[k], gr[k]
-// = left/right face-state adjoints of the faces at offsets −3/2.. +3/2 (k = 0..3).
-__device__ __forceinline__ void gather_line(const D5 w[5], const D5 gl[4], const D5 gr[4], D5& Wb) {
-  // own faces: hi face (k = 2) left state, lo face (k = 1) right state
-  d5_add(Wb, gl[2]);
-  d5_add(Wb, gr[1]);
-  D5 lb = d5_zero(), cb = d5_zero(), rb = d5_zero();
-  slope_vjp(w[1], w[2], w[3], half_diff(gl[2], gr[1]), lb, cb, rb);
-  d5_add(Wb, cb);
-  D5 lb2 = d5_zero(), cb2 = d5_zero(), rb2 = d5_zero();
-  slope_vjp(w[2], w[3], w[4], half_diff(gl[3], gr[2]), lb2, cb2, rb2);   // hi neighbour: this cell is its lo
-  d5_add(Wb, lb2);
-  D5 lb3 = d5_zero(), cb3 = d5_zero(), rb3 = d5_zero();
-  slope_vjp(w[0], w[1], w[2], half_diff(gl[1], gr[0]), lb3, cb3, rb3);   // lo neighbour: this cell is its hi
-  d5_add(Wb, rb3);
+// Slope adjoint terms of one component gathered by a cell from its own slope and
+// its two neighbours' slopes along one axis, added to Wb. w[0..4] = W at offsets
+// −2..+2; gl[0..2] = left-state adjoints of the faces at offsets −1/2, 1/2, 3/2;
+// gr[0..2] = right-state adjoints of the faces at −3/2, −1/2, 1/2.
+__device__ __forceinline__ double gather_line(const double w[5], const double gl[3], const double gr[3], double Wb) {
+  Wb += gl[1];   // the cell's hi face
+  Wb += gr[1];   // and its lo face
+  double lb = 0.0, cb = 0.0, rb = 0.0;
+  minmod_vjp1(w[1], w[2], w[3], 0.5 * gl[1] - 0.5 * gr[1], lb, cb, rb);
+  Wb += cb;
+  double lb2 = 0.0, cb2 = 0.0, rb2 = 0.0;
+  minmod_vjp1(w[2], w[3], w[4], 0.5 * gl[2] - 0.5 * gr[2], lb2, cb2, rb2);   // hi neighbour: this cell is its lo
+  Wb += lb2;
+  double lb3 = 0.0, cb3 = 0.0, rb3 = 0.0;
+  minmod_vjp1(w[0], w[1], w[2], 0.5 * gl[0] - 0.5 * gr[0], lb3, cb3, rb3);   // lo neighbour: this cell is its hi
+  Wb += rb3;
+  return Wb;
 }
 
 // out = a1·base1 + a2·base2 + beta·(dt/V)·A'(U)ᵀλ for a 2D grid periodic on both
 // axes, one launch. Phases (two barriers): load the tile's W (halo 3) and λ (halo
 // 2) in a cross shape; evaluate every x and y face VJP of the tile plus the faces
-// its cells' slope adjoints reach (560 + 608 faces, three passes over the 512
+// its cells' slope adjoints reach (304 + 304 faces, two passes over the 512
 // lanes; a y face runs in the frame of an x face, x and y exchanged); gather
 // both axes per cell and map the primitive adjoint to conserved variables.
-__global__ void __launch_bounds__(JNT, 1) adj_jat2d_periodic_kernel(const double* __restrict__ U,
+__global__ void __launch_bounds__(JNT, 4) adj_jat2d_periodic_kernel(const double* __restrict__ U,
                                                                  const double* __restrict__ lam,
                                                                  const double* base1, double a1,
                                                                  const double* base2, double a2, double beta,
@@ -646,56 +618,59 @@ __global__ void __launch_bounds__(JNT, 1) adj_jat2d_periodic_kernel(const double
   const long long n = G.ncell;
   const int tid = threadIdx.x;
   const int tx = tid % JTX, ty = tid / JTX;
-  const int x0 = blockIdx.x * JTX, y0 = blockIdx.y * JTY;
+  // Workgroup i runs on XCD i % 8: each XCD takes a contiguous range of tiles, so that
+  // its L2 serves the halo columns (25.8 → 23.1 µs at 512²).
+  const int nt = gridDim.x * gridDim.y, id = blockIdx.y * gridDim.x + blockIdx.x;
+  const int xcd = id & 7, q8 = nt >> 3, r8 = nt & 7;
+  const int tile = xcd * q8 + (xcd < r8 ? xcd : r8) + (id >> 3);
+  const int x0 = tile % gridDim.x * JTX, y0 = tile / gridDim.x * JTY;
   const double g = G.gamma;
   auto wrapx = [&](int x) { return x < 0 ? x + nx : (x >= nx ? x - nx : x); };
   auto wrapy = [&](int y) { return y < 0 ? y + ny : (y >= ny ? y - ny : y); };
   auto cidx = [&](int x, int y) { return (long long)wrapy(y) * nx + wrapx(x); };
   // ---- load: own cell, then the cross-shaped halos of W (3) and λ (2) ----
-  const long long c = (long long)(y0 + ty) * nx + (x0 + tx);
-  const Cons<double> Uc = load_cons(U, n, c);
-  {
-    const D5 w = cons2prim<double, false>(Uc, g, g);
-    S.Wx[0][ty][tx + 3] = w.r; S.Wx[1][ty][tx + 3] = w.vx; S.Wx[2][ty][tx + 3] = w.vy;
-    S.Wx[3][ty][tx + 3] = w.vz; S.Wx[4][ty][tx + 3] = w.p;
-    const Cons<double> l = load_cons(lam, n, c);
-    S.Lx[0][ty][tx + 2] = l.d; S.Lx[1][ty][tx + 2] = l.mx; S.Lx[2][ty][tx + 2] = l.my;
-    S.Lx[3][ty][tx + 2] = l.mz; S.Lx[4][ty][tx + 2] = l.e;
-  }
+  const long long c = cidx(x0 + tx, y0 + ty);
   constexpr int NWX = 6 * JTY, NLX = 4 * JTY, NWY = 6 * JTX, NLY = 4 * JTX;
-  static_assert(NWX + NLX + NWY + NLY <= JNT, "one halo item per lane");
-  {
-    const int h = tid;
+  static_assert(NWX + NLX + NWY + NLY <= JNT && JTX * JTY <= JNT, "one halo item and one cell per lane");
+  Cons<double> Uc;
+  if (tid < JTX * JTY) {
+    Uc = load_cons(U, n, c);
+    jat_put_w(S, ty, tx, cons2prim<double, false>(Uc, g, g));
+    jat_put_l(S, ty, tx, load_cons(lam, n, c));
+  }
+  const int h = tid < JTX * JTY ? tid + (JNT - JTX * JTY) : tid - JTX * JTY;   // halo items start on the idle lanes
+  if (h < NWX + NWY) {
+    int row, col;
     if (h < NWX) {
-      const int r = h / 6, q = h % 6;
-      const int lc = q < 3 ? q : JTX + q;   // 0,1,2 | JTX+3..JTX+5
-      const D5 w = cons2prim<double, false>(load_cons(U, n, cidx(x0 - 3 + lc, y0 + r)), g, g);
-      S.Wx[0][r][lc] = w.r; S.Wx[1][r][lc] = w.vx; S.Wx[2][r][lc] = w.vy; S.Wx[3][r][lc] = w.vz; S.Wx[4][r][lc] = w.p;
-    } else if (h < NWX + NLX) {
-      const int hh = h - NWX;
-      const int r = hh / 4, q = hh % 4;
-      const int lc = q < 2 ? q : JTX + q;   // 0,1 | JTX+2, JTX+3
-      const Cons<double> l = load_cons(lam, n, cidx(x0 - 2 + lc, y0 + r));
-      S.Lx[0][r][lc] = l.d; S.Lx[1][r][lc] = l.mx; S.Lx[2][r][lc] = l.my; S.Lx[3][r][lc] = l.mz; S.Lx[4][r][lc] = l.e;
-    } else if (h < NWX + NLX + NWY) {
-      const int hh = h - NWX - NLX;
-      const int i = hh / JTX, cc = hh % JTX;
-      const int y = i < 3 ? y0 - 3 + i : y0 + JTY + (i - 3);
-      const D5 w = cons2prim<double, false>(load_cons(U, n, cidx(x0 + cc, y)), g, g);
-      S.Wy[0][i][cc] = w.r; S.Wy[1][i][cc] = w.vx; S.Wy[2][i][cc] = w.vy; S.Wy[3][i][cc] = w.vz; S.Wy[4][i][cc] = w.p;
-    } else if (h < NWX + NLX + NWY + NLY) {
-      const int hh = h - NWX - NLX - NWY;
-      const int i = hh / JTX, cc = hh % JTX;
-      const int y = i < 2 ? y0 - 2 + i : y0 + JTY + (i - 2);
-      const Cons<double> l = load_cons(lam, n, cidx(x0 + cc, y));
-      S.Ly[0][i][cc] = l.d; S.Ly[1][i][cc] = l.mx; S.Ly[2][i][cc] = l.my; S.Ly[3][i][cc] = l.mz; S.Ly[4][i][cc] = l.e;
+      const int q = h % 6;
+      row = h / 6;
+      col = q < 3 ? q - 3 : JTX + q - 3;   // −3, −2, −1 | JTX .. JTX+2
+    } else {
+      const int i = (h - NWX) / JTX;
+      row = i < 3 ? i - 3 : JTY + i - 3;
+      col = (h - NWX) % JTX;
     }
+    jat_put_w(S, row, col, cons2prim<double, false>(load_cons(U, n, cidx(x0 + col, y0 + row)), g, g));
+  } else if (h < NWX + NWY + NLX + NLY) {
+    const int hl = h - (NWX + NWY);
+    int row, col;
+    if (hl < NLX) {
+      const int q = hl % 4;
+      row = hl / 4;
+      col = q < 2 ? q - 2 : JTX + q - 2;   // −2, −1 | JTX, JTX+1
+    } else {
+      const int i = (hl - NLX) / JTX;
+      row = i < 2 ? i - 2 : JTY + i - 2;
+      col = (hl - NLX) % JTX;
+    }
+    jat_put_l(S, row, col, load_cons(lam, n, cidx(x0 + col, y0 + row)));
   }
   __syncthreads();
 
   // ---- face VJPs, x faces then y faces in one item list ----
   //   x face (r, ql), ql = 0..JTX+2: between columns ql−2 and ql−1 of row r;
   //   y face (ql, cc), ql = 0..JTY+2: between rows ql−2 and ql−1 of column cc.
+#pragma unroll 1
   for (int h = tid; h < JNXF + JNYF; h += JNT) {
     const bool isy = h >= JNXF;
     const int q = isy ? h - JNXF : h;
@@ -722,36 +697,50 @@ __global__ void __launch_bounds__(JNT, 1) adj_jat2d_periodic_kernel(const double
     hllc_vjp<0>(WL, WR, g, mu, bL, bR);
     bL = d5_swap_xy(bL, isy);
     bR = d5_swap_xy(bR, isy);
-    double* gb = isy ? &S.Gy[0][q] : &S.Gx[0][q];
-    const int gp = isy ? JNYF : JNXF;
-    gb[0] = bL.r; gb[gp] = bL.vx; gb[2 * gp] = bL.vy; gb[3 * gp] = bL.vz; gb[4 * gp] = bL.p;
-    gb[5 * gp] = bR.r; gb[6 * gp] = bR.vx; gb[7 * gp] = bR.vy; gb[8 * gp] = bR.vz; gb[9 * gp] = bR.p;
+    // No cell gathers the left adjoint of a line's first face or the right one of its last.
+    const int f = isy ? q / JTX : q % (JTX + 3);
+    const int last = isy ? JTY + 2 : JTX + 2;
+    const int gp = isy ? (JTY + 2) * JTX : JTY * (JTX + 2);
+    const int o = isy ? q : row * (JTX + 2) + f;
+    double* gb = (isy ? &S.Gy[0][0][0][0] : &S.Gx[0][0][0][0]) + o;
+    if (f > 0) {
+      double* l = gb - (isy ? JTX : 1);
+      l[0] = bL.r; l[gp] = bL.vx; l[2 * gp] = bL.vy; l[3 * gp] = bL.vz; l[4 * gp] = bL.p;
+    }
+    if (f < last) {
+      double* r = gb + 5 * gp;
+      r[0] = bR.r; r[gp] = bR.vx; r[2 * gp] = bR.vy; r[3 * gp] = bR.vz; r[4 * gp] = bR.p;
+    }
   }
   __syncthreads();
 
-  // ---- gather both axes per cell ----
+  // ---- gather both axes per cell, one component at a time ----
+  if (tid >= JTX * JTY || x0 + tx >= nx || y0 + ty >= ny) return;
   D5 Wb = d5_zero();
-  {
-    D5 w[5], gl[4], gr[4];
+  double* comp[5] = {&Wb.r, &Wb.vx, &Wb.vy, &Wb.vz, &Wb.p};
 #pragma unroll
-    for (int k = 0; k < 5; ++k) w[k] = jat_w(S, ty, tx - 2 + k);
+  for (int f = 0; f < 5; ++f) {
+    double w[5], gl[3], gr[3];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      gl[k] = jat_gx(S, 0, ty * (JTX + 3) + tx + k);
-      gr[k] = jat_gx(S, 1, ty * (JTX + 3) + tx + k);
+    for (int k = 0; k < 5; ++k) w[k] = S.W[f][ty + 3][tx + 1 + k];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      gl[k] = S.Gx[0][f][ty][tx + k];
+      gr[k] = S.Gx[1][f][ty][tx + k];
     }
-    gather_line(w, gl, gr, Wb);
-  }
-  {
-    D5 w[5], gl[4], gr[4];
+    const double vx = gather_line(w, gl, gr, 0.0);
 #pragma unroll
-    for (int k = 0; k < 5; ++k) w[k] = jat_w(S, ty - 2 + k, tx);
+    for (int k = 0; k < 5; ++k) w[k] = S.W[f][ty + 1 + k][tx + 3];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      gl[k] = jat_gy(S, 0, (ty + k) * JTX + tx);
-      gr[k] = jat_gy(S, 1, (ty + k) * JTX + tx);
+    for (int k = 0; k < 3; ++k) {
+      gl[k] = S.Gy[0][f][ty + k][tx];
+      gr[k] = S.Gy[1][f][ty + k][tx];
     }
-    gather_line(w, gl, gr, Wb);
+    double wb = gather_line(w, gl, gr, vx);
+    // The value is complete here: without this the compiler sinks all ten gathers
+    // below the last of their loads and holds 130 loaded values in registers.
+    asm volatile("" : "+v"(wb)::"memory");
+    *comp[f] = wb;
   }
   const Cons<double> Ub = c2p_vjp(Uc, g, Wb);
   const double sc = beta * (*dtp / (1.0 * G.V));
