@@ -7,8 +7,8 @@
 //
 // Bound: the link (57 GB/s each way from pinned memory) and the threads' page faults. Measured,
 // runtime and here (GB/s): down 2 MiB 17.7 and 26.6, 16 MiB 16.9 and 34, 195 MiB 17.5 and 39.4; down
-// into a fresh array of 195 MiB 10.4 and 17.7; up 2 MiB 25.9 and 31.6, 64 MiB 29.5 and 38.5. At 512 KiB
-// both take 27-34 µs, so smaller copies go to the runtime.
+// into a fresh array of 195 MiB 10.4 and 17.7; up 2 MiB 25.9 and 31.6, 64 MiB 29.5 and 38.5. Below 4 MiB
+// what is gained goes into waking the threads: a lone 0.6 MiB download took 50 µs and 130.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -28,7 +28,7 @@ constexpr size_t kPiece = (size_t)128 << 10; // bytes per thread at a time
 constexpr int kSlots = 16;                   // pinned slots of the process (32 MiB)
 constexpr int kSlotsPerCopy = 4;
 // Copies of at most this many bytes go to the runtime.
-constexpr size_t kDirect = (size_t)512 << 10;
+constexpr size_t kDirect = (size_t)4 << 20;
 
 // A slot's event belongs to the device it was made on.
 struct Slot {
