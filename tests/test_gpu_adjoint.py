@@ -165,6 +165,18 @@ def test_fused_tile_form_matches_three_pass_form_and_oracle(O, dims):
     sim.close()
 
 
+@pytest.mark.parametrize("dims,bcs", [
+    ((3, 65), [("reflecting", "outflow"), ("outflow", "reflecting")]),
+    ((130, 2, 3), "outflow"),
+    ((66, 3), "periodic"),
+    ((64, 4, 1 + 2), [("periodic", "periodic"), ("reflecting", "reflecting"), ("outflow", "outflow")]),
+])
+def test_passes_on_lines_shorter_than_the_stencil(O, dims, bcs):
+    """Axes of two and three cells (both boundaries inside one stencil) and cell counts
+    around a wave's 64; the bound is that of the other sizes."""
+    test_step_vjp_matches_oracle(O, dims, bcs, 31)
+
+
 @pytest.mark.parametrize("dims", [(10, 10), (16, 48), (18, 33), (15, 64), (50, 37), (17, 40), (40, 9), (129, 19)])
 def test_fused_tiles_of_any_size(O, dims):
     """Sizes that leave the last tiles partly filled, the smallest that wrap once, and

@@ -9,7 +9,7 @@
 //                     flux VJP applied to area·(λ_left − λ_right) (one side at a
 //                     domain boundary, with the ghost folded back), giving the
 //                     adjoints of the two face states;
-//   adj_cell_kernel   one lane per cell: gathers the face-state adjoints of its
+//   adj_cell_kernel   one lane per cell and axis: gathers the face-state adjoints of its
 //                     own faces and the slope adjoints of itself and its two
 //                     neighbours per axis (minmod active branch), maps the
 //                     primitive adjoint to conserved variables and writes
@@ -277,14 +277,6 @@ __device__ __forceinline__ void minmod_vjp1(double l, double c, double r, double
     cb -= sb;
   }
 }
-__device__ __forceinline__ void slope_vjp(const D5& l, const D5& c, const D5& r, const D5& sb, D5& lb, D5& cb,
-                                          D5& rb) {
-  minmod_vjp1(l.r, c.r, r.r, sb.r, lb.r, cb.r, rb.r);
-  minmod_vjp1(l.vx, c.vx, r.vx, sb.vx, lb.vx, cb.vx, rb.vx);
-  minmod_vjp1(l.vy, c.vy, r.vy, sb.vy, lb.vy, cb.vy, rb.vy);
-  minmod_vjp1(l.vz, c.vz, r.vz, sb.vz, lb.vz, cb.vz, rb.vz);
-  minmod_vjp1(l.p, c.p, r.p, sb.p, lb.p, cb.p, rb.p);
-}
 
 __device__ __forceinline__ D5 load_w(const double* __restrict__ W, long long n, long long c) {
   D5 w;
@@ -315,40 +307,49 @@ __device__ __forceinline__ AxisGeo axis_geo(const GridDev& G) {
   return a;
 }
 
-// Face value of cell c (coordinate p along A) toward side h (±½) with the
-// neighbours resolved: periodic wrap, else the ghost of the cell itself.
-template <int A>
-__device__ __forceinline__ D5 face_state(const double* __restrict__ W, const GridDev& G, long long c, int p, double h) {
-  const AxisGeo ax = axis_geo<A>(G);
-  const long long n = G.ncell;
-  const D5 wc = load_w(W, n, c);
-  const bool per = G.bc[2 * A] == BC_PERIODIC;
-  D5 wl, wr;
-  if (p > 0) wl = load_w(W, n, c - ax.stride);
-  else if (per) wl = load_w(W, n, c + (long long)(ax.n - 1) * ax.stride);
-  else wl = ghost(wc, G.bc[2 * A], A + 1);
-  if (p < ax.n - 1) wr = load_w(W, n, c + ax.stride);
-  else if (per) wr = load_w(W, n, c - (long long)(ax.n - 1) * ax.stride);
-  else wr = ghost(wc, G.bc[2 * A + 1], A + 1);
-  return face_value(wc, slope(wl, wc, wr), h);
+// The three coordinates of slot or cell s in a box of m0 × m1 × any; in 32 bits where all
+// of the box's `total` items fit (a 64-bit quotient is some 100 instructions).
+__device__ __forceinline__ void split3(long long s, long long total, int m0, int m1, int& i, int& j, int& k) {
+  if (total <= 0xffffffffLL) {
+    const unsigned u = (unsigned)s, r = u / (unsigned)m0;
+    i = (int)(u - r * (unsigned)m0);
+    k = (int)(r / (unsigned)m1);
+    j = (int)(r - (unsigned)k * (unsigned)m1);
+  } else {
+    i = (int)(s % m0);
+    j = (int)((s / m0) % m1);
+    k = (int)(s / ((long long)m0 * m1));
+  }
 }
+__device__ __forceinline__ D5 d5_select(bool on, const D5& a, const D5& b) {
+  D5 o;
+  o.r = on ? a.r : b.r; o.vx = on ? a.vx : b.vx; o.vy = on ? a.vy : b.vy; o.vz = on ? a.vz : b.vz; o.p = on ? a.p : b.p;
+  return o;
+}
+
+struct AdjFaces {
+  double* gL[3];
+  double* gR[3];
+};
 
 // Face slots along A: (n_A + 1) per line, slot coordinate q ∈ [0, n_A] is the
 // face between cells q−1 and q (periodic axes use q ∈ [0, n_A) with q = 0 the
-// wrapped face). Output gL/gR: 5 SoA fields over the slots.
+// wrapped face). Output gL/gR: 5 SoA fields over the slots. A domain boundary's face
+// has one side in the grid: the other is its ghost, and the ghost's adjoint folds back.
 template <int A>
-__global__ void __launch_bounds__(256) adj_face_kernel(const double* __restrict__ W, const double* __restrict__ lam,
-                                                       GridDev G, double* __restrict__ gL, double* __restrict__ gR) {
+__device__ __forceinline__ void adj_face(const double* __restrict__ W, const double* __restrict__ lam, const GridDev& G,
+                                         long long s, double* __restrict__ gL, double* __restrict__ gR) {
   const int m0 = A == 0 ? G.n[0] + 1 : G.n[0];
   const int m1 = A == 1 ? G.n[1] + 1 : G.n[1];
   const int m2 = A == 2 ? G.n[2] + 1 : G.n[2];
   const long long ns = (long long)m0 * m1 * m2;
-  const long long s = (long long)blockIdx.x * 256 + threadIdx.x;
   if (s >= ns) return;
-  const int i = (int)(s % m0), j = (int)((s / m0) % m1), k = (int)(s / ((long long)m0 * m1));
+  int i, j, k;
+  split3(s, ns, m0, m1, i, j, k);
   const int q = A == 0 ? i : (A == 1 ? j : k);
   const AxisGeo ax = axis_geo<A>(G);
-  const bool per = G.bc[2 * A] == BC_PERIODIC;
+  const int blo = G.bc[2 * A], bhi = G.bc[2 * A + 1];
+  const bool per = blo == BC_PERIODIC;
   const long long n = G.ncell;
   D5 bL = d5_zero(), bR = d5_zero();
   if (per && q == ax.n) {   // unused slot of a periodic axis
@@ -356,52 +357,64 @@ __global__ void __launch_bounds__(256) adj_face_kernel(const double* __restrict_
     store_w(gR, ns, s, bR);
     return;
   }
-  const int ci = A == 0 ? (q < ax.n ? q : ax.n - 1) : i;
-  const int cj = A == 1 ? (q < ax.n ? q : ax.n - 1) : j;
-  const int ck = A == 2 ? (q < ax.n ? q : ax.n - 1) : k;
-  const long long cell = ((long long)ck * G.n[1] + cj) * G.n[0] + ci;   // cell q (or the last cell at q = n)
+  const bool isL = per || q > 0, isR = q < ax.n;   // is there a cell on this side
+  const int qr = isR ? q : ax.n - 1;
+  const int ql = q > 0 ? q - 1 : (per ? ax.n - 1 : 0);
+  const int ci = A == 0 ? qr : i, cj = A == 1 ? qr : j, ck = A == 2 ? qr : k;
+  const long long cr = ((long long)ck * G.n[1] + cj) * G.n[0] + ci;   // cell q (or the last cell at q = n)
+  const long long cl = cr + (long long)(ql - qr) * ax.stride;         // cell q−1 (or the first at q = 0)
+  const bool hll = ql > 0 || per, hrr = qr < ax.n - 1 || per;
+  const long long cll = ql > 0 ? cl - ax.stride : (per ? cl + (long long)(ax.n - 1) * ax.stride : cl);
+  const long long crr = qr < ax.n - 1 ? cr + ax.stride : (per ? cr - (long long)(ax.n - 1) * ax.stride : cr);
+  // All four cells of the face's line are read at once; ghosts replace by selection.
+  D5 w0 = load_w(W, n, cll), w1 = load_w(W, n, cl), w2 = load_w(W, n, cr), w3 = load_w(W, n, crr);
+  Cons<double> ll = load_cons(lam, n, cl), lr = load_cons(lam, n, cr);
+  const D5 c1 = w1;
+  w1 = d5_select(isL, w1, ghost(w2, blo, A + 1));
+  w2 = d5_select(isR, w2, ghost(c1, bhi, A + 1));
+  w0 = d5_select(hll, w0, ghost(c1, blo, A + 1));
+  w3 = d5_select(hrr, w3, ghost(w2, bhi, A + 1));
+  D5 WL = face_value(w1, slope(w0, w1, w2), 0.5);
+  D5 WR = face_value(w2, slope(w1, w2, w3), -0.5);
+  if (!isL) WL = ghost(WR, blo, A + 1);
+  if (!isR) WR = ghost(WL, bhi, A + 1);
   const double a = G.area[A];
-  const double g = G.gamma;
-  if (q == 0 && !per) {
-    // lo boundary face: F = hllc(ghost(WR), WR), acc[0] −= a·F
-    const D5 WR = face_state<A>(W, G, cell, 0, -0.5);
-    const D5 Wg = ghost(WR, G.bc[2 * A], A + 1);
-    const Cons<double> lr = load_cons(lam, n, cell);
-    Cons<double> mu;
-    mu.d = -a * lr.d; mu.mx = -a * lr.mx; mu.my = -a * lr.my; mu.mz = -a * lr.mz; mu.e = -a * lr.e;
-    D5 gb = d5_zero();
-    hllc_vjp<A>(Wg, WR, g, mu, gb, bR);
-    d5_add(bR, ghostT<A>(gb, G.bc[2 * A]));
-  } else if (q == ax.n) {
-    // hi boundary face: F = hllc(WL, ghost(WL)), acc[n−1] += a·F
-    const D5 WL = face_state<A>(W, G, cell, ax.n - 1, 0.5);
-    const D5 Wg = ghost(WL, G.bc[2 * A + 1], A + 1);
-    const Cons<double> ll = load_cons(lam, n, cell);
-    Cons<double> mu;
-    mu.d = a * ll.d; mu.mx = a * ll.mx; mu.my = a * ll.my; mu.mz = a * ll.mz; mu.e = a * ll.e;
-    D5 gb = d5_zero();
-    hllc_vjp<A>(WL, Wg, g, mu, bL, gb);
-    d5_add(bL, ghostT<A>(gb, G.bc[2 * A + 1]));
-  } else {
-    // interior (or wrapped) face between cells q−1 and q
-    const long long cl = q > 0 ? cell - ax.stride : cell + (long long)(ax.n - 1) * ax.stride;
-    const int ql = q > 0 ? q - 1 : ax.n - 1;
-    const D5 WL = face_state<A>(W, G, cl, ql, 0.5);
-    const D5 WR = face_state<A>(W, G, cell, q, -0.5);
-    const Cons<double> ll = load_cons(lam, n, cl), lr = load_cons(lam, n, cell);
-    Cons<double> mu;
-    mu.d = a * ll.d - a * lr.d;
-    mu.mx = a * ll.mx - a * lr.mx;
-    mu.my = a * ll.my - a * lr.my;
-    mu.mz = a * ll.mz - a * lr.mz;
-    mu.e = a * ll.e - a * lr.e;
-    hllc_vjp<A>(WL, WR, g, mu, bL, bR);
+  const double z = 0.0;
+  Cons<double> mu;
+  mu.d = (isL ? a * ll.d : z) - (isR ? a * lr.d : z);
+  mu.mx = (isL ? a * ll.mx : z) - (isR ? a * lr.mx : z);
+  mu.my = (isL ? a * ll.my : z) - (isR ? a * lr.my : z);
+  mu.mz = (isL ? a * ll.mz : z) - (isR ? a * lr.mz : z);
+  mu.e = (isL ? a * ll.e : z) - (isR ? a * lr.e : z);
+  hllc_vjp<A>(WL, WR, G.gamma, mu, bL, bR);
+  if (!isL) {
+    d5_add(bR, ghostT<A>(bL, blo));
+    bL = d5_zero();
+  }
+  if (!isR) {
+    d5_add(bL, ghostT<A>(bR, bhi));
+    bR = d5_zero();
   }
   store_w(gL, ns, s, bL);
   store_w(gR, ns, s, bR);
 }
 
-// Primitive adjoint gathered by cell c from axis A.
+// The axes' faces in one launch (blockIdx.y = axis): a small grid leaves the chip part
+// idle in a launch of each. Bound: latency of the dependent loads, then hllc_vjp's arithmetic
+// (112 registers, 4 waves per SIMD); one hllc_vjp serves inner and boundary faces, where a
+// wave that held both went through it three times. 60×52×44: three launches of 15.0, 10.7 and
+// 10.6 µs → 16.4 µs.
+template <int RANK>
+__global__ void __launch_bounds__(256) adj_face_kernel(const double* __restrict__ W, const double* __restrict__ lam,
+                                                       GridDev G, AdjFaces F) {
+  const long long s = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (RANK == 1 || blockIdx.y == 0) adj_face<0>(W, lam, G, s, F.gL[0], F.gR[0]);
+  else if (RANK == 2 || blockIdx.y == 1) adj_face<RANK == 1 ? 0 : 1>(W, lam, G, s, F.gL[1], F.gR[1]);
+  else adj_face<RANK == 3 ? 2 : 0>(W, lam, G, s, F.gL[2], F.gR[2]);
+}
+
+// Primitive adjoint gathered by cell c (coordinate p along A) from axis A, added to Wb. The line's
+// cells p−2..p+2 and faces are read at once, at the cell's own place where there is none.
 template <int A>
 __device__ __forceinline__ void gather_axis(const double* __restrict__ W, const double* __restrict__ gL,
                                             const double* __restrict__ gR, const GridDev& G, long long c, int i, int j,
@@ -413,99 +426,109 @@ __device__ __forceinline__ void gather_axis(const double* __restrict__ W, const 
   const long long ns = (long long)m0 * m1 * m2;
   const int p = A == 0 ? i : (A == 1 ? j : k);
   const int nA = ax.n;
-  const bool per = G.bc[2 * A] == BC_PERIODIC;
+  const int blo = G.bc[2 * A], bhi = G.bc[2 * A + 1];
+  const bool per = blo == BC_PERIODIC;
   const long long n = G.ncell;
-  // slot of face coordinate qf along A (wrapped on periodic axes)
-  auto slot = [&](int qf) -> long long {
-    if (per) qf = qf < 0 ? qf + nA : (qf >= nA ? qf - nA : qf);
-    const int si = A == 0 ? qf : i, sj = A == 1 ? qf : j, sk = A == 2 ? qf : k;
-    return ((long long)sk * m1 + sj) * m0 + si;
+  const long long fstride = A == 0 ? 1 : (A == 1 ? (long long)m0 : (long long)m0 * m1);
+  const long long f0 = ((long long)k * m1 + j) * m0 + i;   // slot of the lo face
+  // slot of face coordinate p + d and cell at p + d (wrapped on periodic axes, also those of
+  // one cell; clamped else)
+  auto slot = [&](int d) -> long long {
+    int x = p + d;
+    if (per) x = x < 0 ? max(x + nA, 0) : (x >= nA ? min(x - nA, nA - 1) : x);
+    else x = x < 0 ? 0 : (x > nA ? nA : x);
+    return f0 + (long long)(x - p) * fstride;
   };
-  auto cell_at = [&](int pp) -> long long {   // cell at coordinate pp (wrapped when periodic)
-    if (per) pp = pp < 0 ? pp + nA : (pp >= nA ? pp - nA : pp);
-    return c + (long long)(pp - p) * ax.stride;
+  auto cell_at = [&](int d) -> long long {
+    int x = p + d;
+    if (per) x = x < 0 ? max(x + nA, 0) : (x >= nA ? min(x - nA, nA - 1) : x);
+    else x = x < 0 ? 0 : (x >= nA ? nA - 1 : x);
+    return c + (long long)(x - p) * ax.stride;
   };
-  const D5 wc = load_w(W, n, c);
-  // own faces
-  const D5 ghi = load_w(gL, ns, slot(p + 1));
-  const D5 glo = load_w(gR, ns, slot(p));
-  d5_add(Wb, ghi);
-  d5_add(Wb, glo);
-  // own slope
-  {
-    const bool hl = p > 0 || per, hr = p < nA - 1 || per;
-    const D5 wl = hl ? load_w(W, n, cell_at(p - 1)) : ghost(wc, G.bc[2 * A], A + 1);
-    const D5 wr = hr ? load_w(W, n, cell_at(p + 1)) : ghost(wc, G.bc[2 * A + 1], A + 1);
-    D5 sb;
-    sb.r = 0.5 * ghi.r - 0.5 * glo.r;
-    sb.vx = 0.5 * ghi.vx - 0.5 * glo.vx;
-    sb.vy = 0.5 * ghi.vy - 0.5 * glo.vy;
-    sb.vz = 0.5 * ghi.vz - 0.5 * glo.vz;
-    sb.p = 0.5 * ghi.p - 0.5 * glo.p;
-    D5 lb = d5_zero(), cb = d5_zero(), rb = d5_zero();
-    slope_vjp(wl, wc, wr, sb, lb, cb, rb);
-    d5_add(Wb, cb);
-    if (!hl) d5_add(Wb, ghostT<A>(lb, G.bc[2 * A]));
-    if (!hr) d5_add(Wb, ghostT<A>(rb, G.bc[2 * A + 1]));
-  }
-  // slope of the hi neighbour h (c is its lo neighbour)
-  if (p < nA - 1 || per) {
-    const long long h = cell_at(p + 1);
-    const D5 wh = load_w(W, n, h);
-    const bool hr = p + 1 < nA - 1 || per;
-    const D5 whr = hr ? load_w(W, n, cell_at(p + 2)) : ghost(wh, G.bc[2 * A + 1], A + 1);
-    const D5 a = load_w(gL, ns, slot(p + 2)), b = load_w(gR, ns, slot(p + 1));
-    D5 sb;
-    sb.r = 0.5 * a.r - 0.5 * b.r;
-    sb.vx = 0.5 * a.vx - 0.5 * b.vx;
-    sb.vy = 0.5 * a.vy - 0.5 * b.vy;
-    sb.vz = 0.5 * a.vz - 0.5 * b.vz;
-    sb.p = 0.5 * a.p - 0.5 * b.p;
-    D5 lb = d5_zero(), cb = d5_zero(), rb = d5_zero();
-    slope_vjp(wc, wh, whr, sb, lb, cb, rb);
-    d5_add(Wb, lb);
-  }
-  // slope of the lo neighbour l (c is its hi neighbour)
-  if (p > 0 || per) {
-    const long long l = cell_at(p - 1);
-    const D5 wl = load_w(W, n, l);
-    const bool hl = p - 1 > 0 || per;
-    const D5 wll = hl ? load_w(W, n, cell_at(p - 2)) : ghost(wl, G.bc[2 * A], A + 1);
-    const D5 a = load_w(gL, ns, slot(p)), b = load_w(gR, ns, slot(p - 1));
-    D5 sb;
-    sb.r = 0.5 * a.r - 0.5 * b.r;
-    sb.vx = 0.5 * a.vx - 0.5 * b.vx;
-    sb.vy = 0.5 * a.vy - 0.5 * b.vy;
-    sb.vz = 0.5 * a.vz - 0.5 * b.vz;
-    sb.p = 0.5 * a.p - 0.5 * b.p;
-    D5 lb = d5_zero(), cb = d5_zero(), rb = d5_zero();
-    slope_vjp(wll, wl, wc, sb, lb, cb, rb);
-    d5_add(Wb, rb);
+  const bool hl = p > 0 || per, hr = p < nA - 1 || per;
+  const bool hl2 = p > 1 || per, hr2 = p < nA - 2 || per;
+  const long long cc[5] = {cell_at(-2), cell_at(-1), c, cell_at(1), cell_at(2)};
+  const long long sl[3] = {slot(0), slot(1), slot(2)}, sr[3] = {slot(-1), slot(0), slot(1)};
+  double* out[5] = {&Wb.r, &Wb.vx, &Wb.vy, &Wb.vz, &Wb.p};
+#pragma unroll
+  for (int f = 0; f < 5; ++f) {
+    const double* Wf = W + f * n;
+    const double* gl = gL + f * ns;
+    const double* gr = gR + f * ns;
+    double w[5], l[3], r[3];
+#pragma unroll
+    for (int d = 0; d < 5; ++d) w[d] = Wf[cc[d]];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      l[d] = gl[sl[d]];
+      r[d] = gr[sr[d]];
+    }
+    const bool flipl = f == A + 1 && blo == BC_REFLECTING, fliph = f == A + 1 && bhi == BC_REFLECTING;
+    if (!hl) w[1] = flipl ? -w[2] : w[2];
+    if (!hr) w[3] = fliph ? -w[2] : w[2];
+    if (!hl2) w[0] = flipl ? -w[1] : w[1];
+    if (!hr2) w[4] = fliph ? -w[3] : w[3];
+    double v = *out[f];
+    v += l[1];   // own hi face
+    v += r[1];   // own lo face
+    double lb = 0.0, cb = 0.0, rb = 0.0;
+    minmod_vjp1(w[1], w[2], w[3], 0.5 * l[1] - 0.5 * r[1], lb, cb, rb);
+    v += cb;
+    if (!hl) v += flipl ? -lb : lb;
+    if (!hr) v += fliph ? -rb : rb;
+    double lb2 = 0.0, cb2 = 0.0, rb2 = 0.0;
+    minmod_vjp1(w[2], w[3], w[4], 0.5 * l[2] - 0.5 * r[2], lb2, cb2, rb2);   // hi neighbour: c is its lo
+    if (hr) v += lb2;
+    double lb3 = 0.0, cb3 = 0.0, rb3 = 0.0;
+    minmod_vjp1(w[0], w[1], w[2], 0.5 * l[0] - 0.5 * r[0], lb3, cb3, rb3);   // lo neighbour: c is its hi
+    if (hl) v += rb3;
+    asm volatile("" : "+v"(v)::"memory");   // complete here: keeps the next field's loads out of this one's registers
+    *out[f] = v;
   }
 }
 
-struct AdjFaces {
-  const double* gL[3];
-  const double* gR[3];
-};
-
 // out = a1·base1 + a2·base2 + (beta·dt/V)·A'(U)ᵀλ (base2 may be null). out may
 // alias base1 or base2 (each lane reads and writes its own cell only).
+// One wave per axis of 64 cells, the sums joined through LDS: a lane that walked the axes one
+// after the other left 2 waves per SIMD at 60×52×44 and its loads in a chain. Field by field
+// the gather needs 68 registers; with all fields' loads in flight it needs 186 and is slower.
+// 60×52×44: 26.7 → 21.1 µs (25.0 with 186 registers). Whole A'ᵀλ in passes, before and now (µs):
+// 200 cells 12.0, 11.9; 60² 25.9, 13.7; 400² 51, 39; 1200×1000 279, 236; 24×20×16 31.5, 14.9;
+// 60×52×44 64.6, 42.7; 128×128×96 488, 418.
 template <int RANK>
-__global__ void __launch_bounds__(256) adj_cell_kernel(const double* __restrict__ U, const double* __restrict__ W,
+__global__ void __launch_bounds__(64 * RANK) adj_cell_kernel(const double* __restrict__ U, const double* __restrict__ W,
                                                        AdjFaces F, const double* base1, double a1,
                                                        const double* base2, double a2, double beta,
                                                        const double* __restrict__ dtp, GridDev G, double* out) {
-  const long long c = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (c >= G.ncell) return;
-  const int i = (int)(c % G.n[0]), j = (int)((c / G.n[0]) % G.n[1]), k = (int)(c / ((long long)G.n[0] * G.n[1]));
-  D5 Wb = d5_zero();
-  gather_axis<0>(W, F.gL[0], F.gR[0], G, c, i, j, k, Wb);
-  if constexpr (RANK > 1) gather_axis<1>(W, F.gL[1], F.gR[1], G, c, i, j, k, Wb);
-  if constexpr (RANK > 2) gather_axis<2>(W, F.gL[2], F.gR[2], G, c, i, j, k, Wb);
-  const Cons<double> Ub = c2p_vjp(load_cons(U, G.ncell, c), G.gamma, Wb);
-  const double s = beta * (*dtp / (1.0 * G.V));
+  __shared__ double part[RANK > 1 ? RANK - 1 : 1][5][64];
   const long long n = G.ncell;
+  const int lane = threadIdx.x & 63, axis = threadIdx.x >> 6;
+  const long long c = (long long)blockIdx.x * 64 + lane;
+  const bool on = c < n;
+  D5 Wb = d5_zero();
+  if (on) {
+    int i, j, k;
+    split3(c, n, G.n[0], G.n[1], i, j, k);
+    if (RANK == 1 || axis == 0) gather_axis<0>(W, F.gL[0], F.gR[0], G, c, i, j, k, Wb);
+    else if (RANK == 2 || axis == 1) gather_axis<RANK == 1 ? 0 : 1>(W, F.gL[1], F.gR[1], G, c, i, j, k, Wb);
+    else gather_axis<RANK == 3 ? 2 : 0>(W, F.gL[2], F.gR[2], G, c, i, j, k, Wb);
+  }
+  if constexpr (RANK > 1) {
+    if (axis > 0) {
+      double(*o)[64] = part[axis - 1];
+      o[0][lane] = Wb.r; o[1][lane] = Wb.vx; o[2][lane] = Wb.vy; o[3][lane] = Wb.vz; o[4][lane] = Wb.p;
+    }
+    __syncthreads();
+    if (axis > 0) return;
+#pragma unroll
+    for (int x = 0; x < RANK - 1; ++x) {
+      Wb.r += part[x][0][lane]; Wb.vx += part[x][1][lane]; Wb.vy += part[x][2][lane]; Wb.vz += part[x][3][lane];
+      Wb.p += part[x][4][lane];
+    }
+  }
+  if (!on) return;
+  const Cons<double> Ub = c2p_vjp(load_cons(U, n, c), G.gamma, Wb);
+  const double s = beta * (*dtp / (1.0 * G.V));
   const double ub[5] = {Ub.d, Ub.mx, Ub.my, Ub.mz, Ub.e};
 #pragma unroll
   for (int f = 0; f < 5; ++f) {

@@ -1,6 +1,8 @@
 // Launchers of the reverse-mode kernels (adjoint.h), Float64 uniform grids.
 // Built once, in the fast arithmetic profile (FMA contraction, refined hardware
 // reciprocals): the reverse mode needs no bit parity with the reference.
+#include <algorithm>
+
 #include "adjoint.h"
 #include "host.h"
 
@@ -18,36 +20,46 @@ void adj_launch_prim(hipStream_t s, const double* U, double* W, const GridDev& G
   hipLaunchKernelGGL(VH_PROFILE_NS::adj_prim_kernel, dim3(grid_for(G.ncell)), dim3(256), 0, s, U, W, G);
 }
 
+static VH_PROFILE_NS::AdjFaces faces_of(double* const gL[3], double* const gR[3], int rank) {
+  VH_PROFILE_NS::AdjFaces F{};
+  for (int d = 0; d < rank; ++d) {
+    F.gL[d] = gL[d];
+    F.gR[d] = gR[d];
+  }
+  return F;
+}
+
+template <int RANK>
+static void launch_faces(hipStream_t s, const double* W, const double* lam, const GridDev& G,
+                         const VH_PROFILE_NS::AdjFaces& F) {
+  long long slots = 0;
+  for (int d = 0; d < RANK; ++d) slots = std::max(slots, adj_face_slots(G, d));
+  hipLaunchKernelGGL(VH_PROFILE_NS::adj_face_kernel<RANK>, dim3(grid_for(slots), RANK), dim3(256), 0, s, W, lam, G, F);
+}
+
 void adj_launch_faces(hipStream_t s, const double* W, const double* lam, const GridDev& G, double* const gL[3],
                       double* const gR[3]) {
-  hipLaunchKernelGGL(VH_PROFILE_NS::adj_face_kernel<0>, dim3(grid_for(adj_face_slots(G, 0))), dim3(256), 0, s, W, lam, G,
-                     gL[0], gR[0]);
-  if (G.rank > 1)
-    hipLaunchKernelGGL(VH_PROFILE_NS::adj_face_kernel<1>, dim3(grid_for(adj_face_slots(G, 1))), dim3(256), 0, s, W, lam, G,
-                       gL[1], gR[1]);
-  if (G.rank > 2)
-    hipLaunchKernelGGL(VH_PROFILE_NS::adj_face_kernel<2>, dim3(grid_for(adj_face_slots(G, 2))), dim3(256), 0, s, W, lam, G,
-                       gL[2], gR[2]);
+  const VH_PROFILE_NS::AdjFaces F = faces_of(gL, gR, G.rank);
+  if (G.rank == 3) launch_faces<3>(s, W, lam, G, F);
+  else if (G.rank == 2) launch_faces<2>(s, W, lam, G, F);
+  else launch_faces<1>(s, W, lam, G, F);
+}
+
+template <int RANK>
+static void launch_cells(hipStream_t s, const double* U, const double* W, const VH_PROFILE_NS::AdjFaces& F,
+                         const double* base1, double a1, const double* base2, double a2, double beta,
+                         const double* dtp, const GridDev& G, double* out) {
+  hipLaunchKernelGGL(VH_PROFILE_NS::adj_cell_kernel<RANK>, dim3((unsigned)((G.ncell + 63) / 64)), dim3(64 * RANK), 0, s,
+                     U, W, F, base1, a1, base2, a2, beta, dtp, G, out);
 }
 
 void adj_launch_cells(hipStream_t s, const double* U, const double* W, double* const gL[3], double* const gR[3],
                       const double* base1, double a1, const double* base2, double a2, double beta,
                       const double* dtp, const GridDev& G, double* out) {
-  VH_PROFILE_NS::AdjFaces F;
-  for (int d = 0; d < 3; ++d) {
-    F.gL[d] = gL[d];
-    F.gR[d] = gR[d];
-  }
-  const dim3 grid(grid_for(G.ncell));
-  if (G.rank == 3)
-    hipLaunchKernelGGL(VH_PROFILE_NS::adj_cell_kernel<3>, grid, dim3(256), 0, s, U, W, F, base1, a1, base2, a2, beta, dtp, G,
-                       out);
-  else if (G.rank == 2)
-    hipLaunchKernelGGL(VH_PROFILE_NS::adj_cell_kernel<2>, grid, dim3(256), 0, s, U, W, F, base1, a1, base2, a2, beta, dtp, G,
-                       out);
-  else
-    hipLaunchKernelGGL(VH_PROFILE_NS::adj_cell_kernel<1>, grid, dim3(256), 0, s, U, W, F, base1, a1, base2, a2, beta, dtp, G,
-                       out);
+  const VH_PROFILE_NS::AdjFaces F = faces_of(gL, gR, G.rank);
+  if (G.rank == 3) launch_cells<3>(s, U, W, F, base1, a1, base2, a2, beta, dtp, G, out);
+  else if (G.rank == 2) launch_cells<2>(s, U, W, F, base1, a1, base2, a2, beta, dtp, G, out);
+  else launch_cells<1>(s, U, W, F, base1, a1, base2, a2, beta, dtp, G, out);
 }
 
 bool adj_launch_jat_fused(hipStream_t s, const double* U, const double* lam, const double* base1, double a1,
@@ -60,8 +72,8 @@ bool adj_launch_jat_fused(hipStream_t s, const double* U, const double* lam, con
   if (out == U || out == lam) return false;   // other tiles read these cells; the passes read them before out is written
   // The last tile's halo (two cells past the tile) has to wrap around once only:
   // every size but 1..9 and 17. The fused form is the faster one at all the others:
-  // 10² 15.3 µs in passes, 7.7 fused; 50×37 21 and 11; 100² 23 and 10; 512² 67 and 23;
-  // 1500×1100 391 and 134; 2048² 848 and 353.
+  // 10² 10.8 µs in passes, 7.7 fused; 50×37 14 and 11; 100² 15 and 10; 512² 47 and 23;
+  // 1500×1100 319 and 134; 2048² 749 and 352.
   const int tx = (G.n[0] + JTX - 1) / JTX, ty = (G.n[1] + JTY - 1) / JTY;
   if (tx * JTX + 2 >= 2 * G.n[0] || ty * JTY + 2 >= 2 * G.n[1]) return false;
   const dim3 grid(tx, ty);
