@@ -549,9 +549,9 @@ def gravity_leg(V, args):
     warm = time.perf_counter() - t0
     ncell = n ** 3
     per_it = cold / max(it_cold, 1)
-    # algorithmic HBM bytes per CG iteration: matvec 16 B/cell (read p, write Ap),
-    # update 48 B/cell (read φ, r, p, Ap; write φ, r), direction 24 B/cell (read r, p; write p)
-    bytes_it = 88 * ncell
+    # algorithmic HBM bytes per CG iteration: direction and p·Ap 24 B/cell (read r, p; write p),
+    # update 40 B/cell (read φ, r, p, with Ap formed again from p; write φ, r)
+    bytes_it = 64 * ncell
     res = {"workload": f"3D {n}^3 periodic Jeans ripple, gamma=5/3, G=1, CG tol 1e-8, FP64 {args.mode} profile",
            "cells": ncell,
            "poisson_cold": {"iterations": it_cold, "relres": rr_cold, "seconds": cold,
