@@ -195,6 +195,18 @@ def test_evolve_in_legs_bitwise(O, graph):
     s.close()
 
 
+@pytest.mark.parametrize("graph", [True, False])
+def test_infinite_final_time_ends_the_loop(graph):
+    """As on uniform grids: without a CFL limit the first step takes t to infinity."""
+    m = two_level_2d()
+    s = _sim(m, np.float64, use_graph=graph)
+    U = np.zeros((5, m.ncell))
+    U[0] = 1.0
+    s.upload(U)
+    assert s.evolve(np.inf, max_steps=20) == (np.inf, 1)
+    s.close()
+
+
 @pytest.mark.parametrize("nblocks,edges,most", [(3, (8, 16), 1), (12, (8, 16, 24, 32), 2), (40, (6, 16, 24), 6)])
 def test_default_chunks_and_side_streams_bitwise(O, nblocks, edges, most):
     """The default z planes per tile follow the mesh (short on meshes that do not fill the

@@ -172,6 +172,29 @@ def test_line_step_loop_bitwise(V, O, n, bc, dtype):
     sim.close()
 
 
+@pytest.mark.parametrize("dims", [(50,), (2100,), (12, 10), (9, 8, 7)])
+def test_infinite_final_time_ends_the_loop(V, dims):
+    """tfinal = inf is a final time: the loop ends when t is no longer below it. A gas
+    at rest without pressure has no CFL limit, so its first step takes t to infinity."""
+    U = np.zeros((5,) + tuple(reversed(dims)))
+    U[0] = 1.0
+    sim = make_sim(V, dims, [(2, 2)] * len(dims), 1.4, np.float64, U)
+    sim.problem.tfinal = np.inf
+    V.evolve(sim, max_steps=20)
+    assert (sim.step_count, sim.t) == (1, np.inf)
+    # with a CFL limit the steps are those of a run without a final time
+    U0 = smooth_state(dims, seed=5)
+    out = []
+    for run in (lambda: V.evolve(sim, max_steps=20), lambda: V.run_steps(sim, 20)):
+        sim.upload(U0)
+        sim.t, sim.step_count = 0.0, 0
+        run()
+        out.append((sim.step_count, sim.t, sim.state()))
+    assert out[0][:2] == out[1][:2] and out[0][0] == 20
+    assert np.array_equal(out[0][2], out[1][2])
+    sim.close()
+
+
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_device_dt_loop_bitwise(V, O, dtype):
     dims = (40, 24, 20)

@@ -66,8 +66,8 @@ hipError_t copy_down(void* host, const void* dev, size_t bytes, hipStream_t s);
 
 // Clock kernels of the uniform-grid context, shared with the block context.
 // clock (kClockDoubles): [0] t, [1] dt, [2] max CFL term, [3] steps; of a step loop also
-// [4] cfl, [5] tfinal (infinite: no clip), [6] the time at which the loop ends, [7] non-zero
-// once it has ended. `host` is pinned memory that receives a copy (null: none).
+// [4] cfl, [5] tfinal (0: none; infinite is a final time as any other), [6] the time at which
+// the loop ends, [7] non-zero once it has ended. `host` is pinned memory that receives a copy (null: none).
 constexpr int kClockDoubles = 8;
 void enqueue_dt_finalize(hipStream_t s, const double* partials, int np, double cfl, double* clock, double* host);
 void enqueue_set_dt(hipStream_t s, double* clock, double dt);

@@ -35,7 +35,7 @@ struct LineLDS {
 };
 
 // At most max_steps steps from U in place and time t, to tstop and no further than tfinal
-// (infinite: no final time). host: the clock (host.h) at the end. PL: items per lane.
+// (0: no final time). host: the clock (host.h) at the end. PL: items per lane.
 template <typename T, bool FLOOR64, int PL>
 __global__ void __launch_bounds__(kLineLanes, 1) rk_line_kernel(T* __restrict__ U, GridDev G, double t, double cflnum,
                                                                 double tfinal, double tstop, long long max_steps,
@@ -46,7 +46,7 @@ __global__ void __launch_bounds__(kLineLanes, 1) rk_line_kernel(T* __restrict__ 
   const long long nn = n;
   const int blo = G.bc[0], bhi = G.bc[1];
   const bool per = blo == BC_PERIODIC;
-  const bool clip = tfinal < HUGE_VAL;
+  const bool clip = tfinal > 0.0;
   double dt = 0.0, m = 0.0;
   long long k = 0;
   T* wf = &S.w[0][0];

@@ -56,7 +56,7 @@ __device__ __forceinline__ void clock_to_host(const double* clock, double* host)
 __device__ __forceinline__ void clock_next(double* clock, double m, double* dt_log) {
   const double tfinal = clock[5];
   double dt = m == 0.0 ? HUGE_VAL : clock[4] / m;
-  if (tfinal < HUGE_VAL) {
+  if (tfinal > 0.0) {
     dt = vmin(dt, tfinal - clock[0]);
     if (!(clock[0] < clock[6])) clock[7] = 1.0;
   }
@@ -146,7 +146,7 @@ void enqueue_set_dt(hipStream_t s, double* clock, double dt) {
 void enqueue_loop_begin(hipStream_t s, const double* partials, int np, double t, double cfl, double tfinal, bool clip,
                         double* clock, double* dt_log) {
   hipLaunchKernelGGL(loop_begin_kernel, dim3(1), dim3(kClockLanes), 0, s, partials, np, t, cfl,
-                     clip ? tfinal : HUGE_VAL, tfinal * (1 - 1e-12), clock, dt_log);
+                     clip ? tfinal : 0.0, tfinal * (1 - 1e-12), clock, dt_log);
 }
 void enqueue_step_tail(hipStream_t s, const double* partials, int np, double* clock, double* host, double* dt_log) {
   hipLaunchKernelGGL(step_tail_kernel, dim3(1), dim3(kClockLanes), 0, s, partials, np, clock, host, dt_log);
@@ -740,9 +740,9 @@ static int run_line(vh_grid* g, double cfl, double tfinal, int64_t max_steps, do
   while ((max_steps <= 0 || k < max_steps) && (!clip || *t_io < tstop)) {
     const int64_t n = max_steps > 0 ? std::min(max_steps - k, kMost) : kMost;
     if (g->mode == VH_FAST)
-      fast::launch_line(g->dtype, g->stream, g->U, g->G, *t_io, cfl, clip ? tfinal : HUGE_VAL, tstop, n, clk);
+      fast::launch_line(g->dtype, g->stream, g->U, g->G, *t_io, cfl, clip ? tfinal : 0.0, tstop, n, clk);
     else
-      exact::launch_line(g->dtype, g->stream, g->U, g->G, *t_io, cfl, clip ? tfinal : HUGE_VAL, tstop, n, clk);
+      exact::launch_line(g->dtype, g->stream, g->U, g->G, *t_io, cfl, clip ? tfinal : 0.0, tstop, n, clk);
     VH_HIP(hipGetLastError());
     VH_HIP(hipStreamSynchronize(g->stream));
     *t_io = clk[0];
