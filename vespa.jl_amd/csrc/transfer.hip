@@ -95,13 +95,15 @@ void copy_pieces(char* dst, const char* src, size_t n) {
   });
 }
 
-bool is_pinned(const void* p) {
+// Ordinary host memory: what the runtime knows nothing of. Pinned, managed and device memory
+// given as the host side is the runtime's to copy (a CPU copy could not read the last).
+bool is_pageable(const void* p) {
   hipPointerAttribute_t a{};
   if (hipPointerGetAttributes(&a, p) != hipSuccess) {
     (void)hipGetLastError();
-    return false;
+    return true;
   }
-  return a.type == hipMemoryTypeHost;
+  return a.type == hipMemoryTypeUnregistered;
 }
 
 hipError_t staged(char* dst, const char* src, size_t bytes, bool up, hipStream_t s, const std::vector<Slot>& slots) {
@@ -142,7 +144,7 @@ hipError_t host_copy(void* dst, const void* src, size_t bytes, bool up, hipStrea
   if (e != hipSuccess) return e;
   // the slots' events are the current device's: a stream of another takes the plain copy
   if (!s || hipStreamGetDevice(s, &stream_device) != hipSuccess) stream_device = device;
-  if (bytes > kDirect && HostPool::threads() > 1 && stream_device == device && !is_pinned(up ? src : dst)) {
+  if (bytes > kDirect && HostPool::threads() > 1 && stream_device == device && is_pageable(up ? src : dst)) {
     const size_t chunks = (bytes + kChunk - 1) / kChunk;
     std::vector<Slot> slots = slot_pool().take((int)std::min<size_t>(kSlotsPerCopy, chunks), device);
     bool usable = !slots.empty();
