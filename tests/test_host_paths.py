@@ -60,3 +60,17 @@ def test_device_memory_as_the_host_side_is_not_touched_by_the_cpu(stub):
         assert len([l for l in log() if l[0] == "copy"]) == 4
         assert C.string_at(a.ptr, 8 * MIB) == h.tobytes()
         """)
+
+
+def test_copies_without_threads(stub):
+    """Where no thread can be made (a process at its limit) large copies still work, in
+    the calling thread, and no exception reaches the C entry."""
+    run(stub, """
+        from vespa_jl_amd._lib import DeviceBuffer
+        S.stub_no_threads(1)
+        a = DeviceBuffer(9 * MIB + 5)
+        h = np.random.default_rng(1).integers(0, 256, 9 * MIB + 5, dtype=np.uint8)
+        o = np.zeros_like(h)
+        a.upload(h).download(o)
+        assert np.array_equal(h, o)
+        """)

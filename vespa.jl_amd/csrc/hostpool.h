@@ -9,6 +9,7 @@
 #include <cstdlib>
 #include <functional>
 #include <mutex>
+#include <system_error>
 #include <thread>
 
 namespace vh {
@@ -17,7 +18,8 @@ namespace vh {
 // on the pool's workers and the caller, returning when all are done. Created on
 // first use with min(hardware threads, 16) threads (VESPAHIP_HOST_THREADS
 // overrides, 1 = serial); a child process after fork() builds its own (it
-// inherits no worker threads). The pool is never destroyed: its workers sleep
+// inherits no worker threads). Where the system gives fewer threads the pool has
+// fewer, down to the caller alone. The pool is never destroyed: its workers sleep
 // until the process ends.
 class HostPool {
  public:
@@ -53,8 +55,10 @@ class HostPool {
   static void pause() { __builtin_ia32_pause(); }
 
   explicit HostPool(int workers) : pid_(getpid()) {
-    for (int i = 0; i < workers; ++i) std::thread([this] { loop(); }).detach();
-    nworkers_ = workers;
+    try {
+      for (; nworkers_ < workers; ++nworkers_) std::thread([this] { loop(); }).detach();
+    } catch (const std::system_error&) {
+    }
   }
   void loop() {
     long long seen = 0;

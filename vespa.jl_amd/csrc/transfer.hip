@@ -15,6 +15,7 @@
 #include <condition_variable>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <vector>
 
 #include "host.h"
@@ -42,6 +43,13 @@ class SlotPool {
  public:
   std::vector<Slot> take(int want, int device) {
     std::vector<Slot> got;
+    try {
+      got.reserve(want);
+      std::lock_guard<std::mutex> lk(mu_);
+      free_.reserve(kSlots);
+    } catch (const std::bad_alloc&) {
+      return {};
+    }
     std::unique_lock<std::mutex> lk(mu_);
     for (;;) {
       while ((int)got.size() < want && !free_.empty()) {
@@ -89,10 +97,14 @@ SlotPool& slot_pool() {
 }
 
 void copy_pieces(char* dst, const char* src, size_t n) {
-  HostPool::run((int)((n + kPiece - 1) / kPiece), [&](int i) {
-    const size_t o = (size_t)i * kPiece;
-    memcpy(dst + o, src + o, std::min(kPiece, n - o));
-  });
+  try {
+    HostPool::run((int)((n + kPiece - 1) / kPiece), [&](int i) {
+      const size_t o = (size_t)i * kPiece;
+      memcpy(dst + o, src + o, std::min(kPiece, n - o));
+    });
+  } catch (const std::exception&) {   // the pool could not take the job (out of memory)
+    memcpy(dst, src, n);
+  }
 }
 
 // Ordinary host memory: what the runtime knows nothing of. Pinned, managed and device memory
