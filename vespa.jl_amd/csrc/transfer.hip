@@ -2,13 +2,14 @@
 //
 // The runtime moves pageable memory through its own staging with one thread; a fresh host
 // array also takes its page faults in that thread. Here the copy is cut into chunks that
-// pass through pinned slots, the DMA of one chunk running while the pool's threads copy
-// others between the slots and the caller's array.
+// pass through pinned slots, one chunk crossing the link (up by the runtime, down by
+// store_kernel) while the pool's threads copy others between the slots and the caller's array.
 //
 // Bound: the link (57 GB/s each way from pinned memory) and the threads' page faults. Measured,
-// runtime and here (GB/s): down 2 MiB 17.7 and 26.6, 16 MiB 16.9 and 34, 195 MiB 17.5 and 39.4; down
-// into a fresh array of 195 MiB 10.4 and 17.7; up 2 MiB 25.9 and 31.6, 64 MiB 29.5 and 38.5. Below 4 MiB
-// what is gained goes into waking the threads: a lone 0.6 MiB download took 50 µs and 130.
+// runtime and here (GB/s): down 5 MiB 17.6 and 40, 20 MiB 17.6 and 43, 200 MiB 17.7 and 48.6; down
+// into a fresh array of 200 MiB 10.7 and 16.7; up 8 MiB 34.6 and 36.3, 64 MiB 30.8 and 38.9. Copies of up
+// to 4 MiB stay with the runtime: what is gained goes into waking the threads there (a lone
+// 0.6 MiB download took 50 µs and 130).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -28,6 +29,7 @@ constexpr size_t kChunk = (size_t)2 << 20;   // bytes per slot
 constexpr size_t kPiece = (size_t)128 << 10; // bytes per thread at a time
 constexpr int kSlots = 16;                   // pinned slots of the process (32 MiB)
 constexpr int kSlotsPerCopy = 4;
+constexpr int kStoreWgs = 32;                // workgroups of store_kernel
 // Copies of at most this many bytes go to the runtime.
 constexpr size_t kDirect = (size_t)4 << 20;
 
@@ -118,7 +120,33 @@ bool is_pageable(const void* p) {
   return a.type == hipMemoryTypeUnregistered;
 }
 
-hipError_t staged(char* dst, const char* src, size_t bytes, bool up, hipStream_t s, const std::vector<Slot>& slots) {
+// n bytes to a pinned slot (16-byte aligned), 16 bytes per lane and pass. A kernel and not the
+// runtime's copy, since that runs on an engine which the driver also clears freed device memory
+// with: for some ms after a large free (a rollout's 860 MB) its downloads took 942 µs per 10 MiB against
+// 266 at rest, the kernel's 234 and 232. Bound: the link, reached with 16 workgroups or more.
+typedef unsigned U4 __attribute__((ext_vector_type(4)));
+__global__ void __launch_bounds__(256) store_kernel(const char* __restrict__ src, char* __restrict__ dst, size_t n) {
+  const size_t nv = n / 16, lane = (size_t)blockIdx.x * 256 + threadIdx.x;
+  for (size_t i = lane; i < nv; i += (size_t)gridDim.x * 256)
+    __builtin_nontemporal_store(__builtin_nontemporal_load((const U4*)src + i), (U4*)dst + i);
+  if (lane < n % 16) dst[nv * 16 + lane] = src[nv * 16 + lane];
+}
+
+// Whether store_kernel may read the bytes at src: an allocation of the device that holds them
+// all, 16-byte aligned. Everything else, errors included, is left to the runtime.
+bool kernel_reads(const char* src, size_t bytes, int device) {
+  hipPointerAttribute_t a{};
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if ((uintptr_t)src % 16 == 0 && hipPointerGetAttributes(&a, src) == hipSuccess && a.type == hipMemoryTypeDevice &&
+      a.device == device && hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)src) == hipSuccess)
+    return (size_t)(src - (const char*)base) + bytes <= size;
+  (void)hipGetLastError();
+  return false;
+}
+
+hipError_t staged(char* dst, const char* src, size_t bytes, bool up, hipStream_t s, int device,
+                  const std::vector<Slot>& slots) {
   const size_t n = (bytes + kChunk - 1) / kChunk, ns = slots.size();
   auto len = [&](size_t c) { return std::min(kChunk, bytes - c * kChunk); };
   hipError_t e = hipSuccess;
@@ -132,9 +160,18 @@ hipError_t staged(char* dst, const char* src, size_t bytes, bool up, hipStream_t
       if (e == hipSuccess) e = hipEventRecord(sl.ev, s);
     }
   } else {
+    const bool kernel = kernel_reads(src, bytes, device);
     auto issue = [&](size_t c) {
       const Slot& sl = slots[c % ns];
-      hipError_t r = hipMemcpyAsync(sl.mem, src + c * kChunk, len(c), hipMemcpyDeviceToHost, s);
+      hipError_t r = hipSuccess;
+      if (kernel) {
+        const char* from = src + c * kChunk;
+        size_t n_bytes = len(c);
+        void* args[] = {&from, (void*)&sl.mem, &n_bytes};
+        r = hipLaunchKernel((const void*)store_kernel, dim3(kStoreWgs), dim3(256), args, 0, s);
+      } else {
+        r = hipMemcpyAsync(sl.mem, src + c * kChunk, len(c), hipMemcpyDeviceToHost, s);
+      }
       return r == hipSuccess ? hipEventRecord(sl.ev, s) : r;
     };
     for (size_t c = 0; c < std::min(n, ns) && e == hipSuccess; ++c) e = issue(c);
@@ -161,7 +198,7 @@ hipError_t host_copy(void* dst, const void* src, size_t bytes, bool up, hipStrea
     std::vector<Slot> slots = slot_pool().take((int)std::min<size_t>(kSlotsPerCopy, chunks), device);
     bool usable = !slots.empty();
     for (const Slot& sl : slots) usable = usable && sl.device == device;
-    if (usable) e = staged((char*)dst, (const char*)src, bytes, up, s, slots);
+    if (usable) e = staged((char*)dst, (const char*)src, bytes, up, s, device, slots);
     slot_pool().give_back(slots);
     if (usable) return e;
   }
