@@ -75,3 +75,21 @@ def test_copies_without_threads(stub):
         assert L.vh_buffer_download(addr(o), a.ptr + 1, o.size) == 0   # odd source: no kernel
         assert np.array_equal(h[1:], o)
         """)
+
+
+def test_small_host_batches_wait_once(stub):
+    """The flux backend queues its three uploads, the kernel and the download, and waits
+    for the last only; a small copy without a stream is the runtime's synchronous one."""
+    run(stub, """
+        from vespa_jl_amd._lib import DeviceBuffer
+        WL = np.ones((100, 5)); F = np.empty_like(WL); ax = np.ones(100, np.int32)
+        V.compute_face_fluxes(V.HIPFlux(), V.IdealHydro(1.4), F, WL, WL, ax)
+        S.stub_clear()
+        V.compute_face_fluxes(V.HIPFlux(), V.IdealHydro(1.4), F, WL, WL, ax)
+        assert [l[0] for l in log()] == ["copy", "copy", "copy", "launch", "copy", "sync"]
+        a = DeviceBuffer(800).upload(WL[:20])
+        S.stub_clear()
+        a.download(F[:20])
+        a.upload(F[:20])
+        assert [l[0] for l in log()] == ["copy", "copy"]
+        """)

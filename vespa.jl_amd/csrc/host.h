@@ -63,6 +63,8 @@ inline int cu_count(int device) {
 // complete on return (transfer.hip).
 hipError_t copy_up(void* dev, const void* host, size_t bytes, hipStream_t s);
 hipError_t copy_down(void* host, const void* dev, size_t bytes, hipStream_t s);
+// copy_up that may still be under way on return: host stays as it is until s is waited for.
+hipError_t enqueue_up(void* dev, const void* host, size_t bytes, hipStream_t s);
 
 // Clock kernels of the uniform-grid context, shared with the block context.
 // clock (kClockDoubles): [0] t, [1] dt, [2] max CFL term, [3] steps; of a step loop also

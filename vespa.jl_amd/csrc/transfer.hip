@@ -186,29 +186,39 @@ hipError_t staged(char* dst, const char* src, size_t bytes, bool up, hipStream_t
   return e == hipSuccess ? es : e;
 }
 
-hipError_t host_copy(void* dst, const void* src, size_t bytes, bool up, hipStream_t s) {
-  if (bytes == 0) return hipStreamSynchronize(s);
+// The copy through the slots, complete on return; false where it is left to the runtime.
+bool through_slots(void* dst, const void* src, size_t bytes, bool up, hipStream_t s, hipError_t* e) {
   int device = 0, stream_device = 0;
-  hipError_t e = hipGetDevice(&device);
-  if (e != hipSuccess) return e;
+  if (bytes <= kDirect || HostPool::threads() <= 1 || hipGetDevice(&device) != hipSuccess) return false;
   // the slots' events are the current device's: a stream of another takes the plain copy
   if (!s || hipStreamGetDevice(s, &stream_device) != hipSuccess) stream_device = device;
-  if (bytes > kDirect && HostPool::threads() > 1 && stream_device == device && is_pageable(up ? src : dst)) {
-    const size_t chunks = (bytes + kChunk - 1) / kChunk;
-    std::vector<Slot> slots = slot_pool().take((int)std::min<size_t>(kSlotsPerCopy, chunks), device);
-    bool usable = !slots.empty();
-    for (const Slot& sl : slots) usable = usable && sl.device == device;
-    if (usable) e = staged((char*)dst, (const char*)src, bytes, up, s, device, slots);
-    slot_pool().give_back(slots);
-    if (usable) return e;
-  }
-  e = hipMemcpyAsync(dst, src, bytes, up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, s);
+  if (stream_device != device || !is_pageable(up ? src : dst)) return false;
+  const size_t chunks = (bytes + kChunk - 1) / kChunk;
+  std::vector<Slot> slots = slot_pool().take((int)std::min<size_t>(kSlotsPerCopy, chunks), device);
+  bool usable = !slots.empty();
+  for (const Slot& sl : slots) usable = usable && sl.device == device;
+  if (usable) *e = staged((char*)dst, (const char*)src, bytes, up, s, device, slots);
+  slot_pool().give_back(slots);
+  return usable;
+}
+
+hipError_t host_copy(void* dst, const void* src, size_t bytes, bool up, hipStream_t s) {
+  if (bytes == 0) return hipStreamSynchronize(s);
+  hipError_t e = hipSuccess;
+  if (through_slots(dst, src, bytes, up, s, &e)) return e;
+  const hipMemcpyKind kind = up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
+  if (!s) return hipMemcpy(dst, src, bytes, kind);   // 1 KiB down 13 µs; queued and waited for, 22
+  e = hipMemcpyAsync(dst, src, bytes, kind, s);
   const hipError_t es = hipStreamSynchronize(s);
   return e == hipSuccess ? es : e;
 }
 
 }  // namespace
 
+hipError_t enqueue_up(void* dev, const void* host, size_t bytes, hipStream_t s) {
+  hipError_t e = hipSuccess;
+  return through_slots(dev, host, bytes, true, s, &e) ? e : hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
+}
 hipError_t copy_up(void* dev, const void* host, size_t bytes, hipStream_t s) { return host_copy(dev, host, bytes, true, s); }
 hipError_t copy_down(void* host, const void* dev, size_t bytes, hipStream_t s) {
   return host_copy(host, dev, bytes, false, s);

@@ -413,9 +413,9 @@ static int face_flux_host(const T* WL, const T* WR, const int32_t* ax, int64_t n
   T* dF = (T*)(base + 2 * nv_al);
   int32_t* dax = (int32_t*)(base + 3 * nv_al);
   hipStream_t s = g_stage.stream;
-  VH_HIP(copy_up(dWL, WL, nv, s));
-  VH_HIP(copy_up(dWR, WR, nv, s));
-  VH_HIP(copy_up(dax, ax, (size_t)nf * sizeof(int32_t), s));
+  VH_HIP(enqueue_up(dWL, WL, nv, s));
+  VH_HIP(enqueue_up(dWR, WR, nv, s));
+  VH_HIP(enqueue_up(dax, ax, (size_t)nf * sizeof(int32_t), s));
   exact::launch_face_flux(sizeof(T) == 8 ? 0 : 1, nf, s, dWL, dWR, dax, gamma, dF);
   VH_HIP(hipGetLastError());
   VH_HIP(copy_down(F, dF, nv, s));
