@@ -93,3 +93,57 @@ def test_small_host_batches_wait_once(stub):
         a.upload(F[:20])
         assert [l[0] for l in log()] == ["copy", "copy"]
         """)
+
+
+LOOP = """
+        clk = (C.c_double * 8).from_address(S.stub_pinned(64))
+        looks = []
+        @C.CFUNCTYPE(None, C.c_char_p)
+        def on_sync(kind):
+            if kind == b"event" and not looks:   # the loop's first reduction: dt = cfl
+                clk[2] = 1.0
+            elif kind == b"stream":              # the clock after what was queued
+                looks.append(steps() - sum(looks))
+                clk[0], clk[1], clk[3], clk[5] = t0 + 0.3 * sum(looks), 0.3, sum(looks), tfinal
+                if not clk[0] < tfinal * (1 - 1e-12): clk[7] = 1.0
+        S.stub_on_sync(on_sync)
+"""
+
+
+@pytest.mark.parametrize("legs,queued", [(1, [1]), (2, [2]), (3, [3]), (8, [8]), (12, [8, 4])])
+def test_steps_queued_for_a_leg(stub, legs, queued):
+    """A loop with a final time queues one step, learns dt from the first reduction
+    and queues what the leg holds (at most 8 before the first look at the clock): a leg of
+    one step is one step, not eight of which seven do nothing."""
+    run(stub, f"""
+        prob = V.Problem("l", (24, 20), ((0.0, 1.0),) * 2, 1.4, "periodic", lambda x, y, z: (1.0, 0.0, 0.0, 0.0, 1.0), 1.0, 0.3)
+        sim = V.Simulation(V.UniformMesh((24, 20), prob.domain), prob)
+        t0, tfinal = 0.0, {legs} * 0.3 - 0.1
+        prob.tfinal = tfinal
+        def steps(): return (len([l for l in log() if l[0] == "launch"]) - 2) // 3   # cfl and begin, then 3 per step
+        S.stub_clear()
+        {LOOP}
+        V.evolve(sim)
+        assert looks == {queued}, looks
+        """)
+
+
+@pytest.mark.parametrize("legs,queued", [(1, [1]), (2, [2]), (8, [8]), (12, [8, 4])])
+def test_block_steps_queued_for_a_leg(stub, legs, queued):
+    run(stub, f"""
+        from vespa_jl_amd import blockmesh as BM
+        m = BM.BlockMesh(2, 0, (1.0 / 8, 1.0 / 8), 1.4, [0], [[8, 8, 1]], [[0, 0, 0]], [[0] * 4 + [1, 1]])
+        s = BM.BlockSimulation(m, np.float64, cfl=0.3)
+        s.set_launch(use_graph=False)
+        t0, tfinal = 0.0, {legs} * 0.3 - 0.1
+        per = None
+        def launches(): return len([l for l in log() if l[0] == "launch"])
+        S.stub_clear()
+        s.step(0.1)
+        per = launches()   # the dt, then a step's launches; in a loop a tail follows them
+        def steps(): return (launches() - 2) // per
+        S.stub_clear()
+        {LOOP}
+        s.evolve(tfinal)
+        assert looks == {queued}, looks
+        """)

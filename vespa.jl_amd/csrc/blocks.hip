@@ -1058,6 +1058,7 @@ struct vh_blocks {
   int npartials = 0;
   double* clock = nullptr;
   double* clock_host = nullptr;   // pinned copy of the clock, written by its kernels
+  hipEvent_t look = nullptr;      // recorded behind the first reduction of a step loop
   bool in_loop = false;           // kernels of a step loop look at its end flag
   hipStream_t stream = nullptr;
   // Side streams of a stage's launches, one per shape class beyond the first, with the
@@ -1757,8 +1758,9 @@ int vh_blocks_create(vh_blocks** out, int32_t rank, int32_t nblocks, int32_t max
   int ncu = 0;
   if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, m->device) == hipSuccess && ncu > 0)
     m->ncu = ncu;
-  if (hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess) {
-    delete m;
+  if (hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess ||
+      hipEventCreateWithFlags(&m->look, hipEventDisableTiming) != hipSuccess) {
+    vh_blocks_destroy(m);
     return fail(-2, "stream creation failed%s", "");
   }
   const long long n = m->T.off[m->T.nb];
@@ -1793,6 +1795,7 @@ int vh_blocks_destroy(vh_blocks* m) {
   (void)hipFree(m->partials);
   (void)hipFree(m->clock);
   if (m->clock_host) (void)hipHostFree(m->clock_host);
+  if (m->look) (void)hipEventDestroy(m->look);
   for (int i = 0; i < kBlockClasses - 1; ++i) {
     if (m->side[i]) (void)hipStreamDestroy(m->side[i]);
     if (m->ev_join[i]) (void)hipEventDestroy(m->ev_join[i]);
@@ -1856,6 +1859,10 @@ int vh_blocks_run(vh_blocks* m, double cfl, double tfinal, int64_t max_steps, in
   int64_t k = 0;
   double t = *t_io;
   int rc = 0;
+  if (clip && !(t < tfinal * (1 - 1e-12))) {   // nothing to do; the clock's copy stays unwritten
+    if (steps) *steps = 0;
+    return 0;
+  }
   if (subcycle) {
     // evolve! with subcycling (src/driver.jl:581-605): root dt from level 0;
     // with self-gravity one Poisson solve per root step, g held over every
@@ -1877,16 +1884,13 @@ int vh_blocks_run(vh_blocks* m, double cfl, double tfinal, int64_t max_steps, in
     }
     VH_HIP(hipStreamSynchronize(m->stream));
   } else {
-    enqueue_cfl(m, -1);
-    enqueue_loop_begin(m->stream, m->partials, kCflWgs, t, cfl, tfinal, clip, m->clock);
-    const int64_t limit = max_steps > 0 ? max_steps : INT64_MAX;
-    int64_t queued = 0;
     double* clk = m->clock_host;
     clk[0] = t;
     clk[3] = 0.0;
-    clk[7] = clip && !(t < tfinal * (1 - 1e-12)) ? 1.0 : 0.0;
-    while (queued < limit && clk[7] == 0.0) {
-      int64_t n = loop_chunk(clip, limit - queued, queued ? clk : nullptr);
+    clk[7] = 0.0;
+    enqueue_cfl(m, -1);
+    enqueue_loop_begin(m->stream, m->partials, kCflWgs, t, cfl, tfinal, clip, m->clock, clk);
+    auto queue = [&](int64_t n) -> int {
       const int saved = m->use_graph;
       if (m->grav) {
         // solve_poisson! before each step (src/driver.jl:498), g held over the step;
@@ -1894,17 +1898,18 @@ int vh_blocks_run(vh_blocks* m, double cfl, double tfinal, int64_t max_steps, in
         long long it = 0;
         double rr = 0.0;
         m->grav->B.rho = m->U;
-        if ((rc = grav_csr_solve(m->stream, m->dtype, m->grav->A, m->grav->P, m->grav->B, &it, &rr))) return rc;
+        if (int rs = grav_csr_solve(m->stream, m->dtype, m->grav->A, m->grav->P, m->grav->B, &it, &rr)) return rs;
         enqueue_grav_accel(m);
         m->use_graph = 0;
-        n = 1;
       }
-      for (int64_t i = 0; i < n && !rc; ++i) rc = single_rate_step(m);
+      int rs = 0;
+      for (int64_t i = 0; i < n && !rs; ++i) rs = single_rate_step(m);
       m->use_graph = saved;
-      if (rc) return rc;
-      queued += n;
-      if (clip || queued >= limit) VH_HIP(hipStreamSynchronize(m->stream));
-    }
+      return rs;
+    };
+    if ((rc = run_step_loop(m->stream, m->look, clk, t, cfl, tfinal, clip, max_steps > 0 ? max_steps : INT64_MAX,
+                            m->grav != nullptr, queue)))
+      return rc;
     t = clk[0];
     k = (int64_t)clk[3];
   }
@@ -2293,7 +2298,7 @@ int vh_blocks_time_steps(vh_blocks* m, double cfl, int64_t nsteps, int32_t metho
   };
   // two untimed steps (the first builds the graph when graphs are used)
   enqueue_cfl(m, -1);
-  enqueue_loop_begin(m->stream, m->partials, kCflWgs, 0.0, cfl, 0.0, false, m->clock);
+  enqueue_loop_begin(m->stream, m->partials, kCflWgs, 0.0, cfl, 0.0, false, m->clock, nullptr);
   int rc = one_step();
   if (!rc) rc = one_step();
   hipEvent_t e0 = nullptr, e1 = nullptr;

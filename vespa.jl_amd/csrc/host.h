@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+
 #include "common.h"
 
 namespace vh {
@@ -77,13 +79,43 @@ void enqueue_set_dt(hipStream_t s, double* clock, double dt);
 // tail after each step's stage 2 advances the clock and sets the next dt from the
 // partials of the new state (and stores it to *dt_log unless null).
 void enqueue_loop_begin(hipStream_t s, const double* partials, int np, double t, double cfl, double tfinal, bool clip,
-                        double* clock, double* dt_log = nullptr);
+                        double* clock, double* host, double* dt_log = nullptr);
 void enqueue_step_tail(hipStream_t s, const double* partials, int np, double* clock, double* host,
                        double* dt_log = nullptr);
-// Steps to queue before the host looks at the clock again: all that are left without
-// a final time; with one, 8 before the first look (clk null) and then as many as the
-// remaining time holds at the current dt, at most 64. Steps queued beyond the end do nothing.
-long long loop_chunk(bool clip, long long left, const double* clk);
+// Steps of dt until time_left has passed: 1 to most (1 also for a NaN).
+long long steps_within(double time_left, double dt, long long most);
+
+// The host side of a step loop on s: queue(n) queues n steps with their tails, clk is the clock's
+// pinned copy. Without a final time (clip false) all steps are queued at once. With one, the host
+// looks at the clock before it queues more than the remaining time holds at the current dt, at
+// most 64 steps; steps queued beyond the end do nothing, but their launches take time
+// (eight queued for a leg of one step made it 100 µs where a look per step took 64, at
+// 64²). So one step is queued first, which is always taken, and the host waits for
+// begin's reduction while it runs (`look` is recorded behind begin), and reads the largest CFL
+// term alone: the rest of the clock may be on its way from that step's tail. one_by_one:
+// queue() needs the step before it to have ended.
+template <typename Queue>
+int run_step_loop(hipStream_t s, hipEvent_t look, const volatile double* clk, double t, double cfl, double tfinal,
+                  bool clip, long long limit, bool one_by_one, Queue queue) {
+  if (clip && !one_by_one && limit > 1) VH_HIP(hipEventRecord(look, s));
+  for (long long queued = 0; queued < limit && clk[7] == 0.0;) {
+    const bool first = queued == 0;
+    long long n = limit - queued;
+    if (one_by_one || (clip && first)) n = 1;
+    else if (clip) n = steps_within(clk[5] - clk[0], clk[1], n < 64 ? n : 64);
+    if (int rc = queue(n)) return rc;
+    queued += n;
+    if (clip && first && !one_by_one && queued < limit) {
+      VH_HIP(hipEventSynchronize(look));
+      const double m = clk[2];
+      n = steps_within(tfinal - t, m == 0.0 ? HUGE_VAL : cfl / m, limit < 8 ? limit : 8) - 1;
+      if (int rc = n > 0 ? queue(n) : 0) return rc;
+      queued += n;
+    }
+    if (clip || queued >= limit) VH_HIP(hipStreamSynchronize(s));
+  }
+  return 0;
+}
 
 }  // namespace vh
 

@@ -78,7 +78,7 @@ __global__ void __launch_bounds__(kClockLanes) dt_finalize_kernel(const double* 
 
 __global__ void __launch_bounds__(kClockLanes) loop_begin_kernel(const double* __restrict__ partials, int np, double t,
                                                                  double cfl, double tfinal, double tstop, double* clock,
-                                                                 double* dt_log) {
+                                                                 double* host, double* dt_log) {
   __shared__ double red[kClockLanes / 64];
   const double m = partials_max(partials, np, red);
   if (threadIdx.x == 0) {
@@ -89,6 +89,7 @@ __global__ void __launch_bounds__(kClockLanes) loop_begin_kernel(const double* _
     clock[6] = tstop;
     clock[7] = 0.0;
     clock_next(clock, m, dt_log);
+    clock_to_host(clock, host);
   }
 }
 
@@ -144,21 +145,16 @@ void enqueue_set_dt(hipStream_t s, double* clock, double dt) {
   hipLaunchKernelGGL(set_dt_kernel, dim3(1), dim3(1), 0, s, clock, dt);
 }
 void enqueue_loop_begin(hipStream_t s, const double* partials, int np, double t, double cfl, double tfinal, bool clip,
-                        double* clock, double* dt_log) {
+                        double* clock, double* host, double* dt_log) {
   hipLaunchKernelGGL(loop_begin_kernel, dim3(1), dim3(kClockLanes), 0, s, partials, np, t, cfl,
-                     clip ? tfinal : 0.0, tfinal * (1 - 1e-12), clock, dt_log);
+                     clip ? tfinal : 0.0, tfinal * (1 - 1e-12), clock, host, dt_log);
 }
 void enqueue_step_tail(hipStream_t s, const double* partials, int np, double* clock, double* host, double* dt_log) {
   hipLaunchKernelGGL(step_tail_kernel, dim3(1), dim3(kClockLanes), 0, s, partials, np, clock, host, dt_log);
 }
-long long loop_chunk(bool clip, long long left, const double* clk) {
-  if (!clip) return left;
-  double n = 8.0;
-  if (clk) {
-    n = std::ceil((clk[5] - clk[0]) / clk[1]);
-    n = n >= 1.0 ? std::min(n, 64.0) : 1.0;   // also for a NaN
-  }
-  return std::min<long long>(left, (long long)n);
+long long steps_within(double time_left, double dt, long long most) {
+  const double n = std::ceil(time_left / dt);
+  return n >= 1.0 ? (long long)std::min(n, (double)most) : 1;
 }
 
 }  // namespace vh
@@ -187,6 +183,7 @@ struct vh_grid {
   int npartials;
   double* clock;
   double* clock_host;    // pinned copy of the clock, written by its kernels
+  hipEvent_t look;       // recorded behind the first reduction of a step loop
   double* totals_partials;
   hipStream_t stream;
   struct AdjWork* adj;   // reverse-mode work buffers (allocated on first use)
@@ -604,7 +601,8 @@ int vh_grid_create(vh_grid** out, int32_t rank, const int64_t* dims, const doubl
     vh_grid_destroy(g);
     return fail(-2, "device allocation of %s%lld bytes failed", "", (long long)(2 * bytes));
   }
-  if (hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking) != hipSuccess) {
+  if (hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking) != hipSuccess ||
+      hipEventCreateWithFlags(&g->look, hipEventDisableTiming) != hipSuccess) {
     vh_grid_destroy(g);
     return fail(-2, "stream creation failed%s", "");
   }
@@ -629,6 +627,7 @@ int vh_grid_destroy(vh_grid* g) {
   if (g->partials) (void)hipFree(g->partials);
   if (g->clock) (void)hipFree(g->clock);
   if (g->clock_host) (void)hipHostFree(g->clock_host);
+  if (g->look) (void)hipEventDestroy(g->look);
   if (g->totals_partials) (void)hipFree(g->totals_partials);
   if (g->pg) (void)hipFree(g->pg);
   if (g->stream) (void)hipStreamDestroy(g->stream);
@@ -758,35 +757,37 @@ int vh_grid_run(vh_grid* g, double cfl, double tfinal, int64_t max_steps, double
   if (!clip && max_steps <= 0) return fail(-1, "need tfinal > 0 or max_steps > 0%s", "");
   if (int rc = need_parent_states(g)) return rc;
   VH_HIP(hipSetDevice(g->device));
+  if (clip && !(*t_io < tfinal * (1 - 1e-12))) {   // nothing to do; the clock's copy stays unwritten
+    if (steps) *steps = 0;
+    return 0;
+  }
   if (line_fits(g)) return run_line(g, cfl, tfinal, max_steps, t_io, steps);
-  enqueue_cfl(g);   // CFL partials of the current state
-  enqueue_loop_begin(g->stream, g->partials, g->cfl_blocks, *t_io, cfl, tfinal, clip, g->clock);
-  const int64_t limit = max_steps > 0 ? max_steps : INT64_MAX;
-  int64_t queued = 0;
   double* clk = g->clock_host;
   clk[0] = *t_io;
   clk[3] = 0.0;
-  clk[7] = clip && !(*t_io < tfinal * (1 - 1e-12)) ? 1.0 : 0.0;
-  while (queued < limit && clk[7] == 0.0) {
-    int64_t n = loop_chunk(clip, limit - queued, queued ? clk : nullptr);
+  clk[7] = 0.0;
+  enqueue_cfl(g);   // CFL partials of the current state
+  enqueue_loop_begin(g->stream, g->partials, g->cfl_blocks, *t_io, cfl, tfinal, clip, g->clock, clk);
+  auto queue = [&](int64_t n) -> int {
     if (g->grav) {   // φ(ρⁿ), held over the step (src/driver.jl:498)
       long long it;
       double rr;
       g->grav->B.rho = g->U;
       int rc = grav_solve(g->stream, g->dtype == VH_F64 ? 0 : 1, g->G, g->grav->P, g->grav->B, &it, &rr);
       if (rc) return rc;
-      n = 1;
     }
     g->G.stop = g->clock + 7;
     for (int64_t i = 0; i < n; ++i) {
       enqueue_step(g);
-      enqueue_step_tail(g->stream, g->partials, g->stage_blocks, g->clock, g->clock_host);
+      enqueue_step_tail(g->stream, g->partials, g->stage_blocks, g->clock, clk);
     }
     g->G.stop = nullptr;
-    queued += n;
     VH_HIP(hipGetLastError());
-    if (clip || queued >= limit) VH_HIP(hipStreamSynchronize(g->stream));
-  }
+    return 0;
+  };
+  if (int rc = run_step_loop(g->stream, g->look, clk, *t_io, cfl, tfinal, clip, max_steps > 0 ? max_steps : INT64_MAX,
+                             g->grav != nullptr, queue))
+    return rc;
   *t_io = clk[0];
   if (steps) *steps = (int64_t)clk[3];
   return 0;
@@ -970,7 +971,7 @@ int vh_grid_time_steps(vh_grid* g, double cfl, int64_t nsteps, double* ms_stage1
     if (hipEventCreate(&ev[i]) != hipSuccess) rc = fail(-2, "hipEventCreate failed%s", "");
   if (!rc) {
     enqueue_cfl(g);
-    enqueue_loop_begin(g->stream, g->partials, g->cfl_blocks, 0.0, cfl, 0.0, false, g->clock);
+    enqueue_loop_begin(g->stream, g->partials, g->cfl_blocks, 0.0, cfl, 0.0, false, g->clock, nullptr);
     for (int64_t k = 0; k < nsteps; ++k) {
       enqueue_step(g, ev[3 * k], ev[3 * k + 1], ev[3 * k + 2]);
       enqueue_step_tail(g->stream, g->partials, g->stage_blocks, g->clock, nullptr);
@@ -1221,7 +1222,7 @@ int vh_adjoint_forward(vh_adjoint* a, double cfl) {
   VH_HIP(hipEventRecord(e0, g->stream));
   VH_HIP(hipMemcpyAsync(a->ckpt, g->U, nb, hipMemcpyDeviceToDevice, g->stream));
   enqueue_cfl(g);
-  enqueue_loop_begin(g->stream, g->partials, g->cfl_blocks, 0.0, cfl, 0.0, false, g->clock, a->dts);
+  enqueue_loop_begin(g->stream, g->partials, g->cfl_blocks, 0.0, cfl, 0.0, false, g->clock, nullptr, a->dts);
   // The last segment's states are kept as the forward run produces them (the
   // backward pass starts there and needs no recompute for it).
   const size_t n5 = 5 * (size_t)g->G.ncell;
