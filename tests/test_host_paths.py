@@ -147,3 +147,45 @@ def test_block_steps_queued_for_a_leg(stub, legs, queued):
         s.evolve(tfinal)
         assert looks == {queued}, looks
         """)
+
+
+@pytest.mark.parametrize("call", ["hipStreamCreateWithFlags", "hipEventCreateWithFlags", "hipEventRecord",
+                                  "hipStreamWaitEvent"])
+def test_block_stages_stay_ordered_when_a_fork_or_join_fails(stub, call):
+    """The shape classes of a stage run side by side on forked streams. Whatever call of the
+    fork or the join fails, every launch of a stage still follows all of the one before it
+    (the happens-before order of the log), and the context's stream ends behind them all."""
+    run(stub, f"""
+        from vespa_jl_amd import blockmesh as BM
+        m = BM.random_block_pairs(12, seed=3, rank=3)
+        def known(ops):
+            hb, ev, host, seen, n = {{}}, {{}}, set(), [], 0
+            for o in ops:
+                h = hb.setdefault(o[1], set()) if o[0] != "event" else None
+                if o[0] == "launch":
+                    h |= host
+                    seen.append((o[1], set(h)))
+                    h.add(len(seen) - 1)
+                elif o[0] == "record": ev[o[2]] = set(h)
+                elif o[0] == "wait": h |= ev.get(o[2], set())
+                elif o[0] == "sync": host |= h
+            return seen, hb, host
+        most = 0
+        for fail_at in [-1] + list(range(16)):
+            s = BM.BlockSimulation(m, np.float64, cfl=0.3)
+            S.stub_clear()
+            S.stub_fail({call!r}.encode(), fail_at)
+            s.step(0.1)
+            S.stub_fail(b"", -1)
+            seen, hb, host = known([l for l in log() if l[0] in ("launch", "record", "wait", "sync")])
+            k = (len(seen) - 3) // 2   # the dt, then twice: link fluxes and k classes
+            assert k >= 3 and len(seen) == 2 * k + 3
+            stage = [0, 1] + [2] * k + [3] + [4] * k
+            most = max(most, len(set(st for st, _ in seen)))
+            for i, (_, h) in enumerate(seen):
+                missing = [j for j in range(i) if stage[j] != stage[i] and j not in h]
+                assert not missing, ({call!r}, fail_at, i, missing)
+            assert hb[seen[0][0]] | host == set(range(len(seen))), ({call!r}, fail_at)
+            s.close()
+        assert most >= 3   # without a failure they do run side by side
+        """)

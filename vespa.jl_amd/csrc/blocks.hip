@@ -1162,9 +1162,9 @@ static void enqueue_link(vh_blocks* m, const void* Us) {
 
 static int ensure_side_streams(vh_blocks* m) {
   if (m->ev_fork) return 0;
-  for (int i = 0; i < kBlockClasses - 1; ++i) {
-    VH_HIP(hipStreamCreateWithFlags(&m->side[i], hipStreamNonBlocking));
-    VH_HIP(hipEventCreateWithFlags(&m->ev_join[i], hipEventDisableTiming));
+  for (int i = 0; i < kBlockClasses - 1; ++i) {   // what an earlier call made is kept
+    if (!m->side[i]) VH_HIP(hipStreamCreateWithFlags(&m->side[i], hipStreamNonBlocking));
+    if (!m->ev_join[i]) VH_HIP(hipEventCreateWithFlags(&m->ev_join[i], hipEventDisableTiming));
   }
   VH_HIP(hipEventCreateWithFlags(&m->ev_fork, hipEventDisableTiming));
   return 0;
@@ -1177,22 +1177,32 @@ static int ensure_side_streams(vh_blocks* m) {
 // in sequence and side by side: 400 blocks f64 0.87 and 0.65 ms, 3000 blocks f64 4.97 and
 // 4.36, f32 3.22 and 2.65. One kernel holding every shape was slower (5.41 ms for 3000 blocks:
 // the shapes share one register budget and spill twice as much).
+// A class that cannot be forked runs on the context's stream, and the host waits for one
+// that cannot be joined to it: no failure leaves launches unordered.
 static void enqueue_tiles(vh_blocks* m, bool stage2, int l, const void* Us, const void* U0, void* Uout) {
   const double* dtp = m->clock + 1;
   const int* co = m->H.tile_class_off.data() + (size_t)l * (kBlockClasses + 1);
   int np = 0, launches = 0;
   for (int c = 0; c < kBlockClasses; ++c) launches += class_wgs(m, l, c) > 0;
-  const bool fork = launches > 1 && ensure_side_streams(m) == 0;
-  if (fork) (void)hipEventRecord(m->ev_fork, m->stream);
+  bool failed = false;
+  auto ok = [&](hipError_t e) {
+    failed |= e != hipSuccess;
+    return e == hipSuccess;
+  };
+  bool fork = launches > 1;
+  if (fork && ensure_side_streams(m)) {
+    fork = false;
+    failed = true;
+  }
+  if (fork) fork = ok(hipEventRecord(m->ev_fork, m->stream));
   int used = 0;
+  bool joinable[kBlockClasses] = {};
   for (int c = 0, i = 0; c < kBlockClasses; ++c) {
     const int wgs = class_wgs(m, l, c);
     if (wgs == 0) continue;
     hipStream_t s = m->stream;
-    if (fork && i > 0) {
-      s = m->side[used];
-      (void)hipStreamWaitEvent(s, m->ev_fork, 0);
-    }
+    const bool aside = fork && i > 0 && ok(hipStreamWaitEvent(m->side[used], m->ev_fork, 0));
+    if (aside) s = m->side[used];
     BlocksDev B = blocks_dev(m);
     B.tiles = m->d_tiles + m->H.tile_list_off[l] + co[c];
     B.ntiles = co[c + 1] - co[c];
@@ -1200,11 +1210,16 @@ static void enqueue_tiles(vh_blocks* m, bool stage2, int l, const void* Us, cons
       fast::launch_block_stage(m->dtype, m->T.rank, c, stage2, wgs, s, Us, U0, Uout, dtp, m->partials + np, B);
     else
       exact::launch_block_stage(m->dtype, m->T.rank, c, stage2, wgs, s, Us, U0, Uout, dtp, m->partials + np, B);
-    if (fork && i > 0) (void)hipEventRecord(m->ev_join[used++], s);
+    if (aside) {
+      joinable[used] = ok(hipEventRecord(m->ev_join[used], s));
+      ++used;
+    }
     np += wgs;
     ++i;
   }
-  for (int i = 0; i < used; ++i) (void)hipStreamWaitEvent(m->stream, m->ev_join[i], 0);
+  for (int i = 0; i < used; ++i)
+    if (!joinable[i] || !ok(hipStreamWaitEvent(m->stream, m->ev_join[i], 0))) (void)hipStreamSynchronize(m->side[i]);
+  if (failed) (void)hipGetLastError();   // dealt with
   if (l == 0 && stage2) m->stage_wgs = np;
 }
 
