@@ -343,9 +343,12 @@ int vh_blocks_run(vh_blocks* m, double cfl, double tfinal, int64_t max_steps, in
 /* conserved_totals(sim) (src/diagnostics.jl:16-31): sum of U*V in Float64. */
 int vh_blocks_totals(vh_blocks* m, double* out5);
 
-/* Launch shape: z planes per tile (0 = whole block), cap on the persistent
- * workgroups (0 = 3 per compute unit), and whether the single-rate step is
- * replayed from a captured HIP graph (1, the default) or enqueued eagerly. */
+/* Launch shape: z planes per tile (0 = whole block, -1 = the default: chosen from the
+ * number of tiles, anew for the mesh of each regrid and each tile width), cap on
+ * the workgroups of a stage launch (0 = none for the compiled tile shapes, whose workgroups take
+ * one tile each, and 3 per compute unit for the runtime shape, whose take several),
+ * and whether the single-rate step is replayed from a captured HIP graph (1, the
+ * default) or enqueued eagerly. */
 int vh_blocks_set_launch(vh_blocks* m, int32_t zchunk, int32_t max_workgroups, int32_t use_graph);
 /* Widest tile along x (4..32, default 32); tiles take min(nx, max_tile_x)
  * columns and as many rows as fit 256 lanes. */

@@ -43,6 +43,17 @@ def random_mesh(n=14, seed=3, rank=3, edges=(8, 16, 24)):
     return BM.random_block_pairs(n, seed=seed, rank=rank, edges=edges)
 
 
+def three_boxes():
+    """Three 32³ blocks far apart, the same refined into eight each, and the map of the
+    second mesh's blocks to the first's: few and many tiles of one state."""
+    box = [[0, 0, 0], [128, 0, 0], [0, 128, 0]]
+    fine = [[b[0] + 32 * (o & 1), b[1] + 32 * (o >> 1 & 1), b[2] + 32 * (o >> 2)] for b in box for o in range(8)]
+    kw = dict(rank=3, maxlevel=1, h0=(1.0 / 32,) * 3, gamma=1.4)
+    small = BM.BlockMesh(level=[0] * 3, dims=[[32] * 3] * 3, origin=box, bc=[[2] * 6] * 3, **kw)
+    large = BM.BlockMesh(level=[1] * 24, dims=[[32] * 3] * 24, origin=fine, bc=[[2] * 6] * 24, **kw)
+    return small, large, [i // 8 for i in range(24)]
+
+
 MESHES = {
     "2d_two_level": two_level_2d,
     "3d_two_level": two_level_3d,
@@ -205,6 +216,24 @@ def test_infinite_final_time_ends_the_loop(graph):
     s.upload(U)
     assert s.evolve(np.inf, max_steps=20) == (np.inf, 1)
     s.close()
+
+
+def test_regrid_chooses_the_planes_of_the_new_mesh():
+    """A regrid of a 3D mesh whose new default differs, eager as the refinement driver
+    runs it, then stepped: the state of a fresh context on the new mesh."""
+    small, large, src = three_boxes()
+    a = _sim(small, np.float64, use_graph=False)
+    a.upload(_state(small, np.float64))
+    a.evolve(max_steps=2)
+    a.regrid(large, src)
+    b = _sim(large, np.float64)
+    b.upload(a.state())
+    assert a.info()["zchunk"] == b.info()["zchunk"] == 2
+    for s in (a, b):
+        s.evolve(max_steps=2)
+    np.testing.assert_array_equal(a.state(), b.state())
+    a.close()
+    b.close()
 
 
 @pytest.mark.parametrize("nblocks,edges,most", [(3, (8, 16), 1), (12, (8, 16, 24, 32), 2), (40, (6, 16, 24), 6)])

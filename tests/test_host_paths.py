@@ -189,3 +189,31 @@ def test_block_stages_stay_ordered_when_a_fork_or_join_fails(stub, call):
             s.close()
         assert most >= 3   # without a failure they do run side by side
         """)
+
+
+def test_automatic_z_planes_follow_the_mesh(stub):
+    """The automatic number of planes per tile stays automatic when only graphs are
+    switched off, and is chosen anew by a regrid and by another tile width; an explicit one
+    stays, and -1 goes back to the rule."""
+    run(stub, """
+        from vespa_jl_amd import blockmesh as BM
+        from test_gpu_blocks import three_boxes
+        small, large, src = three_boxes()
+        want = BM.BlockSimulation(large, np.float64).info()["zchunk"]
+        wide = BM.BlockSimulation(large, np.float64)
+        wide.set_tiling(4)
+        assert BM.BlockSimulation(small, np.float64).info()["zchunk"] == 1 and want == 2
+        for set_up in (lambda s: None, lambda s: s.set_launch(use_graph=False),
+                       lambda s: (s.set_launch(zchunk=5), s.set_launch(zchunk=-1))):
+            s = BM.BlockSimulation(small, np.float64)
+            set_up(s)
+            s.regrid(large, src)
+            assert s.info()["zchunk"] == want
+            s.set_tiling(4)
+            assert s.info()["zchunk"] == wide.info()["zchunk"] == 4
+        s = BM.BlockSimulation(small, np.float64)
+        s.set_launch(zchunk=1)
+        s.regrid(large, src)
+        assert s.info()["zchunk"] == 1
+        assert L.vh_blocks_set_launch(s._h, -2, 0, 0) != 0
+        """)

@@ -224,7 +224,7 @@ def evolve_amr(qb: QuadBlocks, U0: np.ndarray, tfinal: float, cfl: float = 0.4, 
         # graph would be captured, instantiated and destroyed per regrid for a
         # few replays (measured on the Sedov run: whole run 0.069 -> 0.059 s,
         # regrid tables 6.5 -> 5.3 ms without graphs).
-        sim.set_launch(zchunk=sim.info()["zchunk"], use_graph=False)
+        sim.set_launch(use_graph=False)
     sim.upload(np.ascontiguousarray(U0, dtype=dtype))
     t, steps = 0.0, 0
     snaps = {}

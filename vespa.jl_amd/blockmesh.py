@@ -406,7 +406,10 @@ class BlockSimulation:
         finally:
             b.free()
 
-    def set_launch(self, zchunk: int = 8, max_workgroups: int = 0, use_graph: bool = True):
+    def set_launch(self, zchunk: int = -1, max_workgroups: int = 0, use_graph: bool = True):
+        """z planes per tile (-1: the library's choice for the mesh, chosen anew by a regrid;
+        0: whole blocks), workgroup cap (0: none for the compiled tile shapes, 3 per compute
+        unit for the others), and whether single-rate steps replay a captured graph."""
         self._check(self._lib.vh_blocks_set_launch(self._h, int(zchunk), int(max_workgroups), int(bool(use_graph))))
 
     def set_tiling(self, max_tile_x: int = 32):

@@ -1019,7 +1019,7 @@ struct vh_blocks {
   int dtype = VH_F64, mode = VH_EXACT, device = 0;
   size_t esize = 8;
   int zchunk = 8;
-  bool zchunk_auto = true;   // zchunk follows the mesh until vh_blocks_set_launch sets it
+  bool zchunk_auto = true;   // zchunk follows the mesh and the tile width (vh_blocks_set_launch: -1)
   int max_tx = 32;        // widest tile along x
   int max_wgs = 0;        // persistent workgroups (0: 3 per CU)
   int ncu = 256;
@@ -2068,25 +2068,32 @@ int vh_blocks_totals(vh_blocks* m, double* out5) {
   return 0;
 }
 
+// Rebuilds the tables for another tile shape (the stream is idle: the arena can be rewritten).
+static int retile(vh_blocks* m, int zchunk, int max_tx) {
+  if (zchunk != m->zchunk || max_tx != m->max_tx) {
+    HostTables& H = m->H2;
+    int rc = build_tables(m->T, zchunk, H, max_tx);
+    if (rc) return rc;
+    std::swap(m->H, H);
+    m->zchunk = zchunk;
+    m->max_tx = max_tx;
+    rc = upload_tables(m, m->H, m->T.nb, m->arena_cur);
+    if (rc) return rc;
+  }
+  return alloc_partials(m);
+}
+
 int vh_blocks_set_launch(vh_blocks* m, int32_t zchunk, int32_t max_workgroups, int32_t use_graph) {
   if (!m) return fail(-1, "null argument%s", "");
-  if (zchunk < 0 || max_workgroups < 0) return fail(-1, "bad launch argument%s", "");
+  if (zchunk < -1 || max_workgroups < 0) return fail(-1, "bad launch argument%s", "");
   VH_HIP(hipSetDevice(m->device));
   VH_HIP(hipStreamSynchronize(m->stream));
   drop_graph(m);
   m->use_graph = use_graph ? 1 : 0;
   m->max_wgs = max_workgroups;
-  m->zchunk_auto = false;
-  if (zchunk != m->zchunk) {
-    HostTables& H = m->H2;
-    int rc = build_tables(m->T, zchunk, H, m->max_tx);
-    if (rc) return rc;
-    std::swap(m->H, H);
-    m->zchunk = zchunk;
-    rc = upload_tables(m, m->H, m->T.nb, m->arena_cur);   // the stream is idle: the arena can be rewritten
-    if (rc) return rc;
-  }
-  return alloc_partials(m);
+  const int rc = retile(m, zchunk < 0 ? default_zchunk(m->T, m->max_tx) : zchunk, m->max_tx);
+  if (!rc) m->zchunk_auto = zchunk < 0;
+  return rc;
 }
 
 int vh_blocks_set_tiling(vh_blocks* m, int32_t max_tile_x) {
@@ -2095,15 +2102,8 @@ int vh_blocks_set_tiling(vh_blocks* m, int32_t max_tile_x) {
   if (max_tile_x == m->max_tx) return 0;
   VH_HIP(hipSetDevice(m->device));
   VH_HIP(hipStreamSynchronize(m->stream));
-  HostTables& H = m->H2;
-  int rc = build_tables(m->T, m->zchunk, H, max_tile_x);
-  if (rc) return rc;
   drop_graph(m);
-  std::swap(m->H, H);
-  m->max_tx = max_tile_x;
-  rc = upload_tables(m, m->H, m->T.nb, m->arena_cur);   // the stream is idle: the arena can be rewritten
-  if (rc) return rc;
-  return alloc_partials(m);
+  return retile(m, m->zchunk_auto ? default_zchunk(m->T, max_tile_x) : m->zchunk, max_tile_x);
 }
 
 int vh_blocks_info(const vh_blocks* m, int64_t* counts6, int32_t* zchunk, int32_t* workgroups) {
