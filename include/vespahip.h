@@ -223,9 +223,10 @@ int vh_grid_accumulate_flux(vh_grid* g, void* acc_host);
 /* Wait for all work queued on the context's stream. */
 int vh_grid_sync(vh_grid* g);
 
-/* Launch shape of the fused stage kernels: tile variant (0 = library default)
- * and z planes per workgroup (0 = default). See vh_grid_tile_count for the
- * available tile variants of the grid's rank. Used by the autotuner. */
+/* Launch shape of the fused stage kernels: tile variant (a new grid's is chosen from
+ * its sizes and type) and z planes per workgroup (0 = the library's choice for
+ * that variant). See vh_grid_tile_count for the available tile variants of the grid's
+ * rank. Used by the autotuner. */
 int vh_grid_set_launch(vh_grid* g, int32_t tile_variant, int32_t zchunk);
 int vh_grid_tile_count(const vh_grid* g);
 int vh_grid_get_launch(const vh_grid* g, int32_t* tile_x, int32_t* tile_y, int32_t* zchunk,

@@ -217,3 +217,35 @@ def test_automatic_z_planes_follow_the_mesh(stub):
         assert s.info()["zchunk"] == 1
         assert L.vh_blocks_set_launch(s._h, -2, 0, 0) != 0
         """)
+
+
+def test_launch_defaults_of_a_grid(stub):
+    """zchunk 0 is the library's march for the variant (the default variant's is the one a new
+    grid has), and the tuners try the defaults and marches shorter than them."""
+    run(stub, """
+        from vespa_jl_amd import autotune as AT, blockmesh as BM
+        def sim(dims, T=np.float64):
+            prob = V.Problem("l", dims, ((0.0, 1.0),) * len(dims), 1.4, "periodic", lambda x, y, z: (1.0, 0.0, 0.0, 0.0, 1.0), 1.0, 0.3)
+            return V.Simulation(V.UniformMesh(dims, prob.domain), prob, eltype=T)
+        for dims in ((60, 52, 44), (96, 96, 96), (171, 130, 97), (256, 256, 128), (33, 20), (50,)):
+            for T in (np.float64, np.float32):
+                s = sim(dims, T)
+                d = s.launch()
+                for v in range(s.tile_count()):
+                    s.set_launch(v, 0)
+                    if s.launch()["tile"] == d["tile"]: assert s.launch() == d, (dims, d, s.launch())
+                s.set_launch(0, 7)
+                assert s.launch()["zchunk"] == (7 if len(dims) == 3 else 1)
+        s = sim((60, 52, 44))
+        d = s.launch()
+        r = AT.tune_grid(s, steps=1, use_cache=False)
+        tried = [(t["tile"], t["zchunk"]) for t in r["trials"]]
+        assert (d["tile"], d["zchunk"]) in tried and d["zchunk"] == 1
+        assert {1, 2, 4, 8, 16, 32} <= {z for _, z in tried}
+        m = BM.random_block_pairs(12, seed=3, rank=3)
+        b = BM.BlockSimulation(m, np.float64, cfl=0.3)
+        z = b.info()["zchunk"]
+        r = AT.tune_blocks(b, steps=1, use_cache=False)
+        assert {-1, 0, 1, 2, 4, 8, 16} <= {t["zchunk"] for t in r["trials"]}
+        assert {t["max_tile_x"] for t in r["trials"] if t["zchunk"] == -1 and t["max_workgroups"] == 0} == {16, 32}
+        """)

@@ -11,8 +11,10 @@ runs apply it without sweeping.
 * block meshes: widest tile along x × z planes per tile × persistent workgroups
   per compute unit.
 
-Every candidate computes the same values (launch shape never changes the
-arithmetic); the state advanced during the sweep is restored afterwards.
+The library's own choice of z planes (0 for a grid, -1 for a block mesh) is always
+among the default candidates, so that tuning never ends with a slower launch than an
+untuned run has. Every candidate computes the same values (launch shape never changes
+the arithmetic); the state advanced during the sweep is restored afterwards.
 """
 from __future__ import annotations
 
@@ -50,9 +52,14 @@ def _store(d: dict) -> None:
         pass
 
 
+# Part of every key: raised when the kernels or their default launches change, so that
+# picks made for earlier ones are tuned anew.
+_KERNELS = 2
+
+
 def _device_sig() -> str:
     from ._lib import device_cu_count
-    return f"cu{device_cu_count()}"
+    return f"k{_KERNELS}:cu{device_cu_count()}"
 
 
 def _grid_key(sim) -> str:
@@ -60,8 +67,9 @@ def _grid_key(sim) -> str:
             f"{_device_sig()}")
 
 
-def tune_grid(sim, steps: int = 5, zchunks=(8, 16, 32), use_cache: bool = True) -> dict:
-    """Pick the tile variant and z chunk of a uniform-grid Simulation."""
+def tune_grid(sim, steps: int = 5, zchunks=(0, 1, 2, 4, 8, 16, 32), use_cache: bool = True) -> dict:
+    """Pick the tile variant and z chunk (0: the library's for the variant) of a
+    uniform-grid Simulation. The z chunks of the result are the ones they stand for."""
     key = _grid_key(sim)
     cache = _load() if use_cache else {}
     if key in cache:
@@ -70,13 +78,18 @@ def tune_grid(sim, steps: int = 5, zchunks=(8, 16, 32), use_cache: bool = True) 
         return dict(c, cached=True)
     U0, t0, n0 = sim.state(), sim.t, sim.step_count
     zs = zchunks if sim.mesh.rank == 3 else (0,)
-    trials = []
+    trials, seen = [], set()
     for v in range(sim.tile_count()):
         for z in zs:
             sim.set_launch(v, z)
+            launch = sim.launch()
+            if (v, launch["zchunk"]) in seen:
+                continue
+            seen.add((v, launch["zchunk"]))
             sim.upload(U0)
             r = sim.time_steps(steps)
-            trials.append({"tile_variant": v, "zchunk": z, "step_ms": r["step_ms"], "tile": sim.launch()["tile"]})
+            trials.append({"tile_variant": v, "zchunk": launch["zchunk"], "step_ms": r["step_ms"],
+                           "tile": launch["tile"]})
     best = min(trials, key=lambda d: d["step_ms"])
     sim.set_launch(best["tile_variant"], best["zchunk"])
     sim.upload(U0)
@@ -94,10 +107,11 @@ def _blocks_key(bsim) -> str:
     return f"blocks:{':'.join(map(str, sig))}:{bsim.eltype.name}:{_device_sig()}"
 
 
-def tune_blocks(bsim, steps: int = 3, max_tile_x=(16, 32), zchunks=(0, 8, 16), wgs_per_cu=(0, 4),
+def tune_blocks(bsim, steps: int = 3, max_tile_x=(16, 32), zchunks=(-1, 0, 1, 2, 4, 8, 16), wgs_per_cu=(0, 4),
                 use_cache: bool = True) -> dict:
-    """Pick the tiling, z planes per tile and persistent workgroup count of a
-    BlockSimulation (single-rate graph replays are timed)."""
+    """Pick the tiling, z planes per tile (-1: the library's choice, which follows the
+    mesh; 0: whole blocks) and workgroup cap of a BlockSimulation (single-rate graph
+    replays are timed)."""
     key = _blocks_key(bsim)
     cache = _load() if use_cache else {}
     if key in cache:

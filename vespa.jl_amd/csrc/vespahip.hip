@@ -227,6 +227,16 @@ static void free_grav(vh_grid* g) {
 
 static const int kMaxCflBlocks = 2048;
 
+// Default planes per workgroup of a 3D tile variant (march_planes; three Float64 workgroups of
+// 256 lanes per compute unit, four Float32).
+static int default_march(const vh_grid* g, int variant, double* cost = nullptr) {
+  const GridDev& G = g->G;
+  const TileShape t = tile_for(3, variant);
+  const long long columns = (long long)((G.n[0] + t.tx - 1) / t.tx) * ((G.n[1] + t.ty - 1) / t.ty);
+  const int per_cu = (g->dtype == VH_F64 ? 3 : 4) * 256 / (t.tx * t.ty);
+  return march_planes(columns, G.n[2], 16, per_cu > 0 ? per_cu : 1, cu_count(g->device), cost);
+}
+
 static int configure(vh_grid* g, int variant, int zchunk) {
   GridDev& G = g->G;
   if (variant < 0 || variant >= tile_count_for_rank(G.rank))
@@ -238,7 +248,7 @@ static int configure(vh_grid* g, int variant, int zchunk) {
   G.tiles_x = (G.n[0] + t.tx - 1) / t.tx;
   G.tiles_y = (G.n[1] + t.ty - 1) / t.ty;
   if (G.rank == 3) {
-    if (zchunk <= 0) zchunk = 32;
+    if (zchunk <= 0) zchunk = default_march(g, variant);
     if (zchunk > G.n[2]) zchunk = G.n[2];
   } else {
     zchunk = 1;
@@ -259,35 +269,22 @@ static int configure(vh_grid* g, int variant, int zchunk) {
   return 0;
 }
 
-// Default launch shape; the autotuner in the host package can override it per
-// workload. 3D: Float32 32×8 cells, Float64 16×16 (5% faster at 96³ and 128³, where rows
+// Default tile variant (with its default march); the autotuner in the host package can override
+// both per workload. 3D: Float32 32×8 cells, Float64 16×16 (5% faster at 96³ and 128³, where rows
 // start on 128-byte lines) or 32×8 when that is estimated faster; on rows that do not,
 // a 16-cell Float64 row segment touches two lines for one line of data and 16×16
-// is charged 10% (171×130×97, 8 planes: 111/140 µs against 105/121). Planes per workgroup
-// by march_planes (three Float64 workgroups per compute unit, four Float32). 2D:
+// is charged 10% (171×130×97, 8 planes: 111/140 µs against 105/121). 2D:
 // Float64 16×16 (512², walls: 15.7/20.0 µs against 19.0/20.2 for 32×8), Float32 32×8
 // (1024²: 19.0/23.3 against 22.3/26.0).
-static void default_launch(const vh_grid* g, int* variant, int* zchunk) {
+static int default_variant(const vh_grid* g) {
   const GridDev& G = g->G;
-  const bool f64 = g->dtype == VH_F64;
-  *zchunk = 0;
-  *variant = G.rank == 2 && f64 ? 2 : 0;
-  if (G.rank < 3) return;
-  const int cus = cu_count(g->device), per_cu = f64 ? 3 : 4;
-  auto shape = [&](int v, double* cost) {
-    const TileShape t = tile_for(3, v);
-    const long long columns = (long long)((G.n[0] + t.tx - 1) / t.tx) * ((G.n[1] + t.ty - 1) / t.ty);
-    return march_planes(columns, G.n[2], 16, per_cu, cus, cost);
-  };
+  if (g->dtype != VH_F64 || G.rank == 1) return 0;
+  if (G.rank == 2) return 2;
   double wide, square;
-  *zchunk = shape(0, &wide);
-  if (!f64) return;
-  const int zs = shape(2, &square);
+  default_march(g, 0, &wide);
+  default_march(g, 2, &square);
   if ((G.n[0] * g->esize) % 128) square *= 1.1;
-  if (square <= wide) {
-    *variant = 2;
-    *zchunk = zs;
-  }
+  return square <= wide ? 2 : 0;
 }
 
 static void enqueue_stage_dt(vh_grid* g, bool stage2, const void* Us, const void* U0, void* Uout,
@@ -589,9 +586,7 @@ int vh_grid_create(vh_grid** out, int32_t rank, const int64_t* dims, const doubl
     G.area[a] = ar;
   }
   if (hipGetDevice(&g->device) != hipSuccess) { delete g; return fail(-2, "no HIP device%s", ""); }
-  int variant, zchunk;
-  default_launch(g, &variant, &zchunk);
-  int rc = configure(g, variant, zchunk);
+  int rc = configure(g, default_variant(g), 0);
   if (rc) { vh_grid_destroy(g); return rc; }
   const size_t bytes = (size_t)5 * n * g->esize;
   if (hipMalloc(&g->U, bytes) != hipSuccess || hipMalloc(&g->U1, bytes) != hipSuccess ||
