@@ -258,6 +258,10 @@ int vh_grid_step_vjp(vh_grid* g, const void* dU, double dt, const void* dWbar, v
  * boundary). Both give the same values to round-off. */
 int vh_grid_set_adjoint_form(vh_grid* g, int32_t fused);
 
+/* 1 if the tiled kernel is the one that runs on a periodic nx × ny grid (with fused = 1,
+ * outputs apart from the inputs), else 0. Host only. */
+int vh_adjoint_fused_covers(int64_t nx, int64_t ny);
+
 /* Checkpointed rollout of nsteps steps with the device CFL dt: the forward
  * keeps the state every `every` steps and each step's dt; the backward
  * recomputes each segment from its checkpoint and applies the step VJPs in

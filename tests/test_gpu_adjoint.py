@@ -183,6 +183,7 @@ def test_fused_tiles_of_any_size(O, dims):
     two (17 and 9 cells) that stay with the three-pass form; the bound is that of the
     whole tiles (the forms differ in summation order only)."""
     print(f"fused jat {dims}", flush=True)
+    assert AD.fused_covers(*dims) == (dims not in ((17, 40), (40, 9)))
     shape = (5,) + tuple(reversed(dims))
     U = random_state(shape[1:], seed=21, vmax=0.4)
     g = O.make_grid(dims, [(0.0, 1.0)] * 2, "periodic", 1.4)

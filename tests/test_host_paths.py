@@ -249,3 +249,28 @@ def test_launch_defaults_of_a_grid(stub):
         assert {-1, 0, 1, 2, 4, 8, 16} <= {t["zchunk"] for t in r["trials"]}
         assert {t["max_tile_x"] for t in r["trials"] if t["zchunk"] == -1 and t["max_workgroups"] == 0} == {16, 32}
         """)
+
+
+def test_sizes_of_the_fused_reverse_form(stub):
+    """The tiled kernel runs (one launch per evaluation, the passes take three) on periodic
+    sizes of 10 to 16 and above 17, and not where its output is the state it reads."""
+    run(stub, """
+        from vespa_jl_amd import adjoint as AD
+        from vespa_jl_amd._lib import DeviceBuffer
+        for n in range(2, 70):
+            assert AD.fused_covers(n, 32) == AD.fused_covers(32, n) == (10 <= n <= 16 or n > 17)
+        def launches(dims, bc="periodic", fused=True, alias=False):
+            prob = V.Problem("l", dims, ((0.0, 1.0),) * len(dims), 1.4, bc, lambda x, y, z: (1.0, 0.0, 0.0, 0.0, 1.0), 1.0, 0.3)
+            sim = V.Simulation(V.UniformMesh(dims, prob.domain), prob)
+            AD.set_form(sim, fused)
+            U, w, o = (DeviceBuffer(40 * sim.ncell) for _ in range(3))
+            S.stub_clear()
+            V.check(L.vh_grid_step_vjp(sim._h, U.ptr, 0.1, w.ptr, U.ptr if alias else o.ptr))
+            return len([l for l in log() if l[0] == "launch"]) - 2   # the dt and stage 1
+        for dims in ((10, 10), (16, 48), (18, 33), (50, 37), (32, 32), (64, 16)):
+            assert launches(dims) == 2 and launches(dims, fused=False) == 6
+            assert launches(dims, alias=True) == 4
+        for dims in ((17, 40), (40, 17), (9, 40), (40, 9), (12,), (16, 16, 16)):
+            assert launches(dims) == 6
+        assert launches((32, 32), "outflow") == 6
+        """)

@@ -35,7 +35,7 @@ EXPORTED = (
     "vh_blocks_enable_gravity", "vh_blocks_disable_gravity", "vh_blocks_solve_poisson", "vh_blocks_phi_upload",
     "vh_blocks_phi_download", "vh_blocks_apply_laplacian", "vh_blocks_gravity_accel",
     "vh_grid_step_vjp", "vh_adjoint_create", "vh_adjoint_destroy", "vh_adjoint_forward",
-    "vh_adjoint_backward", "vh_adjoint_info", "vh_grid_set_adjoint_form",
+    "vh_adjoint_backward", "vh_adjoint_info", "vh_grid_set_adjoint_form", "vh_adjoint_fused_covers",
     "vh_grid_step_bflux", "vh_grid_bflux_count", "vh_grid_set_parent_ghost",
     "vh_grid_enable_gravity", "vh_grid_disable_gravity", "vh_grid_solve_poisson", "vh_grid_phi_upload",
     "vh_grid_phi_download", "vh_grid_apply_laplacian", "vh_grid_gravity_accel",
@@ -151,6 +151,8 @@ def load_library(path: str | None = None):
     L.vh_adjoint_backward.argtypes = [vp, vp, vp]
     L.vh_adjoint_info.argtypes = [vp, dp, dp, i64p, dp]
     L.vh_grid_set_adjoint_form.argtypes = [vp, C.c_int32]
+    L.vh_adjoint_fused_covers.argtypes = [C.c_int64, C.c_int64]
+    L.vh_adjoint_fused_covers.restype = C.c_int
     L.vh_grid_step_bflux.argtypes = [vp, C.c_double, vp]
     L.vh_grid_step_bflux.restype = C.c_int
     L.vh_grid_set_parent_ghost.argtypes = [vp, vp]

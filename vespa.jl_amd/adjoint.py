@@ -41,6 +41,11 @@ def set_form(sim, fused: bool) -> None:
     check(load_library().vh_grid_set_adjoint_form(sim._h, int(bool(fused))))
 
 
+def fused_covers(nx: int, ny: int) -> bool:
+    """Whether the single tiled kernel is the form that runs on a periodic nx × ny grid."""
+    return bool(load_library().vh_adjoint_fused_covers(int(nx), int(ny)))
+
+
 def step_vjp(sim, U: np.ndarray, dt: float, wbar: np.ndarray) -> np.ndarray:
     """(∂ step(U, dt)/∂U)ᵀ wbar on the GPU for host arrays shaped like sim.state()."""
     _require_f64(sim)

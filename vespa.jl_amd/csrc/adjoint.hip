@@ -62,6 +62,15 @@ void adj_launch_cells(hipStream_t s, const double* U, const double* W, double* c
   else launch_cells<1>(s, U, W, F, base1, a1, base2, a2, beta, dtp, G, out);
 }
 
+// The last tile's halo (two cells past the tile) has to wrap around once only:
+// every size but 1..9 and 17. The fused form is the faster one at all the others:
+// 10² 10.8 µs in passes, 7.7 fused; 50×37 14 and 11; 100² 15 and 10; 512² 47 and 23;
+// 1500×1100 319 and 134; 2048² 749 and 352.
+bool adj_fused_covers(long long nx, long long ny) {
+  auto covers = [](long long n, int tile) { return n > 0 && (n + tile - 1) / tile * tile + 2 < 2 * n; };
+  return covers(nx, VH_PROFILE_NS::JTX) && covers(ny, VH_PROFILE_NS::JTY);
+}
+
 bool adj_launch_jat_fused(hipStream_t s, const double* U, const double* lam, const double* base1, double a1,
                           const double* base2, double a2, double beta, const double* dtp, const GridDev& G,
                           double* out) {
@@ -70,13 +79,8 @@ bool adj_launch_jat_fused(hipStream_t s, const double* U, const double* lam, con
   const bool periodic = G.bc[0] == BC_PERIODIC && G.bc[2] == BC_PERIODIC;
   if (G.rank != 2 || !periodic) return false;
   if (out == U || out == lam) return false;   // other tiles read these cells; the passes read them before out is written
-  // The last tile's halo (two cells past the tile) has to wrap around once only:
-  // every size but 1..9 and 17. The fused form is the faster one at all the others:
-  // 10² 10.8 µs in passes, 7.7 fused; 50×37 14 and 11; 100² 15 and 10; 512² 47 and 23;
-  // 1500×1100 319 and 134; 2048² 749 and 352.
-  const int tx = (G.n[0] + JTX - 1) / JTX, ty = (G.n[1] + JTY - 1) / JTY;
-  if (tx * JTX + 2 >= 2 * G.n[0] || ty * JTY + 2 >= 2 * G.n[1]) return false;
-  const dim3 grid(tx, ty);
+  if (!adj_fused_covers(G.n[0], G.n[1])) return false;
+  const dim3 grid((G.n[0] + JTX - 1) / JTX, (G.n[1] + JTY - 1) / JTY);
   hipLaunchKernelGGL(VH_PROFILE_NS::adj_jat2d_periodic_kernel, grid, dim3(VH_PROFILE_NS::JNT), 0, s, U, lam, base1, a1,
                      base2, a2, beta, dtp, G, out);
   return true;

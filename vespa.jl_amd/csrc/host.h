@@ -132,6 +132,7 @@ void adj_launch_cells(hipStream_t s, const double* U, const double* W, double* c
                       const double* dtp, const GridDev& G, double* out);
 // Fused single-kernel form for 2D grids periodic on both axes with 10 to 16 or
 // more than 17 cells along each; returns false (nothing launched) otherwise.
+bool adj_fused_covers(long long nx, long long ny);
 bool adj_launch_jat_fused(hipStream_t s, const double* U, const double* lam, const double* base1, double a1,
                           const double* base2, double a2, double beta, const double* dtp, const GridDev& G,
                           double* out);

@@ -1158,6 +1158,8 @@ int vh_grid_set_adjoint_form(vh_grid* g, int32_t fused) {
   return 0;
 }
 
+int vh_adjoint_fused_covers(int64_t nx, int64_t ny) { return adj_fused_covers(nx, ny) ? 1 : 0; }
+
 int vh_adjoint_destroy(vh_adjoint* a) {
   if (!a) return 0;
   if (a->g && a->g->stream) (void)hipStreamSynchronize(a->g->stream);
