@@ -79,7 +79,10 @@ hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t a, int d) { return
 hipError_t hipGetLastError(void) { return hipSuccess; }
 const char* hipGetErrorString(hipError_t e) { return (void)e, "stub error"; }
 hipError_t hipGetSymbolAddress(void** p, const void* s) { return *p = (void*)s, hipSuccess; }
-hipError_t hipMalloc(void** p, size_t n) { return alloc(p, n, hipMemoryTypeDevice); }
+hipError_t hipMalloc(void** p, size_t n) {
+  say("malloc %zu\n", n);
+  return alloc(p, n, hipMemoryTypeDevice);
+}
 hipError_t hipHostMalloc(void** p, size_t n, unsigned f) { return (void)f, alloc(p, n, hipMemoryTypeHost); }
 static hipError_t release(void* p) {
   const int i = find(p);

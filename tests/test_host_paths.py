@@ -274,3 +274,23 @@ def test_sizes_of_the_fused_reverse_form(stub):
             assert launches(dims) == 6
         assert launches((32, 32), "outflow") == 6
         """)
+
+
+def test_gravity_keeps_no_vector_it_does_not_use(stub):
+    """Work vectors of the Poisson solve: r and two p on a uniform grid, whose operator is
+    applied again instead of stored, and Ap on a block mesh."""
+    run(stub, """
+        from vespa_jl_amd import blockmesh as BM
+        def allocated(f):
+            S.stub_clear()
+            f()
+            return [int(l[1]) for l in log() if l[0] == "malloc"]
+        dims = (16, 12, 10)
+        prob = V.Problem("l", dims, ((0.0, 1.0),) * 3, 1.4, "periodic", lambda x, y, z: (1.0, 0.0, 0.0, 0.0, 1.0), 1.0, 0.3)
+        sim = V.Simulation(V.UniformMesh(dims, prob.domain), prob)
+        a = allocated(lambda: V.enable_gravity(sim))
+        assert 3 * 8 * sim.ncell in a and max(a) == 3 * 8 * sim.ncell and 8 in a
+        m = BM.random_block_pairs(4, seed=3, rank=3)
+        s = BM.BlockSimulation(m, np.float64)
+        assert 4 * 8 * s.ncell in allocated(lambda: s.enable_gravity())
+        """)

@@ -1667,7 +1667,7 @@ static void free_grav(vh_blocks* m) {
   BlockGrav* G = m->grav;
   if (!G) return;
   for (void* p : {(void*)G->rowptr, (void*)G->colidx, (void*)G->coef, (void*)G->vol, (void*)G->glo, (void*)G->ghi,
-                  (void*)G->gsum, G->g, G->B.phi, G->B.work, G->B.state, (void*)G->B.scal, (void*)G->B.partials})
+                  (void*)G->gsum, G->g, G->B.phi, G->B.work, G->B.state, (void*)G->B.sumv, (void*)G->B.partials})
     (void)hipFree(p);
   if (G->B.host_state) (void)hipHostFree(G->B.host_state);
   delete G;
@@ -1957,21 +1957,20 @@ int vh_blocks_enable_gravity(vh_blocks* m, double G, int64_t maxiter, double tol
     return rc;
   }
   hipError_t e = hipMalloc(&Gv->B.phi, m->esize * n);
-  if (e == hipSuccess) e = hipMalloc(&Gv->B.work, 4 * m->esize * n);
+  if (e == hipSuccess) e = hipMalloc(&Gv->B.work, kGravWorkCsr * m->esize * n);
   if (e == hipSuccess) e = hipMalloc(&Gv->g, 3 * m->esize * n);
   if (e == hipSuccess) e = hipMalloc(&Gv->B.state, kGravStateBytes);
-  if (e == hipSuccess) e = hipMalloc(&Gv->B.scal, 8 * sizeof(double));
+  if (e == hipSuccess) e = hipMalloc(&Gv->B.sumv, sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&Gv->B.partials, kGravPartials * sizeof(double));
   if (e == hipSuccess) e = hipHostMalloc(&Gv->B.host_state, kGravStateBytes, 0);
   if (e == hipSuccess) e = hipMemsetAsync(Gv->B.phi, 0, m->esize * n, m->stream);
   if (e == hipSuccess) e = hipMemsetAsync(Gv->g, 0, 3 * m->esize * n, m->stream);
-  if (e == hipSuccess) e = hipMemsetAsync(Gv->B.scal, 0, 8 * sizeof(double), m->stream);
   if (e == hipSuccess) e = hipMemsetAsync(Gv->B.state, 0, kGravStateBytes, m->stream);
   // Σ V accumulated cell by cell in leaf order in Float64 (the mean projections'
   // denominator, src/gravity.jl:230-246, 310-320)
   double sumv = 0.0;
   for (long long i = 0; i < n; ++i) sumv += C.vol[i];
-  if (e == hipSuccess) e = hipMemcpyAsync(Gv->B.scal + 1, &sumv, sizeof(double), hipMemcpyHostToDevice, m->stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(Gv->B.sumv, &sumv, sizeof(double), hipMemcpyHostToDevice, m->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
   if (e != hipSuccess) {
     free_grav(m);

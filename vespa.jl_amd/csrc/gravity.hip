@@ -516,7 +516,7 @@ static int solve_t(hipStream_t s, const Row& row, long long n, const double* vol
   T* phi = (T*)B.phi;
   T* r = (T*)B.work;
   T* p[2] = {r + n, r + 2 * n};
-  T* Ap = r + 3 * n;   // used by the CSR form
+  T* Ap = Row::kStoreAp ? r + 3 * n : nullptr;
   const T* rho = (const T*)B.rho;
   CgState* st = (CgState*)B.state;
   CgState* host = (CgState*)B.host_state;
@@ -524,7 +524,7 @@ static int solve_t(hipStream_t s, const Row& row, long long n, const double* vol
   double* pap = rr + kCgWgs;
   double* aux = pap + kCgWgs;
   double* bb = aux + kCgWgs;
-  const double* sumv = B.scal + 1;   // Σ V, summed cell by cell on the host as the reference does
+  const double* sumv = B.sumv;
   *host = CgState{};
   hipLaunchKernelGGL(cg_clear_kernel, dim3(1), dim3(1), 0, s, st);
   if (P.project_mean) hipLaunchKernelGGL(vsum_kernel<T>, nb, nt, 0, s, rho, vols, vol, n, aux);

@@ -152,15 +152,16 @@ struct GravParams {
 };
 struct GravBuffers {
   void* phi = nullptr;     // ncell values
-  void* work = nullptr;    // 4·ncell values: r, two p, Ap (block meshes)
+  void* work = nullptr;    // r and two p; block meshes also Ap (kGravWork, kGravWorkCsr values per cell)
   const void* rho = nullptr;
   void* state = nullptr;   // CG state block (device)
-  double* scal = nullptr;  // [1]: Σ V (device)
+  double* sumv = nullptr;  // Σ V (device), summed cell by cell on the host as the reference does
   double* partials = nullptr;  // kGravPartials per-workgroup partial sums (device)
   void* host_state = nullptr;  // pinned; the kernels write done, iters, relres here
 };
 constexpr int kGravStateBytes = 64;
 constexpr int kGravPartials = 4096;
+constexpr int kGravWork = 3, kGravWorkCsr = 4;
 void grav_apply(hipStream_t s, int dtype, const GridDev& G, int gper, const void* x, void* out);
 void grav_accel(hipStream_t s, int dtype, const GridDev& G, int gper, const void* phi, void* g);
 int grav_solve(hipStream_t s, int dtype, const GridDev& G, const GravParams& P, GravBuffers& B, long long* iters,

@@ -217,7 +217,7 @@ static void free_grav(vh_grid* g) {
   if (w->B.phi) (void)hipFree(w->B.phi);
   if (w->B.work) (void)hipFree(w->B.work);
   if (w->B.state) (void)hipFree(w->B.state);
-  if (w->B.scal) (void)hipFree(w->B.scal);
+  if (w->B.sumv) (void)hipFree(w->B.sumv);
   if (w->B.partials) (void)hipFree(w->B.partials);
   if (w->B.host_state) (void)hipHostFree(w->B.host_state);
   delete w;
@@ -808,18 +808,17 @@ int vh_grid_enable_gravity(vh_grid* g, double G, int32_t phi_periodic, int64_t m
   w->P.tol = tol;
   const long long n = g->G.ncell;
   hipError_t e = hipMalloc(&w->B.phi, g->esize * n);
-  if (e == hipSuccess) e = hipMalloc(&w->B.work, 4 * g->esize * n);
+  if (e == hipSuccess) e = hipMalloc(&w->B.work, kGravWork * g->esize * n);
   if (e == hipSuccess) e = hipMalloc(&w->B.state, kGravStateBytes);
-  if (e == hipSuccess) e = hipMalloc(&w->B.scal, 8 * sizeof(double));
+  if (e == hipSuccess) e = hipMalloc(&w->B.sumv, sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&w->B.partials, kGravPartials * sizeof(double));
   if (e == hipSuccess) e = hipHostMalloc(&w->B.host_state, kGravStateBytes);
   if (e == hipSuccess) e = hipMemsetAsync(w->B.phi, 0, g->esize * n, g->stream);
-  if (e == hipSuccess) e = hipMemsetAsync(w->B.scal, 0, 8 * sizeof(double), g->stream);
   if (e == hipSuccess) e = hipMemsetAsync(w->B.state, 0, kGravStateBytes, g->stream);
   // Σ V accumulated cell by cell in Float64, as the reference's projections do.
   double sumv = 0.0;
   for (long long i = 0; i < n; ++i) sumv += g->G.V;
-  if (e == hipSuccess) e = hipMemcpyAsync(w->B.scal + 1, &sumv, sizeof(double), hipMemcpyHostToDevice, g->stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(w->B.sumv, &sumv, sizeof(double), hipMemcpyHostToDevice, g->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(g->stream);
   if (e != hipSuccess) {
     free_grav(g);
