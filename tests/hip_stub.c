@@ -118,9 +118,13 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned f) {
   (void)f;
   if (failing("hipStreamCreateWithFlags")) return hipErrorOutOfMemory;
   *s = (hipStream_t)malloc(16);
+  say("stream %p\n", (void*)*s);
   return hipSuccess;
 }
-hipError_t hipStreamDestroy(hipStream_t s) { return (void)s, hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t s) {
+  say("destroy %p\n", (void*)s);
+  return hipSuccess;
+}
 hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t* d) { return (void)s, *d = 0, hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t s) {
   say("sync %p\n", (void*)s);

@@ -294,3 +294,44 @@ def test_gravity_keeps_no_vector_it_does_not_use(stub):
         s = BM.BlockSimulation(m, np.float64)
         assert 4 * 8 * s.ncell in allocated(lambda: s.enable_gravity())
         """)
+
+
+def test_side_streams_are_made_once(stub):
+    """Streams for the shape classes of a stage: none for a mesh of one class, for others as
+    many as its stages fork, taken over from meshes that are gone (a bounded number is kept),
+    never shared by two that live."""
+    run(stub, """
+        from vespa_jl_amd import amr, blockmesh as BM
+        def made(): return [l[1] for l in log() if l[0] == "stream"]
+        def launched(): return {l[1] for l in log() if l[0] == "launch"}
+        def stepped(m, **kw):
+            s = BM.BlockSimulation(m, np.float64, cfl=0.3)
+            s.set_launch(**kw)
+            S.stub_clear()
+            s.evolve(max_steps=1)
+            return s
+        flat = amr.QuadBlocks(3, 8, 1).mesh()
+        m = BM.random_block_pairs(12, seed=3, rank=3)
+        for graph in (True, False):
+            stepped(flat, use_graph=graph).close()
+            assert made() == []
+        a = stepped(m)
+        first = made()
+        assert 2 <= len(first) <= 4 and launched() >= set(first)
+        b = stepped(m, use_graph=False)
+        second = made()
+        assert len(second) == len(first) and not launched() & set(first)
+        a.close()
+        c = stepped(m, use_graph=False)
+        assert made() == [] and launched() >= set(first) and not launched() & set(second)
+        b.close()
+        c.close()
+        S.stub_clear()
+        many = [BM.BlockSimulation(m, np.float64, cfl=0.3) for _ in range(8)]
+        for s in many: s.step(0.1)
+        total = len(made()) - len(many) + len(first) + len(second)   # without the contexts' own
+        S.stub_clear()
+        for s in many: s.close()
+        gone = len([l for l in log() if l[0] == "destroy"]) - len(many)
+        assert total == 8 * len(first) and gone == total - 16
+        """)

@@ -1013,6 +1013,66 @@ struct DevReg {
   void* delta = nullptr;
 };
 
+// A stream beside a context's own and the event that joins it there.
+struct Side {
+  hipStream_t stream = nullptr;
+  hipEvent_t join = nullptr;
+  int device = -1;
+};
+// Side streams that no context holds. To make one takes 0.6 ms and to destroy it 0.25, which
+// a mesh of a few steps would notice (first step and close of a 20-block mesh 1.0 and 2.4 ms with
+// four streams of its own, against 0.64 and 0.2 on one stream), so a context gives its own back
+// here, idle; at most kKept are kept, the rest is destroyed.
+class SidePool {
+ public:
+  static bool take(int device, Side* out) {
+    {
+      std::lock_guard<std::mutex> lk(mu());
+      for (int i = kept(); i-- > 0;)
+        if (list()[i].device == device) {
+          *out = list()[i];
+          list()[i] = list()[--kept()];
+          return true;
+        }
+    }
+    Side s;
+    s.device = device;
+    if (hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking) != hipSuccess) return false;
+    if (hipEventCreateWithFlags(&s.join, hipEventDisableTiming) != hipSuccess) {
+      (void)hipStreamDestroy(s.stream);
+      return false;
+    }
+    *out = s;
+    return true;
+  }
+  static void give_back(const Side& s) {
+    {
+      std::lock_guard<std::mutex> lk(mu());
+      if (kept() < kKept) {
+        list()[kept()++] = s;
+        return;
+      }
+    }
+    (void)hipStreamDestroy(s.stream);
+    (void)hipEventDestroy(s.join);
+  }
+
+ private:
+  static constexpr int kKept = 16;
+  static std::mutex& mu() {
+    static std::mutex* m = new std::mutex();   // never destroyed: contexts may go while the process ends
+    return *m;
+  }
+  static Side* list() {
+    static Side l[kKept];
+    return l;
+  }
+  static int& kept() {
+    static int n = 0;
+    return n;
+  }
+};
+
 struct vh_blocks {
   Topo T;
   HostTables H;
@@ -1061,10 +1121,11 @@ struct vh_blocks {
   hipEvent_t look = nullptr;      // recorded behind the first reduction of a step loop
   bool in_loop = false;           // kernels of a step loop look at its end flag
   hipStream_t stream = nullptr;
-  // Side streams of a stage's launches, one per shape class beyond the first, with the
-  // events that fork them from `stream` and join them to it (made at first use).
-  hipStream_t side[kBlockClasses - 1] = {};
-  hipEvent_t ev_fork = nullptr, ev_join[kBlockClasses - 1] = {};
+  // Side streams of a stage's launches (one per shape class beyond the first) from SidePool,
+  // and the event that forks them from `stream`; made at the first stage that forks.
+  Side side[kBlockClasses - 1];
+  int nside = 0;
+  hipEvent_t ev_fork = nullptr;
   hipGraphExec_t graph = nullptr;
   int graph_np = -1;
   // A regrid does not wait for the stream: the graph it replaces is kept here
@@ -1147,6 +1208,12 @@ static int class_wgs(const vh_blocks* m, int l, int c) {
   const int cap = (m->max_wgs > 0 ? m->max_wgs : 3 * m->ncu) * (256 / block_class_lanes(c));
   return n < cap ? n : cap;
 }
+// Shape classes with tiles in list l.
+static int list_classes(const vh_blocks* m, int l) {
+  int n = 0;
+  for (int c = 0; c < kBlockClasses; ++c) n += class_tiles(m, l, c) > 0;
+  return n;
+}
 // Workgroups of a stage launch over list l (= the CFL partials its stage 2 writes).
 static int list_wgs(const vh_blocks* m, int l) {
   int np = 0;
@@ -1160,14 +1227,11 @@ static void enqueue_link(vh_blocks* m, const void* Us) {
   else exact::launch_link_flux(m->dtype, B.nfaces, m->stream, Us, B, m->d_flux);
 }
 
-static int ensure_side_streams(vh_blocks* m) {
-  if (m->ev_fork) return 0;
-  for (int i = 0; i < kBlockClasses - 1; ++i) {   // what an earlier call made is kept
-    if (!m->side[i]) VH_HIP(hipStreamCreateWithFlags(&m->side[i], hipStreamNonBlocking));
-    if (!m->ev_join[i]) VH_HIP(hipEventCreateWithFlags(&m->ev_join[i], hipEventDisableTiming));
-  }
-  VH_HIP(hipEventCreateWithFlags(&m->ev_fork, hipEventDisableTiming));
-  return 0;
+// n side streams for the context; false if they cannot be had.
+static bool have_sides(vh_blocks* m, int n) {
+  if (!m->ev_fork && hipEventCreateWithFlags(&m->ev_fork, hipEventDisableTiming) != hipSuccess) return false;
+  while (m->nside < n && SidePool::take(m->device, &m->side[m->nside])) ++m->nside;
+  return m->nside >= n;
 }
 
 // The classes of a stage write disjoint cells and read only the stage's input, so they
@@ -1182,15 +1246,15 @@ static int ensure_side_streams(vh_blocks* m) {
 static void enqueue_tiles(vh_blocks* m, bool stage2, int l, const void* Us, const void* U0, void* Uout) {
   const double* dtp = m->clock + 1;
   const int* co = m->H.tile_class_off.data() + (size_t)l * (kBlockClasses + 1);
-  int np = 0, launches = 0;
-  for (int c = 0; c < kBlockClasses; ++c) launches += class_wgs(m, l, c) > 0;
+  int np = 0;
+  const int launches = list_classes(m, l);
   bool failed = false;
   auto ok = [&](hipError_t e) {
     failed |= e != hipSuccess;
     return e == hipSuccess;
   };
   bool fork = launches > 1;
-  if (fork && ensure_side_streams(m)) {
+  if (fork && !have_sides(m, launches - 1)) {
     fork = false;
     failed = true;
   }
@@ -1201,8 +1265,8 @@ static void enqueue_tiles(vh_blocks* m, bool stage2, int l, const void* Us, cons
     const int wgs = class_wgs(m, l, c);
     if (wgs == 0) continue;
     hipStream_t s = m->stream;
-    const bool aside = fork && i > 0 && ok(hipStreamWaitEvent(m->side[used], m->ev_fork, 0));
-    if (aside) s = m->side[used];
+    const bool aside = fork && i > 0 && ok(hipStreamWaitEvent(m->side[used].stream, m->ev_fork, 0));
+    if (aside) s = m->side[used].stream;
     BlocksDev B = blocks_dev(m);
     B.tiles = m->d_tiles + m->H.tile_list_off[l] + co[c];
     B.ntiles = co[c + 1] - co[c];
@@ -1211,14 +1275,15 @@ static void enqueue_tiles(vh_blocks* m, bool stage2, int l, const void* Us, cons
     else
       exact::launch_block_stage(m->dtype, m->T.rank, c, stage2, wgs, s, Us, U0, Uout, dtp, m->partials + np, B);
     if (aside) {
-      joinable[used] = ok(hipEventRecord(m->ev_join[used], s));
+      joinable[used] = ok(hipEventRecord(m->side[used].join, s));
       ++used;
     }
     np += wgs;
     ++i;
   }
   for (int i = 0; i < used; ++i)
-    if (!joinable[i] || !ok(hipStreamWaitEvent(m->stream, m->ev_join[i], 0))) (void)hipStreamSynchronize(m->side[i]);
+    if (!joinable[i] || !ok(hipStreamWaitEvent(m->stream, m->side[i].join, 0)))
+      (void)hipStreamSynchronize(m->side[i].stream);
   if (failed) (void)hipGetLastError();   // dealt with
   if (l == 0 && stage2) m->stage_wgs = np;
 }
@@ -1338,7 +1403,13 @@ static int single_rate_step(vh_blocks* m) {
   if (m->use_graph) {
     if (!m->graph || m->graph_np != np) {
       drop_graph(m);
-      if (int rc = ensure_side_streams(m)) return rc;   // nothing is created inside the capture
+      const int classes = list_classes(m, 0);
+      if (classes > 1 && !have_sides(m, classes - 1)) {   // nothing is created inside a capture
+        (void)hipGetLastError();
+        enqueue();
+        VH_HIP(hipGetLastError());
+        return 0;
+      }
       hipGraph_t gr = nullptr;
       VH_HIP(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
       enqueue();
@@ -1811,10 +1882,7 @@ int vh_blocks_destroy(vh_blocks* m) {
   (void)hipFree(m->clock);
   if (m->clock_host) (void)hipHostFree(m->clock_host);
   if (m->look) (void)hipEventDestroy(m->look);
-  for (int i = 0; i < kBlockClasses - 1; ++i) {
-    if (m->side[i]) (void)hipStreamDestroy(m->side[i]);
-    if (m->ev_join[i]) (void)hipEventDestroy(m->ev_join[i]);
-  }
+  for (int i = 0; i < m->nside; ++i) SidePool::give_back(m->side[i]);
   if (m->ev_fork) (void)hipEventDestroy(m->ev_fork);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;
