@@ -47,12 +47,13 @@ def test_round_trips_from_several_threads():
 
 @pytest.mark.parametrize("nbytes", [4 * MIB + 1, 4 * MIB + 16, 6 * MIB + 15, 9 * MIB + 12345])
 @pytest.mark.parametrize("offset", [0, 1, 8, 16, 2 * MIB + 48])
-def test_download_from_inside_an_allocation(nbytes, offset):
-    """Chunks stored by the kernel (16-byte aligned sources) and by the runtime (others),
+def test_copies_inside_an_allocation(nbytes, offset):
+    """Chunks moved by the kernel (16-byte aligned device addresses) and by the runtime (others),
     with partial 16-byte groups at the end, up to the allocation's last byte."""
-    print(f"download {nbytes} at {offset}", flush=True)
+    print(f"copies of {nbytes} at {offset}", flush=True)
     a = np.random.default_rng(nbytes + offset).integers(0, 256, size=nbytes + offset, dtype=np.uint8)
-    buf = DeviceBuffer(a.nbytes).upload(a)
+    buf = DeviceBuffer(a.nbytes)
+    V.check(V.load_library().vh_buffer_upload(buf.ptr + offset, a.ctypes.data + offset, nbytes))
     out = np.zeros(nbytes + 2, dtype=np.uint8)
     V.check(V.load_library().vh_buffer_download(out.ctypes.data + 1, buf.ptr + offset, nbytes))
     assert np.array_equal(out[1:-1], a[offset:]) and out[0] == 0 and out[-1] == 0

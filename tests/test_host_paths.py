@@ -54,11 +54,11 @@ def test_device_memory_as_the_host_side_is_not_touched_by_the_cpu(stub):
             assert f(a.ptr, b.ptr, 8 * MIB) == 0
             copies = [l for l in log() if l[0] == "copy"]
             assert [[int(x, 16) for x in c[1:3]] + [int(c[3])] for c in copies] == [[a.ptr, b.ptr, 8 * MIB]]
-        h = np.arange(8 * MIB, dtype=np.uint8)
+        h = np.arange(8 * MIB - 1, dtype=np.uint8)
         S.stub_clear()
-        assert L.vh_buffer_upload(a.ptr, addr(h), 8 * MIB) == 0
+        assert L.vh_buffer_upload(a.ptr + 1, addr(h), h.size) == 0   # odd target: no kernel
         assert len([l for l in log() if l[0] == "copy"]) == 4
-        assert C.string_at(a.ptr, 8 * MIB) == h.tobytes()
+        assert C.string_at(a.ptr + 1, h.size) == h.tobytes()
         """)
 
 
@@ -71,9 +71,9 @@ def test_copies_without_threads(stub):
         a = DeviceBuffer(9 * MIB + 5)
         h = np.random.default_rng(1).integers(0, 256, 9 * MIB + 5, dtype=np.uint8)
         o = np.zeros(h.size - 1, np.uint8)
-        a.upload(h)
-        assert L.vh_buffer_download(addr(o), a.ptr + 1, o.size) == 0   # odd source: no kernel
-        assert np.array_equal(h[1:], o)
+        assert L.vh_buffer_upload(a.ptr + 1, addr(h), o.size) == 0     # odd addresses: no kernel
+        assert L.vh_buffer_download(addr(o), a.ptr + 1, o.size) == 0
+        assert np.array_equal(h[:-1], o)
         """)
 
 

@@ -2,12 +2,11 @@
 //
 // The runtime moves pageable memory through its own staging with one thread; a fresh host
 // array also takes its page faults in that thread. Here the copy is cut into chunks that
-// pass through pinned slots, one chunk crossing the link (up by the runtime, down by
-// store_kernel) while the pool's threads copy others between the slots and the caller's array.
+// pass through pinned slots, one chunk crossing the link (move_kernel) while the pool's threads copy others between the slots and the caller's array.
 //
 // Bound: the link (57 GB/s each way from pinned memory) and the threads' page faults. Measured,
-// runtime and here (GB/s): down 5 MiB 17.6 and 40, 20 MiB 17.6 and 43, 200 MiB 17.7 and 48.6; down
-// into a fresh array of 200 MiB 10.7 and 16.7; up 8 MiB 34.6 and 36.3, 64 MiB 30.8 and 38.9. Copies of up
+// runtime and here (GB/s): down 5 MiB 17.6 and 39, 20 MiB 17.6 and 42, 200 MiB 17.5 and 48.6; down
+// into a fresh array of 200 MiB 10.5 and 19.7; up 8 MiB 34.5 and 43, 64 MiB 29.2 and 47.9. Copies of up
 // to 4 MiB stay with the runtime: what is gained goes into waking the threads there (a lone
 // 0.6 MiB download took 50 µs and 130).
 #include <hip/hip_runtime.h>
@@ -29,7 +28,7 @@ constexpr size_t kChunk = (size_t)2 << 20;   // bytes per slot
 constexpr size_t kPiece = (size_t)128 << 10; // bytes per thread at a time
 constexpr int kSlots = 16;                   // pinned slots of the process (32 MiB)
 constexpr int kSlotsPerCopy = 4;
-constexpr int kStoreWgs = 32;                // workgroups of store_kernel
+constexpr int kMoveWgs = 32;                 // workgroups of move_kernel
 // Copies of at most this many bytes go to the runtime.
 constexpr size_t kDirect = (size_t)4 << 20;
 
@@ -100,7 +99,7 @@ SlotPool& slot_pool() {
 
 void copy_pieces(char* dst, const char* src, size_t n) {
   try {
-    HostPool::run((int)((n + kPiece - 1) / kPiece), [&](int i) {
+    HostPool::run_copies((int)((n + kPiece - 1) / kPiece), [&](int i) {
       const size_t o = (size_t)i * kPiece;
       memcpy(dst + o, src + o, std::min(kPiece, n - o));
     });
@@ -120,27 +119,29 @@ bool is_pageable(const void* p) {
   return a.type == hipMemoryTypeUnregistered;
 }
 
-// n bytes to a pinned slot (16-byte aligned), 16 bytes per lane and pass. A kernel and not the
-// runtime's copy, since that runs on an engine which the driver also clears freed device memory
-// with: for some ms after a large free (a rollout's 860 MB) its downloads took 942 µs per 10 MiB against
-// 266 at rest, the kernel's 234 and 232. Bound: the link, reached with 16 workgroups or more.
+// n bytes between a pinned slot and the device, 16 bytes per lane and pass (both 16-byte aligned).
+// A kernel and not the runtime's copy, since that runs on an engine which the driver also
+// clears freed device memory with: for some ms after a large free (a rollout's 860 MB) its
+// downloads took 942 µs per 10 MiB against 266 at rest, the kernel's 234 and 232. Bound: the link;
+// µs per 10 MiB by workgroups, down and up: 8: 247, 450; 16: 235, 252; 32: 232, 227; 128: 234, 236;
+// 512: 226, 292.
 typedef unsigned U4 __attribute__((ext_vector_type(4)));
-__global__ void __launch_bounds__(256) store_kernel(const char* __restrict__ src, char* __restrict__ dst, size_t n) {
+__global__ void __launch_bounds__(256) move_kernel(const char* __restrict__ src, char* __restrict__ dst, size_t n) {
   const size_t nv = n / 16, lane = (size_t)blockIdx.x * 256 + threadIdx.x;
   for (size_t i = lane; i < nv; i += (size_t)gridDim.x * 256)
     __builtin_nontemporal_store(__builtin_nontemporal_load((const U4*)src + i), (U4*)dst + i);
   if (lane < n % 16) dst[nv * 16 + lane] = src[nv * 16 + lane];
 }
 
-// Whether store_kernel may read the bytes at src: an allocation of the device that holds them
+// Whether move_kernel may touch the bytes at p: an allocation of the device that holds them
 // all, 16-byte aligned. Everything else, errors included, is left to the runtime.
-bool kernel_reads(const char* src, size_t bytes, int device) {
+bool kernel_moves(const void* p, size_t bytes, int device) {
   hipPointerAttribute_t a{};
   hipDeviceptr_t base = nullptr;
   size_t size = 0;
-  if ((uintptr_t)src % 16 == 0 && hipPointerGetAttributes(&a, src) == hipSuccess && a.type == hipMemoryTypeDevice &&
-      a.device == device && hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)src) == hipSuccess)
-    return (size_t)(src - (const char*)base) + bytes <= size;
+  if ((uintptr_t)p % 16 == 0 && hipPointerGetAttributes(&a, p) == hipSuccess && a.type == hipMemoryTypeDevice &&
+      a.device == device && hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)p) == hipSuccess)
+    return (size_t)((const char*)p - (const char*)base) + bytes <= size;
   (void)hipGetLastError();
   return false;
 }
@@ -148,7 +149,19 @@ bool kernel_reads(const char* src, size_t bytes, int device) {
 hipError_t staged(char* dst, const char* src, size_t bytes, bool up, hipStream_t s, int device,
                   const std::vector<Slot>& slots) {
   const size_t n = (bytes + kChunk - 1) / kChunk, ns = slots.size();
+  const bool kernel = kernel_moves(up ? dst : src, bytes, device);
   auto len = [&](size_t c) { return std::min(kChunk, bytes - c * kChunk); };
+  // chunk c across the link
+  auto issue = [&](size_t c) {
+    const Slot& sl = slots[c % ns];
+    char* to = up ? dst + c * kChunk : sl.mem;
+    const char* from = up ? sl.mem : src + c * kChunk;
+    size_t count = len(c);
+    void* args[] = {&from, &to, &count};
+    hipError_t r = kernel ? hipLaunchKernel((const void*)move_kernel, dim3(kMoveWgs), dim3(256), args, 0, s)
+                          : hipMemcpyAsync(to, from, count, up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, s);
+    return r == hipSuccess ? hipEventRecord(sl.ev, s) : r;
+  };
   hipError_t e = hipSuccess;
   if (up) {
     for (size_t c = 0; c < n && e == hipSuccess; ++c) {
@@ -156,24 +169,9 @@ hipError_t staged(char* dst, const char* src, size_t bytes, bool up, hipStream_t
       if (c >= ns) e = hipEventSynchronize(sl.ev);
       if (e != hipSuccess) break;
       copy_pieces(sl.mem, src + c * kChunk, len(c));
-      e = hipMemcpyAsync(dst + c * kChunk, sl.mem, len(c), hipMemcpyHostToDevice, s);
-      if (e == hipSuccess) e = hipEventRecord(sl.ev, s);
+      e = issue(c);
     }
   } else {
-    const bool kernel = kernel_reads(src, bytes, device);
-    auto issue = [&](size_t c) {
-      const Slot& sl = slots[c % ns];
-      hipError_t r = hipSuccess;
-      if (kernel) {
-        const char* from = src + c * kChunk;
-        size_t n_bytes = len(c);
-        void* args[] = {&from, (void*)&sl.mem, &n_bytes};
-        r = hipLaunchKernel((const void*)store_kernel, dim3(kStoreWgs), dim3(256), args, 0, s);
-      } else {
-        r = hipMemcpyAsync(sl.mem, src + c * kChunk, len(c), hipMemcpyDeviceToHost, s);
-      }
-      return r == hipSuccess ? hipEventRecord(sl.ev, s) : r;
-    };
     for (size_t c = 0; c < std::min(n, ns) && e == hipSuccess; ++c) e = issue(c);
     for (size_t c = 0; c < n && e == hipSuccess; ++c) {
       e = hipEventSynchronize(slots[c % ns].ev);
