@@ -136,11 +136,11 @@ def cpu_baseline(U, n, steps=2):
 def blocks_leg(V, args):
     """Batched uneven AMR blocks: `args.blocks` blocks with edges drawn from
     {8, 16, 24, 32}, glued in random conforming and 2:1 pairs, smooth seeded
-    state, single-rate SSP-RK2 with the device CFL dt. One persistent launch per
-    RK stage replayed from a HIP graph (headline of the leg), the same launches
-    enqueued eagerly, and one launch per block per stage (the comparison loop).
-    Tile width, z planes per tile and the persistent workgroup count are picked
-    by the autotuner first (timed graph replays of each candidate)."""
+    state, single-rate SSP-RK2 with the device CFL dt. One launch per tile-shape
+    class and RK stage replayed from a HIP graph (headline of the leg), the same
+    launches enqueued eagerly ("persistent"), and one launch per block per stage (the
+    comparison loop). Tile width, z planes per tile and the cap on the workgroups are
+    picked by the autotuner first (timed graph replays of each candidate)."""
     import numpy as np
     from vespa_jl_amd import blockmesh as BM
     m = BM.random_block_pairs(args.blocks, seed=2024, rank=3, edges=(8, 16, 24, 32))

@@ -296,8 +296,8 @@ int vh_adjoint_info(const vh_adjoint* a, double* ms_forward, double* ms_backward
  * side with the fine area; reconstruction across a block face uses one
  * representative neighbour (lib/HGBackend/src/HGBackend.jl:178-200): the
  * neighbour cell, the coarse cell containing the position, or the finer cell at
- * the lo corner of the coarse face. One persistent launch per RK stage covers
- * every block.
+ * the lo corner of the coarse face. An RK stage is one launch for each class of
+ * tile shapes, over every block.
  */
 typedef struct vh_blocks vh_blocks;
 
@@ -434,10 +434,10 @@ int vh_blocks_apply_laplacian(vh_blocks* m, const void* dx, void* dout);
 int vh_blocks_gravity_accel(vh_blocks* m, void* dg);
 
 /* Time nsteps single-rate steps (device dt) with HIP events after two untimed
- * steps. method 0: one persistent launch per stage, eager; 1: one launch per
- * block per stage (the comparison loop); 2: persistent launches replayed from a
- * HIP graph. ms_stage2 (optional): mean duration of the persistent stage-2
- * launch over up to 20 further eager steps. */
+ * steps. method 0: the stepping of vh_blocks_run, eager; 1: one launch per
+ * block per stage (the comparison loop); 2: as 0, replayed from a HIP graph.
+ * ms_stage2 (optional): mean duration of stage 2's launches over up to 20
+ * further eager steps. */
 int vh_blocks_time_steps(vh_blocks* m, double cfl, int64_t nsteps, int32_t method, double* ms_step,
                          double* ms_stage2);
 

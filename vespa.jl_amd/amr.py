@@ -18,7 +18,7 @@ tables, uploads them in one copy next to the current ones, and a remap kernel
 injects each parent cell's conserved values into its children device to
 device, so Σ U·V is unchanged; no device memory is allocated unless the mesh
 outgrows every earlier one. Between
-regrids the leaves are advanced by the batched kernel (one persistent launch
+regrids the leaves are advanced by the batched kernel (one launch
 per RK stage).
 """
 from __future__ import annotations

@@ -8,8 +8,8 @@ runs apply it without sweeping.
 
 * uniform grids: tile variant (``vh_grid_tile_count`` shapes) × z planes per
   workgroup;
-* block meshes: widest tile along x × z planes per tile × persistent workgroups
-  per compute unit.
+* block meshes: widest tile along x × z planes per tile × cap on the workgroups per
+  compute unit.
 
 The library's own choice of z planes (0 for a grid, -1 for a block mesh) is always
 among the default candidates, so that tuning never ends with a slower launch than an

@@ -297,7 +297,7 @@ def table_digest(mesh: BlockMesh, zchunk: int = 0, nthreads: int = 0) -> int:
 
 class BlockSimulation:
     """Device-resident simulation on a block mesh (the HGBackend Simulation,
-    src/driver.jl:27-79): one persistent launch per RK stage over every block,
+    src/driver.jl:27-79): per RK stage one launch for each tile-shape class of all blocks,
     link faces between blocks, flux registers for subcycling."""
 
     def __init__(self, mesh: BlockMesh, eltype=np.float64, cfl: float = 0.4):
@@ -499,7 +499,7 @@ class BlockSimulation:
 
     def time_steps(self, nsteps: int, method: str = "graph", stage2: bool = True) -> dict:
         """Time nsteps single-rate steps: method 'persistent' (eager), 'per_block'
-        (one launch per block per stage) or 'graph' (persistent, HIP graph)."""
+        (one launch per block per stage) or 'graph' (the first, from a HIP graph)."""
         C = self._C
         code = {"persistent": 0, "per_block": 1, "graph": 2}[method]
         a, b = C.c_double(), C.c_double()

@@ -13,9 +13,9 @@
 //   link_flux_kernel   one lane per face between two different blocks: the
 //                      HLLC flux from representative-neighbour reconstruction,
 //                      written to a face buffer;
-//   block_stage_kernel one persistent launch over a device tile list; each
-//                      workgroup runs the 2.5-D plane march of stencil.h on its
-//                      tiles (runtime tile shape, block geometry per tile) and,
+//   block_stage_kernel one launch per tile-shape class over a device tile list;
+//                      each workgroup runs the 2.5-D plane march of stencil.h on its
+//                      tiles (block geometry per tile) and,
 //                      for cells that touch link faces, takes those fluxes from
 //                      the buffer and adds everything in the order of the face
 //                      walk: foreign groups of lower-index blocks, the cell's own
@@ -151,8 +151,8 @@ __device__ __forceinline__ void add_link_group(Cons<T>& acc, const BlocksDev& B,
 }
 
 
-// One RK stage over a list of tiles (persistent: workgroup w takes tiles w,
-// w + gridDim.x, ...). STAGE2 as in rk_stage_kernel; the CFL partial of the
+// One RK stage over a list of tiles (workgroup w takes tiles w, w + gridDim.x, ...: one
+// tile each where the launch has a workgroup per tile). STAGE2 as in rk_stage_kernel; the CFL partial of the
 // new state covers the workgroup's tiles.
 // apply_gravity_source! (src/gravity.jl:412-447) for cell c of a block with
 // volume V: (0, −ρg_x·V, −ρg_y·V, −ρg_z·V, −(ρv·g)·V) added to the flux sum, g

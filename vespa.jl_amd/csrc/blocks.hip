@@ -16,8 +16,8 @@
 //     emitting cells);
 //   - flux-register lists: per level, the coarse cells with finer neighbours
 //     (src/reflux.jl:51-103);
-//   - tile lists for one persistent launch per stage (all blocks, per level,
-//     and per block for the launch-per-block comparison).
+//   - tile lists grouped by shape class, one launch each per stage (all blocks, per
+//     level, and per block for the launch-per-block comparison).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -268,8 +268,6 @@ struct BuildScratch {
   std::vector<long long> cost;
 };
 
-// Builds every table of a mesh. Returns 0 or a negative code (message set).
-// nthreads: 0 = the pool's size, 1 = serial; the tables do not depend on it.
 // Tile of a block of n cells, at most max_tx wide; false if no shape fits.
 static bool tile_shape(int rank, const int* n, int max_tx, int* tx, int* ty) {
   if (rank == 1) {
@@ -299,6 +297,8 @@ static int default_zchunk(const Topo& T, int max_tx) {
   return (int)std::min(6LL, std::max(1LL, (planes + 750) / 1500));
 }
 
+// Builds every table of a mesh. Returns 0 or a negative code (message set).
+// nthreads: 0 = the pool's size, 1 = serial; the tables do not depend on it.
 static int build_tables(Topo& T, int zchunk, HostTables& H, int max_tx = 32, int nthreads = 0) {
   const int nb = T.nb, rank = T.rank;
   // ---- candidate neighbours by face plane ----
@@ -1081,7 +1081,7 @@ struct vh_blocks {
   int zchunk = 8;
   bool zchunk_auto = true;   // zchunk follows the mesh and the tile width (vh_blocks_set_launch: -1)
   int max_tx = 32;        // widest tile along x
-  int max_wgs = 0;        // persistent workgroups (0: 3 per CU)
+  int max_wgs = 0;        // cap on a stage's workgroups (0: one per tile, 3 per CU for the runtime shape)
   int ncu = 256;
   int stage_wgs = 0;      // workgroups of the last all-blocks stage-2 launch
   int use_graph = 1;
@@ -1239,7 +1239,9 @@ static bool have_sides(vh_blocks* m, int n) {
 // another each left the chip to its last few workgroups (400 blocks, 5.1 M cells, Float64:
 // 437 µs per stage, of which 8³ and 16³ blocks, a tenth of the cells, took 155). Step times
 // in sequence and side by side: 400 blocks f64 0.87 and 0.65 ms, 3000 blocks f64 4.97 and
-// 4.36, f32 3.22 and 2.65. One kernel holding every shape was slower (5.41 ms for 3000 blocks:
+// 4.36, f32 3.22 and 2.65; eager steps, with the fork's ten or so calls per stage: 20 blocks f64 0.18 and
+// 0.14, 100 blocks 0.44 and 0.31; subcycled steps of 100 blocks 2.36 and 1.61, of 20 blocks f32
+// 0.76 and 0.81. One kernel holding every shape was slower (5.41 ms for 3000 blocks:
 // the shapes share one register budget and spill twice as much).
 // A class that cannot be forked runs on the context's stream, and the host waits for one
 // that cannot be joined to it: no failure leaves launches unordered.
@@ -2395,7 +2397,7 @@ int vh_blocks_time_steps(vh_blocks* m, double cfl, int64_t nsteps, int32_t metho
   } else if (!rc) {
     rc = fail(-2, "hipEventCreate failed%s", "");
   }
-  // Stage-2 launches of the persistent kernel timed one by one (eager steps).
+  // Stage-2 launches timed one by one (eager steps).
   double st2 = 0.0;
   const int k2 = (int)(nsteps < 20 ? nsteps : 20);
   std::vector<hipEvent_t> ev(2 * k2, nullptr);

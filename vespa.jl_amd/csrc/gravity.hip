@@ -115,7 +115,8 @@ __device__ __forceinline__ void for_cells(long long n, F f) {
   }
 }
 
-// x / d for x < 2^31 as a multiplication: m = ceil(2^(31+l)/d) with 2^l >= d exceeds
+// x / d for x < 2^31 as a multiplication (Granlund and Montgomery, Division by invariant integers
+// using multiplication, 1994): m = ceil(2^(31+l)/d) with 2^l >= d exceeds
 // 2^(31+l)/d by less than 2^l/d, so the product is off by less than 1/d.
 struct FastDiv {
   unsigned m;

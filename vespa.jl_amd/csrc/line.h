@@ -18,8 +18,9 @@
 // Bound: latency (barriers, divisions and square roots in sequence) with one wave per SIMD,
 // VALU issue with four. Measured per step, exact Float64 / fast Float32, against three launches
 // per step over many workgroups (16.6 / 14.9 µs at any of these sizes): 64 cells 3.5 / 2.2 µs,
-// 400 cells 5.0 / 2.7, 1023 cells 8.4 / 4.0, 2040 cells 16.1 / 6.5. The limit is the LDS, which is
-// about where the Float64 times meet.
+// 400 cells 5.0 / 2.7, 1023 cells 8.4 / 4.0, 2040 cells 16.1 / 6.5. The limit is the LDS of a
+// Float64 grid, about where the Float64 times meet; Float32 grids have the same limit, though their
+// LDS would hold twice the cells.
 #pragma once
 
 #include "stencil.h"

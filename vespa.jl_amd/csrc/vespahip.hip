@@ -726,8 +726,8 @@ static bool line_fits(const vh_grid* g) {
 static int run_line(vh_grid* g, double cfl, double tfinal, int64_t max_steps, double* t_io, int64_t* steps) {
   const bool clip = tfinal > 0.0;
   const double tstop = tfinal * (1 - 1e-12);
-  // A launch takes at most this many steps (about 5 ms at 400 cells), so that no kernel
-  // runs unboundedly long.
+  // A launch takes at most this many steps, so that no kernel runs unboundedly long (exact
+  // Float64: 10 ms at 400 cells, 33 ms at 2040).
   constexpr int64_t kMost = 2048;
   double* clk = g->clock_host;
   int64_t k = 0;

@@ -10,7 +10,7 @@
 #     for RefMesh `UniformMesh` simulations, and `hip_set_mode!` selecting the
 #     exact (bit-identical) or fast arithmetic profile;
 #   * `HIPBlocks`: block-structured AMR meshes (hanging-node faces, flux
-#     registers, subcycling) advanced by one persistent launch per RK stage;
+#     registers, subcycling) advanced by one launch per tile-shape class and RK stage;
 #   * `hip_step_vjp`: the pullback of one step, and `HIPRollout` (`hip_forward!` /
 #     `hip_backward`): a checkpointed rollout; `hip_step_state` / `hip_rollout_state`
 #     are the state-to-state functions whose ChainRulesCore `rrule`s live in
