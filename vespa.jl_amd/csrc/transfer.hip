@@ -2,7 +2,8 @@
 //
 // The runtime moves pageable memory through its own staging with one thread; a fresh host
 // array also takes its page faults in that thread. Here the copy is cut into chunks that
-// pass through pinned slots, one chunk crossing the link (move_kernel) while the pool's threads copy others between the slots and the caller's array.
+// pass through pinned slots, one chunk crossing the link (move_kernel) while the pool's threads
+// copy others between the slots and the caller's array.
 //
 // Bound: the link (57 GB/s each way from pinned memory) and the threads' page faults. Measured,
 // runtime and here (GB/s): down 5 MiB 17.6 and 39, 20 MiB 17.6 and 42, 200 MiB 17.5 and 48.6; down
